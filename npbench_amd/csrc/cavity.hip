@@ -2,26 +2,32 @@
 // (npbench/benchmarks/cavity_flow/cavity_flow_numpy.py:13-83), FP64, bitwise
 // the NumPy reference.
 //
-// A time step is a chain of whole-grid phases -- copy u, v; build b; nit
-// pressure-Poisson Jacobi iterations; update u, v -- on grids of ~10^4 points
-// (the paper preset is 101 x 101 with 700 steps of 50 iterations: 37,000
-// phases).  One launch per phase would be bound by launches, so one workgroup
-// of kThreadsC threads runs every phase in a loop with a barrier between
-// phases.  The pressure alternates between two buffers (the reference's
-// pn = p.copy() each iteration).  Grids of up to kLdsPoints points (the paper
-// and S presets) keep both buffers in LDS for the whole run and b in
-// registers, so an iteration never leaves the CU (cavity_flow_lds); larger
-// grids use p and a device scratch copy, which the caches hold
-// (cavity_flow_global).  Divisions are by five uniform divisors whose
-// reciprocals are prepared once (division.h).  b needs no zeroing: only its
-// interior is read, and each step writes it first.
+// A time step is a chain of whole-grid phases -- build b; nit pressure-Poisson
+// Jacobi iterations; update u, v -- on grids of ~10^4 points (the paper preset
+// is 101 x 101 with 700 steps of 50 iterations: 37,000 phases).  A launch per
+// phase would be bound by launches, so two forms cut their number:
+//
+// * cavity_pressure advances the pressure by up to kMaxDepth iterations per
+//   launch (temporal blocking): a workgroup holds its block and a halo of one
+//   cell per iteration in registers, so it needs nothing from other
+//   workgroups until the launch ends; cavity_velocity does the velocity update
+//   of one step and the source of the next in one launch.  A step of 20
+//   iterations is 2 launches spread over the chip.
+// * cavity_flow_lds runs every phase of the call in one workgroup with a
+//   barrier between phases, both pressure buffers in LDS and b in registers:
+//   no launches, but one CU.  It stays for the small grids where a phase
+//   costs less than its share of a launch (use_lds below).
+//
+// Divisions are by five uniform divisors whose reciprocals are prepared once
+// (division.h).  b needs no zeroing: only its interior is read, and each step
+// writes it first.
 //
 // The four boundary statements after each iteration (:30-33), applied in the
 // reference's order, leave row 0, column 0 and column nx-1 equal to this
 // iteration's interior next to them (the corners (0,0) and (0,nx-1) take
-// (1,1) and (1,nx-2)) and the last row 0.  So the thread that computes an
-// interior point next to one of those edges also writes the edge copies, and
-// an iteration is a single phase.
+// (1,1) and (1,nx-2)) and the last row 0.  So whoever computes an interior
+// point next to one of those edges also knows the edge's value, and an
+// iteration is a single phase.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -29,12 +35,13 @@
 
 #include "common.h"
 #include "division.h"
+#include "lanes.h"
 
 namespace npbx {
 namespace {
 
 constexpr int kThreadsC = 1024;
-constexpr int kLdsPoints = 10240;  // two FP64 pressure buffers: all 160 KiB of LDS
+constexpr int kLdsPoints = 1024;  // most points of the one-workgroup form
 
 // The reference's scalar expressions, computed on the host as Python computes
 // them (x**2 is the C library's pow, which CPython's float power calls).
@@ -111,28 +118,37 @@ struct InteriorWalk {
   }
 };
 
-constexpr int kChunkP = 6;  // pressure points per chunk (5 loads each)
-constexpr int kChunkB = 4;  // source points per chunk (8 loads each)
 constexpr int kChunkV = 2;  // velocity points per chunk (14 loads each)
-constexpr int kMaxPts = kLdsPoints / kThreadsC;  // interior points per thread, LDS grids
+constexpr int kMaxPts = 2;  // interior points per thread, in the one-workgroup form
 
 // The point computations take their division as a policy (ShortDiv or
 // FullDiv, run by chunk_eval).
 
-// build_up_b (:13-21) at interior point x.
+// build_up_b (:13-21) from the velocities east, west, north (row + 1) and
+// south (row - 1) of a point.
+template <class Div>
+__device__ __forceinline__ double source_from(const CavityArgs& g, const CavityDivisors& dv,
+                                              double ue, double uw, double un, double us,
+                                              double ve, double vw, double vn, double vs,
+                                              Div& div) {
+  const double dudx = div(ue - uw, dv.two_dx);
+  const double dvdy = div(vn - vs, dv.two_dy);
+  const double t1 = g.inv_dt * (dudx + dvdy);
+  const double t2 = dudx * dudx;
+  const double t3 = 2.0 * div(div(un - us, dv.two_dy) * (ve - vw), dv.two_dx);
+  const double t4 = dvdy * dvdy;
+  return g.rho * (((t1 - t2) - t3) - t4);
+}
+
+// The same at interior point x of the fields.
 template <class Div>
 __device__ __forceinline__ double source_at(const CavityArgs& g, const CavityDivisors& dv, int x,
                                             Div& div) {
   const int nx = g.nx;
   const double* u = g.u;
   const double* v = g.v;
-  const double dudx = div(u[x + 1] - u[x - 1], dv.two_dx);
-  const double dvdy = div(v[x + nx] - v[x - nx], dv.two_dy);
-  const double t1 = g.inv_dt * (dudx + dvdy);
-  const double t2 = dudx * dudx;
-  const double t3 = 2.0 * div(div(u[x + nx] - u[x - nx], dv.two_dy) * (v[x + 1] - v[x - 1]), dv.two_dx);
-  const double t4 = dvdy * dvdy;
-  return g.rho * (((t1 - t2) - t3) - t4);
+  return source_from(g, dv, u[x + 1], u[x - 1], u[x + nx], u[x - nx], v[x + 1], v[x - 1],
+                     v[x + nx], v[x - nx], div);
 }
 
 // One pressure iterate (:30-33) at interior point x, with b there.
@@ -235,64 +251,259 @@ __device__ __forceinline__ CavityDivisors cavity_divisors(const CavityArgs& g) {
   return dv;
 }
 
-// Grids of more than kLdsPoints points: the pressure alternates between p and
-// the scratch copy pn, b lives in device memory, and the threads walk their
-// points in chunks.
-__global__ __launch_bounds__(kThreadsC) void cavity_flow_global(CavityArgs g) {
-  const int t = threadIdx.x, nx = g.nx, ny = g.ny;
-  const int np = nx * ny;
-  const InteriorWalk walk(t, nx, ny);
-  const CavityDivisors dv = cavity_divisors(g);
-  double* cur = g.p;  // the current pressure
-  double* nxt = g.pn;
-  for (int step = 0; step < g.nt; ++step) {
-    copy_velocities(g, t, np);
-    // b's interior, from u and v, which the copy above only reads too
-    walk.each<kChunkB>([&](const int(&a)[kChunkB], const int(&)[kChunkB],
-                           const bool(&ok)[kChunkB]) {
-      double bv[kChunkB];
-      chunk_eval(dv, bv, [&](int c, auto& div) { return source_at(g, dv, a[c], div); });
-#pragma unroll
-      for (int c = 0; c < kChunkB; ++c)
-        if (ok[c]) g.b[a[c]] = bv[c];
-    });
-    __syncthreads();
-    for (int q = 0; q < g.nit; ++q) {
-      walk.each<kChunkP>([&](const int(&a)[kChunkP], const int(&fl)[kChunkP],
-                             const bool(&ok)[kChunkP]) {
-        double val[kChunkP];
-        chunk_eval(dv, val, [&](int c, auto& div) { return pressure_at(g, dv, cur, a[c], g.b[a[c]], div); });
-#pragma unroll
-        for (int c = 0; c < kChunkP; ++c)
-          if (ok[c]) store_pressure(nxt, a[c], fl[c], nx, val[c]);
-      });
-      for (int k = t; k < nx; k += kThreadsC) nxt[(ny - 1) * nx + k] = 0.0;  // p[-1, :] = 0
-      __syncthreads();
-      double* tmp = cur;
-      cur = nxt;
-      nxt = tmp;
-    }
-    walk.each<kChunkV>([&](const int(&a)[kChunkV], const int(&)[kChunkV],
-                           const bool(&ok)[kChunkV]) {
-      double nu[kChunkV], nv[kChunkV];
-      chunk_eval(dv, nu, [&](int c, auto& div) {
-        double uu;
-        velocity_at(g, dv, cur, a[c], uu, nv[c], div);
-        return uu;
-      });
-#pragma unroll
-      for (int c = 0; c < kChunkV; ++c) {
-        if (ok[c]) {
-          g.u[a[c]] = nu[c];
-          g.v[a[c]] = nv[c];
-        }
-      }
-    });
-    velocity_boundaries(g, t);
-    __syncthreads();
+// ---- blocked form: a chip-wide launch per group of pressure iterations -----
+//
+// cavity_pressure<R>: 16 waves stacked along y, each holding R rows x 64
+// columns of p and cb b in registers (one column per lane).  A workgroup
+// advances its region `depth` iterations; next to other blocks the outer
+// `depth` cells are halo, computed redundantly and one cell less valid per
+// iteration; at the grid's edges the region ends with the interior, where the
+// edge points hold copies of their interior neighbours (the last row: 0) and
+// need no registers.  West and east are the adjacent lanes (DPP shifts; the
+// outer lanes get themselves back, which at the grid's edge is the copy),
+// north and south the wave's own rows, the two edge rows of a wave go through
+// LDS (one barrier per iteration).  So every block runs the same code.  Only
+// an iteration from memory reads the stored edge (the first of a call may
+// hold anything there): its outer neighbours are loaded beside the region.
+// NARROW: grids narrower than a region (fewer than 64 interior columns or
+// 16 R rows), where the edges fall inside it and are selected per point.
+//
+// The division by den is the short form with its residual negated twice
+// (r = fma(den, m, -n), q = fma(-r, y, m)): the same value, and for n = +-0
+// the quotient keeps n's sign, so exact zeros -- a flow at rest has many --
+// need no fallback.  It is exact where nothing in the IEEE sequence rescales:
+// den in [2^-100, 2^100] and every n zero or of magnitude 2^-900 .. 2^300.
+// The upper side is checked once: |p|, |cb b| < 2^100 on load bound every
+// iterate by 2^100 (1 + depth) and rounding, because an iterate's weights sum
+// to one.  The lower side is the smallest exponent of n over all iterations
+// (frexp gives 0 for n = 0).  A workgroup that leaves the range anywhere
+// starts over from global memory with the division operator.
+//
+// Bound by FP64 issue and the exchange: 15 VALU instructions per point and
+// iteration at four cycles each (9 arithmetic, 4 lane shifts, 1.5 for the
+// range), then the waves' common wait for LDS and the barrier.  201 x 201,
+// 20 iterations in one launch of 140 blocks: 14.2 us (0.6 us an iteration;
+// one workgroup for the whole grid took 33 us).  Sixteen waves of 3 rows
+// measured faster than eight of 6 or four of 12 (1.86, 1.92, 2.04 ms for 100
+// steps): more waves hide more of the shifts' and LDS latencies than the
+// smaller exchange saves.
+constexpr int kWavesP = 16;
+constexpr int kMaxDepth = 24;
+constexpr int kMinExpN = -898;  // |n| >= 2^-899
+
+struct PressureDiv {  // den, its reciprocal
+  double d, y;
+};
+
+template <bool FULL>
+__device__ __forceinline__ double pressure_quotient(double n, const PressureDiv& v, int& emin) {
+  if constexpr (FULL) {
+    return n / v.d;
+  } else {
+    emin = min(emin, __builtin_amdgcn_frexp_exp(n));
+    const double m = n * v.y;
+    const double r = __builtin_fma(v.d, m, -n);
+    return __builtin_fma(-r, v.y, m);
   }
-  if (cur != g.p) {  // an odd number of iterations in all: the result is in pn
-    for (int k = t; k < np; k += kThreadsC) g.p[k] = cur[k];
+}
+
+// Where a block lies: its region's first grid row and column, and the rows
+// and columns [lo, hi) of the region it owns.
+struct Span {
+  int origin, lo, hi;
+};
+
+// Blocks of a direction with n interior points, `width` points per region:
+// regions at the grid's ends have no halo on that side; the last one is
+// shifted back to end with the grid.
+__host__ __device__ inline int span_count(int n, int width, int depth) {
+  return n <= width ? 1 : (n - 2 * depth + width - 2 * depth - 1) / (width - 2 * depth);
+}
+__device__ __forceinline__ Span span_of(int t, int count, int n, int width, int depth) {
+  const int out = width - 2 * depth;
+  const int o = t == count - 1 ? max(n - width, 0) : t * out;
+  return {1 + o, (t == 0 ? 0 : t * out + depth) - o, (t == count - 1 ? n : (t + 1) * out + depth) - o};
+}
+
+// One iteration of the wave's rows x into y (:30-37): ring[r] holds the
+// values west of lane 0 and east of lane 63, `top` and `bottom` the rows
+// outside the region (waves 0 and 15).
+template <int R, bool NARROW, bool FULL>
+__device__ __forceinline__ void pressure_step(const double (&x)[R], double (&y)[R],
+                                              const double (&bb)[R], const double (&ring)[R],
+                                              double top, double bottom, double (*edge)[2][64],
+                                              int lane, int w, int gi0, int gj,
+                                              const CavityArgs& g, const PressureDiv& v,
+                                              bool settled, int& emin) {
+  edge[w][0][lane] = x[0];
+  edge[w][1][lane] = x[R - 1];
+  __syncthreads();
+  double above = edge[max(w - 1, 0)][1][lane];
+  double below = edge[min(w + 1, kWavesP - 1)][0][lane];
+  if (w == 0) above = top;
+  if (w == kWavesP - 1) below = bottom;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const double c = x[r];
+    double north = r == 0 ? above : x[r - 1];
+    double south = r == R - 1 ? below : x[r + 1];
+    double west = lane_from_left_or(ring[r], c), east = lane_from_right_or(ring[r], c);
+    if constexpr (NARROW) {
+      west = settled && gj == 1 ? c : west;
+      east = settled && gj == g.nx - 2 ? c : east;
+      if (settled && gi0 + r == 1) north = c;
+      if (settled && gi0 + r == g.ny - 2) south = 0.0;
+    }
+    const double n = (east + west) * g.dy2 + (south + north) * g.dx2;
+    y[r] = pressure_quotient<FULL>(n, v, emin) - bb[r];
+  }
+}
+
+template <int R, bool NARROW, bool FULL>
+__device__ __forceinline__ void pressure_steps(double (&x)[R], const double (&bb)[R],
+                                               const double (&ring)[R], double top, double bottom,
+                                               double (*edge)[kWavesP][2][64], int lane, int w,
+                                               int gi0, int gj, const CavityArgs& g,
+                                               const PressureDiv& v, int depth, int& emin) {
+  double y[R];
+  pressure_step<R, NARROW, FULL>(x, y, bb, ring, top, bottom, edge[0], lane, w, gi0, gj, g, v,
+                                 false, emin);
+  int k = 1;
+  for (; k + 2 <= depth; k += 2) {
+    pressure_step<R, NARROW, FULL>(y, x, bb, y, y[0], 0.0, edge[1], lane, w, gi0, gj, g, v, true,
+                                   emin);
+    pressure_step<R, NARROW, FULL>(x, y, bb, x, x[0], 0.0, edge[0], lane, w, gi0, gj, g, v, true,
+                                   emin);
+  }
+  if (k < depth) {
+    pressure_step<R, NARROW, FULL>(y, x, bb, y, y[0], 0.0, edge[1], lane, w, gi0, gj, g, v, true,
+                                   emin);
+  } else {
+#pragma unroll
+    for (int r = 0; r < R; ++r) x[r] = y[r];
+  }
+}
+
+template <int R, bool NARROW>
+__global__ __launch_bounds__(64 * kWavesP) void cavity_pressure(CavityArgs g,
+                                                                const double* __restrict__ src,
+                                                                double* __restrict__ dst,
+                                                                int depth, int tiles_x,
+                                                                int tiles_y) {
+  __shared__ double edge[2][kWavesP][2][64];
+  const int lane = threadIdx.x % 64;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int nx = g.nx, ny = g.ny;
+  const Span sx = span_of(blockIdx.x % tiles_x, tiles_x, nx - 2, 64, depth);
+  const Span sy = span_of(blockIdx.x / tiles_x, tiles_y, ny - 2, R * kWavesP, depth);
+  const int gj = sx.origin + lane, gi0 = sy.origin + w * R;
+  const PressureDiv v{g.den, uniform_double(division_reciprocal(g.den))};
+  const bool den_ok = g.den >= 0x1p-100 && g.den <= 0x1p100;
+
+  // p clamped into the grid, cb b into the interior: every load lands on a
+  // value that exists (clamped ones only in a NARROW grid's unused rows and
+  // lanes)
+  double x[R], bb[R], ring[R], top, bottom;
+  const int gjp = min(gj, nx - 1), gjb = min(gj, nx - 2);
+  const int gjr = lane == 0 ? gj - 1 : min(gj + 1, nx - 1);
+  bool bad = !den_ok;
+  auto load_p = [&] {
+#pragma unroll
+    for (int r = 0; r < R; ++r) x[r] = src[min(gi0 + r, ny - 1) * nx + gjp];
+#pragma unroll
+    for (int r = 0; r < R; ++r) ring[r] = src[min(gi0 + r, ny - 1) * nx + gjr];
+    top = src[(sy.origin - 1) * nx + gjp];
+    bottom = src[min(sy.origin + R * kWavesP, ny - 1) * nx + gjp];
+  };
+  load_p();
+#pragma unroll
+  for (int r = 0; r < R; ++r) bb[r] = g.b[min(gi0 + r, ny - 2) * nx + gjb];
+  auto in_range = [](double a) { return fabs(a) < 0x1p100; };
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    bad = bad || !in_range(x[r]) || !in_range(bb[r]) || !in_range(ring[r]);
+  bad = bad || !in_range(top) || !in_range(bottom);
+  int emin = 0;
+  pressure_steps<R, NARROW, false>(x, bb, ring, top, bottom, edge, lane, w, gi0, gj, g, v, depth,
+                                   emin);
+  bad = bad || emin < kMinExpN;
+  if (__syncthreads_or(bad)) {
+    load_p();
+    pressure_steps<R, NARROW, true>(x, bb, ring, top, bottom, edge, lane, w, gi0, gj, g, v, depth,
+                                    emin);
+  }
+
+  // the block's interior points, with the edge copies the boundary statements
+  // make of them
+  if (lane < sx.lo || lane >= sx.hi || gj > nx - 2) return;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int gi = gi0 + r, k = w * R + r;
+    if (k < sy.lo || k >= sy.hi || gi > ny - 2) continue;
+    const int at = gi * nx + gj;
+    store_pressure(dst, at, (gi == 1 ? kRow1 : 0) | (gj == 1 ? kCol1 : 0) |
+                                (gj == nx - 2 ? kColLast : 0), nx, x[r]);
+    if (gi == ny - 2) {  // p[-1, :] = 0, the corners with it
+      dst[at + nx] = 0.0;
+      if (gj == 1) dst[at + nx - 1] = 0.0;
+      if (gj == nx - 2) dst[at + nx + 1] = 0.0;
+    }
+  }
+}
+
+// The velocity update of one step (VEL; otherwise u, v are taken as they are)
+// and the source cb b of the next (SRC), one point per thread: a workgroup
+// computes the new u, v of 16 x 64 points, exchanges them through LDS and
+// forms b for the 14 x 62 inside.  un, vn -> u, v are separate arrays (the
+// reference's copies); boundary points take the boundary conditions
+// (:75-82), the same value from every workgroup that holds them.
+constexpr int kTileVI = 14, kTileVJ = 62;
+
+template <bool VEL, bool SRC>
+__global__ __launch_bounds__(1024) void cavity_velocity(CavityArgs g, const double* __restrict__ p,
+                                                        int tiles_x) {
+  __shared__ double su[16][64], sv[16][64];
+  const int lane = threadIdx.x % 64;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int nx = g.nx, ny = g.ny;
+  const int gi = static_cast<int>(blockIdx.x) / tiles_x * kTileVI + w;
+  const int gj = static_cast<int>(blockIdx.x) % tiles_x * kTileVJ + lane;
+  const bool inside = gi < ny && gj < nx;
+  const bool interior = gi >= 1 && gi <= ny - 2 && gj >= 1 && gj <= nx - 2;
+  const bool owned = interior && w >= 1 && w <= kTileVI && lane >= 1 && lane <= kTileVJ;
+  const CavityDivisors dv = cavity_divisors(g);
+  const int at = gi * nx + gj;
+  double nu = 0.0, nv = 0.0;
+  if (VEL && interior) {
+    double un1[1];
+    chunk_eval(dv, un1, [&](int, auto& div) {
+      double uu;
+      velocity_at(g, dv, p, at, uu, nv, div);
+      return uu;
+    });
+    nu = un1[0];
+  } else if (VEL) {
+    nu = gi == ny - 1 ? 1.0 : 0.0;
+  } else if (inside) {
+    nu = g.un[at];
+    nv = g.vn[at];
+  }
+  if (inside && (owned || !interior) && g.u != g.un) {
+    g.u[at] = nu;
+    g.v[at] = nv;
+  }
+  if constexpr (SRC) {
+    su[w][lane] = nu;
+    sv[w][lane] = nv;
+    __syncthreads();
+    if (!owned) return;
+    double bv[1];
+    chunk_eval(dv, bv, [&](int, auto& div) {
+      return source_from(g, dv, su[w][lane + 1], su[w][lane - 1], su[w + 1][lane],
+                         su[w - 1][lane], sv[w][lane + 1], sv[w][lane - 1], sv[w + 1][lane],
+                         sv[w - 1][lane], div);
+    });
+    g.b[at] = g.cb * bv[0];
   }
 }
 
@@ -390,6 +601,107 @@ __global__ __launch_bounds__(kThreadsC) void cavity_flow_lds(CavityArgs g) {
   for (int k = t; k < np; k += kThreadsC) g.p[k] = cur[k];
 }
 
+// Shape of the pressure launches: rows per wave and iterations per launch
+// with the smallest modelled time for a step.  A launch costs about 4 us
+// (gap, loads, stores) and an iteration 0.1 us (exchange, barrier) plus
+// 0.1 us per row of a wave and per workgroup a CU has to run.
+struct PressurePlan {
+  int rows, depth, rounds;
+};
+
+PressurePlan plan_pressure(int nx, int ny, int nit) {
+  PressurePlan best{};
+  double best_us = INFINITY;
+  for (const int rows : {2, 3, 4, 6}) {
+    for (int rounds = static_cast<int>(cdiv(nit, kMaxDepth)); rounds <= nit; ++rounds) {
+      const int depth = static_cast<int>(cdiv(nit, rounds));
+      if (64 - 2 * depth < 8 || rows * kWavesP - 2 * depth < 8) continue;
+      const int tx = span_count(nx - 2, 64, depth), ty = span_count(ny - 2, rows * kWavesP, depth);
+      const double us = rounds * 4.0 + nit * (0.1 + 0.1 * rows * cdiv(int64_t(tx) * ty, 256));
+      if (us < best_us) {
+        best_us = us;
+        best = {rows, depth, rounds};
+      }
+      if (depth <= 4) break;  // shallower launches only add launches
+    }
+  }
+  return best;
+}
+
+template <int R>
+void launch_rows(const CavityArgs& g, const double* src, double* dst, int depth,
+                 hipStream_t stream) {
+  // a shallower last round has fewer blocks
+  const int tx = span_count(g.nx - 2, 64, depth), ty = span_count(g.ny - 2, R * kWavesP, depth);
+  const dim3 grid(static_cast<unsigned>(tx) * ty), block(64 * kWavesP);
+  if (g.nx - 2 < 64 || g.ny - 2 < R * kWavesP)
+    hipLaunchKernelGGL((cavity_pressure<R, true>), grid, block, 0, stream, g, src, dst, depth,
+                       tx, ty);
+  else
+    hipLaunchKernelGGL((cavity_pressure<R, false>), grid, block, 0, stream, g, src, dst, depth,
+                       tx, ty);
+}
+
+int launch_pressure(const CavityArgs& g, int rows, const double* src, double* dst, int depth,
+                    hipStream_t stream) {
+  switch (rows) {
+    case 2: launch_rows<2>(g, src, dst, depth, stream); break;
+    case 3: launch_rows<3>(g, src, dst, depth, stream); break;
+    case 4: launch_rows<4>(g, src, dst, depth, stream); break;
+    default: launch_rows<6>(g, src, dst, depth, stream); break;
+  }
+  NPBX_LAUNCHED("cavity_pressure");
+  return NPBX_OK;
+}
+
+// The whole call in chip-wide launches: the source of the first step, then
+// per step its pressure rounds and one launch for its velocities and the next
+// step's source.  u, v and p alternate with scratch copies; where an odd
+// number of updates would leave them there, the first launch starts from a
+// copy so that the last one lands in the caller's arrays.
+int blocked_flow(const CavityArgs& a, hipStream_t stream) {
+  const PressurePlan pl = a.nit > 0 ? plan_pressure(a.nx, a.ny, a.nit) : PressurePlan{};
+  const int tiles_x = static_cast<int>(cdiv(a.nx - 2, kTileVJ));
+  const int64_t tiles = int64_t(tiles_x) * cdiv(a.ny - 2, kTileVI);
+  NPBX_REQUIRE(tiles < (int64_t(1) << 31), "cavity_flow: grid too large");
+  const size_t bytes = static_cast<size_t>(a.nx) * a.ny * sizeof(double);
+  const dim3 grid(static_cast<unsigned>(tiles)), block(1024);
+  double *ucur = a.u, *vcur = a.v, *ualt = a.un, *valt = a.vn;
+  double *pcur = a.p, *palt = a.pn;
+  if (static_cast<int64_t>(a.nt) * pl.rounds % 2) {
+    NPBX_HIP(hipMemcpyAsync(palt, pcur, bytes, hipMemcpyDeviceToDevice, stream));
+    std::swap(pcur, palt);
+  }
+  CavityArgs g = a;
+  g.un = ucur, g.vn = vcur;
+  if (a.nt % 2) std::swap(ucur, ualt), std::swap(vcur, valt);
+  g.u = ucur, g.v = vcur;
+  hipLaunchKernelGGL((cavity_velocity<false, true>), grid, block, 0, stream, g, pcur, tiles_x);
+  NPBX_LAUNCHED("cavity_velocity");
+  for (int step = 0; step < a.nt; ++step) {
+    for (int done = 0; done < a.nit; done += pl.depth) {
+      NPBX_TRY(launch_pressure(a, pl.rows, pcur, palt, std::min(pl.depth, a.nit - done), stream));
+      std::swap(pcur, palt);
+    }
+    g.un = ucur, g.vn = vcur, g.u = ualt, g.v = valt;
+    if (step + 1 < a.nt)
+      hipLaunchKernelGGL((cavity_velocity<true, true>), grid, block, 0, stream, g, pcur, tiles_x);
+    else
+      hipLaunchKernelGGL((cavity_velocity<true, false>), grid, block, 0, stream, g, pcur,
+                         tiles_x);
+    NPBX_LAUNCHED("cavity_velocity");
+    std::swap(ucur, ualt);
+    std::swap(vcur, valt);
+  }
+  return NPBX_OK;
+}
+
+// The one-workgroup form while the grid is at most a point per thread: a
+// phase then costs about 1 us.  50 steps of 5 / 20 iterations on the MI355X:
+// 25 x 25 402 / 1049 us against 499 / 1020 in blocks, 33 x 33 551 / 1354
+// against 527 / 1062, 61 x 61 955 / 2235 against 532 / 1064.
+bool use_lds(int64_t nx, int64_t ny) { return nx * ny <= kLdsPoints; }
+
 }  // namespace
 }  // namespace npbx
 
@@ -440,19 +752,15 @@ extern "C" int npbx_cavity_flow(int dtype, int64_t nx, int64_t ny, int64_t nt, i
   g.cpv = dt / (2.0 * rho * dy);
   g.cdx2 = dt / g.dx2;
   g.cdy2 = dt / g.dy2;
+  if (!use_lds(nx, ny)) return blocked_flow(g, as_stream(stream));
   // A time step depends on u, v and p only (b, un, vn are rebuilt each step),
   // so the steps split into launches of about 50 ms of work each: no launch
   // runs for long, whatever nt is.
   const int64_t per_launch = std::max<int64_t>(1, int64_t(150000000) / (np * (nit + 3)));
   for (int64_t done = 0; done < nt; done += per_launch) {
     g.nt = static_cast<int>(std::min<int64_t>(per_launch, nt - done));
-    if (np <= kLdsPoints) {
-      hipLaunchKernelGGL(cavity_flow_lds, dim3(1), dim3(kThreadsC), 0, as_stream(stream), g);
-      NPBX_LAUNCHED("cavity_flow_lds");
-    } else {
-      hipLaunchKernelGGL(cavity_flow_global, dim3(1), dim3(kThreadsC), 0, as_stream(stream), g);
-      NPBX_LAUNCHED("cavity_flow_global");
-    }
+    hipLaunchKernelGGL(cavity_flow_lds, dim3(1), dim3(kThreadsC), 0, as_stream(stream), g);
+    NPBX_LAUNCHED("cavity_flow_lds");
   }
   return NPBX_OK;
 }

@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "common.h"
+#include "lanes.h"
 #include "points.h"
 #include "vecio.h"
 
@@ -40,28 +41,6 @@ constexpr int kRI = kBI + 2 * kDeep;    // staged rows at the deepest launch
 
 std::atomic<int> g_jacobi_deep{kDeep};  // depth per launch; 0 or 1 = plain sweeps
 std::atomic<int> g_jacobi_deep_waves{0};  // waves per workgroup: 4, 8, 16 or 0 = by shape
-
-// Full-wave DPP shifts: lane l receives lane l-1's (from_left) or lane l+1's
-// (from_right) value; lanes 0 and 63 receive 0, which only lanes outside a
-// sweep's columns ever take.
-__device__ __forceinline__ int dpp_shr(int x) {
-  return __builtin_amdgcn_update_dpp(0, x, 0x138, 0xF, 0xF, true);
-}
-__device__ __forceinline__ int dpp_shl(int x) {
-  return __builtin_amdgcn_update_dpp(0, x, 0x130, 0xF, 0xF, true);
-}
-__device__ __forceinline__ float lane_from_left(float x) {
-  return __int_as_float(dpp_shr(__float_as_int(x)));
-}
-__device__ __forceinline__ float lane_from_right(float x) {
-  return __int_as_float(dpp_shl(__float_as_int(x)));
-}
-__device__ __forceinline__ double lane_from_left(double x) {
-  return __hiloint2double(dpp_shr(__double2hiint(x)), dpp_shr(__double2loint(x)));
-}
-__device__ __forceinline__ double lane_from_right(double x) {
-  return __hiloint2double(dpp_shl(__double2hiint(x)), dpp_shl(__double2loint(x)));
-}
 
 template <class S, int NW>
 __global__ __launch_bounds__(64 * NW) void jacobi2d_deep(const S* __restrict__ X,

@@ -83,6 +83,45 @@ def test_cavity_wide_grid(st):
           1.0, 0.1, f"{ny}x{nx}")
 
 
+@pytest.mark.parametrize("ny,nx", [(3, 700), (700, 3), (47, 45), (45, 64), (66, 201), (201, 65),
+                                   (300, 290)])
+@pytest.mark.parametrize("nt,nit", [(2, 1), (1, 2), (3, 7), (2, 20), (1, 24), (1, 25), (2, 51)])
+def test_cavity_blocked_bitwise(st, ny, nx, nt, nit):
+    """Grids past the one-workgroup form: several blocks per direction with
+    partial last ones, grids one block wide or one interior row high, one and
+    several launches per step of even and odd depth up to the deepest, and
+    odd and even update counts (the scratch copies' parity)."""
+    rng = np.random.default_rng(ny * 1000 + nx * 10 + nit)
+    u, v, p = rng.random((ny, nx)), rng.random((ny, nx)) - 0.5, rng.random((ny, nx))
+    check(st, nx, ny, nt, nit, u, v, p, 1.3, 0.07, f"blocked {ny}x{nx} nt={nt} nit={nit}")
+
+
+@pytest.mark.parametrize("case", ["rest", "tiny", "huge", "nan"])
+def test_cavity_blocked_division_range(st, case):
+    """Exact zeros take the short division; values past its range (a
+    pressure of 1e-290, one of 1e200, a NaN) the division operator."""
+    ny, nx = 70, 80
+    rng = np.random.default_rng(4)
+    u, v, p = np.zeros((ny, nx)), np.zeros((ny, nx)), np.zeros((ny, nx))
+    if case == "tiny":
+        p = 1e-290 * rng.random((ny, nx))
+    elif case == "huge":
+        p[30, 40] = 1e200
+    elif case == "nan":
+        p[30, 40] = np.nan
+    from npbench_amd import device
+    dx, dy, dt = grid(nx, ny)
+    want = [u.copy(), v.copy(), p.copy()]
+    with np.errstate(all="ignore"):
+        ref.cavity_flow(nx, ny, 2, 9, want[0], want[1], dt, dx, dy, want[2], 1.0, 0.1)
+    d = [device.to_device(a, torch.float64) for a in (u, v, p)]
+    print(f"cavity_flow range {case}", flush=True)
+    st.cavity_flow(nx, ny, 2, 9, d[0], d[1], dt, dx, dy, d[2], 1.0, 0.1)
+    torch.cuda.synchronize()
+    for name, g, w in zip(("u", "v", "p"), d, want):
+        np.testing.assert_array_equal(g.cpu().numpy(), w, err_msg=f"{case} {name}")
+
+
 def test_cavity_repeat_calls_restart_b(st):
     """b starts at zero on every call: a second, smaller call on other fields
     matches a fresh oracle run."""
