@@ -233,9 +233,9 @@ int npbx_pack_cols(int dtype, const void *A, const void *B, int64_t n,
  * levels -- the default where it applies), "hdiff.shape" = hdiff marching
  * shape (0, the default: by storage type; 1 .. 13: columns per lane, rows
  * per thread, bytes of k per lane),
- * "seidel.blocks" = wavefront
- * slot-blocks (slots x 256-column blocks) per seidel_2d launch (default 2048,
- * about 40 ms), "jacobi.deep" = 2-D Jacobi sweeps per launch at tblock <= 1
+ * "seidel.blocks" = tiles (64 rows of a
+ * group of 4 sweeps) per seidel_2d launch (default 2048; at most 4096 take
+ * effect), "jacobi.deep" = 2-D Jacobi sweeps per launch at tblock <= 1
  * (default 8: LDS-blocked, 64 x 48 points per workgroup; 0 or 1: one launch
  * per sweep), "jacobi.deep_waves" = its waves per workgroup (0, the default:
  * by shape; 4, 8 or 16).  Results do not depend on them. */
@@ -314,11 +314,11 @@ int npbx_channel_flow_launch(int dtype, int64_t nit, void *u, void *v,
 /* ---- 2-D Gauss-Seidel (seidel_2d_numpy.py:4-13) ----------------------------
  * A: (N, N) FP64 (dtype NPBX_F64), updated in place by TSTEPS - 1 sweeps;
  * bitwise the NumPy result.  N <= 16384; N < 3 or TSTEPS <= 1 is a no-op.
- * Rows run in wavefront slots (row i of sweep t with row i+2 of sweep t-1),
- * one workgroup, at most 64 sweeps per slot schedule; the rows of a slot run
- * their recurrences side by side, one lane each.  A launch runs a range of
- * slots of at most "seidel.blocks" slot-blocks, so its duration is bounded
- * whatever N is. */
+ * Tiles of 64 rows and 4 sweeps run as a wavefront over the whole device in
+ * launches of at most "seidel.blocks" tiles, so a launch's duration is bounded
+ * whatever N is.  Under stream capture (and on a device npbx_init was not
+ * called for) each wavefront step is a launch of its own.  Calls on different
+ * streams do not share state. */
 int npbx_seidel2d(int dtype, void *A, int64_t N, int64_t tsteps, void *stream);
 
 /* ---- alternating-direction implicit solver (adi_numpy.py:6-52) -------------

@@ -163,14 +163,18 @@ void set_adi_path(int path);
 // c' and d' in registers; 2 .. 4 where the shape allows them).
 int vadv_path();
 void set_vadv_path(int path);
-// Slot-blocks per seidel_2d launch ("seidel.blocks"; a slot-block is one
-// wavefront slot over one 256-column block).
+// Tiles per seidel_2d launch ("seidel.blocks"; a tile is 64 rows of a group of
+// sweeps).
 int seidel_blocks();
 void set_seidel_blocks(int blocks);
 
 // Resolves the current device's address of npbx_adi_noalloc's fixed scratch
 // array (once per device; npbx_init calls it).
 int adi_noalloc_setup();
+
+// Resolves the current device's seidel_2d counters (once per device;
+// npbx_init calls it).
+int seidel_setup();
 
 // Per-device scratch owned by the library (grow-only, freed at exit).  Used
 // by kernels that need storage beyond their inputs and outputs.

@@ -132,7 +132,8 @@ int npbx_init(int device) {
                 prop.gcnArchName);
   // Set-up of the allocation-free entry point: its fixed scratch array's
   // address on this device.
-  return npbx::adi_noalloc_setup();
+  NPBX_TRY(npbx::adi_noalloc_setup());
+  return npbx::seidel_setup();  // the seidel_2d tiles' counters
 }
 
 // Releases the library-owned workspace of the current device (after the

@@ -118,3 +118,76 @@ def test_seidel2d_largest_n(st):
     check(st, 3, rng.random((16384, 16384)), "n=16384 tsteps=3",
           oracle=c_oracle.seidel_2d_kernel)
 
+
+
+@pytest.mark.parametrize("n", [61, 62, 63, 64, 65, 66, 67, 125, 126, 127, 128, 129, 130, 131, 193])
+@pytest.mark.parametrize("tsteps", [2, 5, 6, 10])
+def test_seidel2d_tile_edges(st, n, tsteps):
+    """Row counts around the 64-row bands (which shift up by a row per sweep
+    of a group) and sweep counts around the groups of four, the last group
+    holding one, two and four sweeps."""
+    from oracle import c_oracle
+    rng = np.random.default_rng(n * 10 + tsteps)
+    check(st, tsteps, rng.random((n, n)), f"edges n={n} tsteps={tsteps}",
+          oracle=c_oracle.seidel_2d_kernel)
+
+
+@pytest.mark.parametrize("case", ["tiny", "huge", "zeros and signs"])
+def test_seidel2d_division_range(st, case):
+    """Values past the short division's range take the operator; zeros of
+    either sign stay on it."""
+    n = 140
+    rng = np.random.default_rng(2)
+    A = rng.random((n, n))
+    if case == "tiny":
+        A *= 1e-300
+    elif case == "huge":
+        A[70, 70] = 1e300
+    else:
+        A[20:120, 20:120] = np.where(rng.random((100, 100)) < 0.5, 0.0, -0.0)
+    from oracle import c_oracle
+    check(st, 6, A, case, oracle=c_oracle.seidel_2d_kernel)
+
+
+def test_seidel2d_two_streams(st):
+    """Calls in flight on two streams do not share state."""
+    from npbench_amd import device
+    from oracle import c_oracle
+    rng = np.random.default_rng(31)
+    grids = [rng.random((n, n)) for n in (150, 260, 150, 260)]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    dev_grids = [device.to_device(A, torch.float64) for A in grids]
+    torch.cuda.synchronize()
+    for rep in range(6):
+        for k, d in enumerate(dev_grids):
+            st.seidel2d(d, 9, stream=streams[k % 2])
+    torch.cuda.synchronize()
+    for A, d in zip(grids, dev_grids):
+        want = A.copy()
+        for rep in range(6):
+            c_oracle.seidel_2d_kernel(9, A.shape[0], want)
+        assert_bitwise(d.cpu().numpy(), want, f"two streams n={A.shape[0]}")
+
+
+@pytest.mark.parametrize("n,tsteps", [(50, 8), (200, 14)])
+def test_seidel2d_captured(st, n, tsteps):
+    """Under capture the tiles run slot by slot; every replay continues the
+    grid as an eager call does."""
+    from npbench_amd import device
+    from oracle import c_oracle
+    rng = np.random.default_rng(n)
+    want = rng.random((n, n))
+    d = device.to_device(want, torch.float64)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        st.seidel2d(d, tsteps)
+    for rep in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        c_oracle.seidel_2d_kernel(tsteps, n, want)
+        assert_bitwise(d.cpu().numpy(), want, f"replay {rep}")
+        st.seidel2d(d, tsteps)  # an eager call between the replays
+        torch.cuda.synchronize()
+        c_oracle.seidel_2d_kernel(tsteps, n, want)
+        assert_bitwise(d.cpu().numpy(), want, f"eager {rep}")
