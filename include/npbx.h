@@ -235,10 +235,10 @@ int npbx_pack_cols(int dtype, const void *A, const void *B, int64_t n,
  * per thread, bytes of k per lane),
  * "seidel.blocks" = tiles (64 rows of a
  * group of 4 sweeps) per seidel_2d launch (default 2048; at most 4096 take
- * effect), "jacobi.deep" = 2-D Jacobi sweeps per launch at tblock <= 1
- * (default 8: LDS-blocked, 64 x 48 points per workgroup; 0 or 1: one launch
- * per sweep), "jacobi.deep_waves" = its waves per workgroup (0, the default:
- * by shape; 4, 8 or 16).  Results do not depend on them. */
+ * effect), "jacobi.deep" = 2-D Jacobi sweeps per launch at
+ * tblock <= 1 (8, the default: up to 28, by size and type; 2 .. 7: at most
+ * that many; 0 or 1: one launch per sweep), "jacobi.deep_waves" = 0, 4, 8 or
+ * 16 (no effect: its workgroups have 16 waves).  Results do not depend on them. */
 int npbx_set_tuning(const char *key, int64_t value);
 int npbx_get_tuning(const char *key, int64_t *value);
 

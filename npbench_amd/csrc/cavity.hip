@@ -307,24 +307,6 @@ __device__ __forceinline__ double pressure_quotient(double n, const PressureDiv&
   }
 }
 
-// Where a block lies: its region's first grid row and column, and the rows
-// and columns [lo, hi) of the region it owns.
-struct Span {
-  int origin, lo, hi;
-};
-
-// Blocks of a direction with n interior points, `width` points per region:
-// regions at the grid's ends have no halo on that side; the last one is
-// shifted back to end with the grid.
-__host__ __device__ inline int span_count(int n, int width, int depth) {
-  return n <= width ? 1 : (n - 2 * depth + width - 2 * depth - 1) / (width - 2 * depth);
-}
-__device__ __forceinline__ Span span_of(int t, int count, int n, int width, int depth) {
-  const int out = width - 2 * depth;
-  const int o = t == count - 1 ? max(n - width, 0) : t * out;
-  return {1 + o, (t == 0 ? 0 : t * out + depth) - o, (t == count - 1 ? n : (t + 1) * out + depth) - o};
-}
-
 // One iteration of the wave's rows x into y (:30-37): ring[r] holds the
 // values west of lane 0 and east of lane 63, `top` and `bottom` the rows
 // outside the region (waves 0 and 15).

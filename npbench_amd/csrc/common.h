@@ -127,9 +127,9 @@ int tiled_sweeps(int kind, int dtype, void* A, void* B, int n, int64_t first, in
 // two levels ending in A and B as in the reference (tiles.hip).
 std::vector<int> sweep_rounds(int64_t nsweeps, int T);
 
-// 2-D Jacobi temporal-blocked in LDS (jacobi2d_deep.hip): sweeps per launch
-// ("jacobi.deep"; 0 or 1 = one launch per sweep), waves per workgroup
-// ("jacobi.deep_waves") and the sweeps themselves.
+// 2-D Jacobi temporal-blocked in registers (jacobi2d_deep.hip): sweeps per
+// launch ("jacobi.deep"; 0 or 1 = one launch per sweep, 8 = by shape), the
+// setting "jacobi.deep_waves" (no effect) and the sweeps themselves.
 int jacobi_deep_depth();
 void set_jacobi_deep_depth(int d);
 int jacobi_deep_waves();

@@ -1,28 +1,36 @@
-// 2-D Jacobi sweeps (jacobi_2d_numpy.py:4-10), temporal-blocked in LDS: a
-// launch advances every grid point by up to kDeep sweeps.
+// 2-D Jacobi sweeps (jacobi_2d_numpy.py:4-10), temporal-blocked in registers:
+// a launch advances every grid point by up to kMaxDepth sweeps.
 //
-// A workgroup owns an output block of kBI rows x kBJ columns and stages the
-// block plus a halo of d cells (d = the launch's depth) in LDS: d + kBI + d
-// rows of at most 64 columns, one wave-wide row, lanes along j.  Each sweep
-// recomputes the staged region shrunk by one cell per side into the other
-// LDS buffer, each of the workgroup's 4, 8 or 16 waves marching a band of
-// consecutive rows, and the last writes only the block to global memory: one read
-// of the region and one write of the block per d sweeps, and one launch
-// instead of d.  Region points on the grid's boundary take, at every level,
-// the value that level's boundary holds in the reference (A's at even
-// levels, B's at odd: the ping-pong never writes boundaries); points past
-// the grid are never read by a point that is computed.  Each level's values
-// are rounded through the storage type, as the plain sweep's stores round
-// them, and each point is jacobi_point -- the reference's
-// ((((c + W) + E) + S) + N) * 0.2 -- so results are bitwise the plain
-// sweeps' (FP64: the NumPy reference's).
+// A workgroup of 16 waves stacked along i holds a region of 16 R rows x 64 V
+// columns, each wave R rows and each lane V adjacent columns of them, and
+// sweeps it `depth` times in place.  Next to other blocks the outer `depth`
+// cells of the region are halo, recomputed by both and one cell less valid
+// per sweep; at the grid's edges the region ends with the interior.  West and
+// east neighbours are the adjacent lanes (full-wave DPP shifts, two per row
+// and sweep whatever V is), north and south the wave's own registers; a
+// wave's two edge rows go to its neighbours through LDS, one barrier per
+// sweep, written as soon as they are computed and read while the rows between
+// them are.
 //
-// Rounds follow sweep_rounds (tiles.hip): depths <= kDeep covering all but
-// the last sweep, their count of the parity that leaves the last two levels
-// in A and B as the reference does, then a depth-1 round.
+// The grid's boundary holds, at every level, what the level's array holds in
+// the reference (A's at even levels, B's at odd: the ping-pong never writes
+// boundaries): the outer lanes carry the two values of their row, which the
+// shifts hand in where the region ends (elsewhere they only reach the halo),
+// and the boundary rows lie in LDS.  NARROW: grids smaller than a region,
+// where the boundary falls inside it and is put back per point after each
+// sweep.  Each level is rounded through the storage type, as the plain
+// sweep's stores round it, and each point is jacobi_point -- the reference's
+// ((((c + W) + E) + S) + N) * 0.2 -- so results are bitwise the plain sweeps'
+// (FP64: the NumPy reference's).
+//
+// Rounds follow sweep_rounds (tiles.hip): depths <= T covering all but the
+// last sweep, their count of the parity that leaves the last two levels in A
+// and B as the reference does, then a depth-1 round.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <vector>
 
 #include "common.h"
@@ -33,124 +41,226 @@
 namespace npbx {
 namespace {
 
-constexpr int kDeep = 8;                // most sweeps per launch
-constexpr int kRJ = 64;                 // staged columns: one wave
-constexpr int kBJ = kRJ - 2 * kDeep;    // output columns per block
-constexpr int kBI = 64;                 // output rows per block
-constexpr int kRI = kBI + 2 * kDeep;    // staged rows at the deepest launch
+constexpr int kDeep = 8;       // "jacobi.deep": 8, the default, lets the shape choose
+constexpr int kMaxDepth = 28;  // most sweeps per launch
+constexpr int kWaves = 16;
 
-std::atomic<int> g_jacobi_deep{kDeep};  // depth per launch; 0 or 1 = plain sweeps
-std::atomic<int> g_jacobi_deep_waves{0};  // waves per workgroup: 4, 8, 16 or 0 = by shape
+std::atomic<int> g_jacobi_deep{kDeep};    // 0 or 1 = plain sweeps
+std::atomic<int> g_jacobi_deep_waves{0};  // accepted; the kernel has 16 waves
 
-template <class S, int NW>
-__global__ __launch_bounds__(64 * NW) void jacobi2d_deep(const S* __restrict__ X,
+// A wave's rows of one level.
+template <class C, int V, int R>
+struct Rows {
+  C v[R][V];
+};
+
+// Rows [r0, r1) of the next level y from x; above and below are the rows
+// outside the wave's, ring its rows' values west of lane 0 and east of lane 63.
+template <class S, int V, int R, class C = typename Storage<S>::C>
+__device__ __forceinline__ void sweep_rows(const Rows<C, V, R>& x, Rows<C, V, R>& y, int r0,
+                                           int r1, const C (&above)[V], const C (&below)[V],
+                                           const C (&ring)[R]) {
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (r < r0 || r >= r1) continue;
+    const C west = lane_from_left_or(ring[r], x.v[r][V - 1]);
+    const C east = lane_from_right_or(ring[r], x.v[r][0]);
+#pragma unroll
+    for (int c = 0; c < V; ++c)
+      y.v[r][c] = Storage<S>::load(Storage<S>::store(jacobi_point<C>(
+          x.v[r][c], c == 0 ? west : x.v[r][c - 1], c == V - 1 ? east : x.v[r][c + 1],
+          r == R - 1 ? below[c] : x.v[r + 1][c], r == 0 ? above[c] : x.v[r - 1][c])));
+  }
+}
+
+template <class S, int V, int R, bool NARROW>
+__global__ __launch_bounds__(64 * kWaves) void jacobi2d_block(const S* __restrict__ X,
                                                               S* __restrict__ Y,
                                                               const S* __restrict__ A,
                                                               const S* __restrict__ B, int n,
-                                                              int parity0, int depth,
-                                                              int tiles_j) {
+                                                              int parity0, int depth, int tiles_j,
+                                                              int tiles_i) {
   using St = Storage<S>;
   using C = typename St::C;
-  __shared__ C buf[2][kRI * kRJ];
+  struct alignas(sizeof(C) * V) Cols {
+    C v[V];
+  };
+  __shared__ Cols edge[2][kWaves][2][64];  // per level parity: each wave's first and last row
+  __shared__ Cols outer[2][2][64];         // per level parity: the rows above and below the region
   const int lane = threadIdx.x % 64;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);  // wave-uniform
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
-  const int ti = tile / tiles_j, tj = tile % tiles_j;
-  const int d = depth;
-  const int ri = kBI + 2 * d, rj = kBJ + 2 * d;
-  const int oi = 1 + ti * kBI - d, oj = 1 + tj * kBJ - d;  // grid point of region (0, 0)
-  const int gj = oj + lane;
-  const bool col_in = lane < rj && gj >= 0 && gj < n;
-  const bool col_bnd = gj == 0 || gj == n - 1;
-  auto bnd = [&](int level) { return ((parity0 + level) & 1) ? B : A; };
+  const Span sj = span_of(tile % tiles_j, tiles_j, n - 2, 64 * V, depth);
+  const Span si = span_of(tile / tiles_j, tiles_i, n - 2, R * kWaves, depth);
+  const int gj = sj.origin + lane * V, gi0 = si.origin + w * R;
+  const S* const bnd[2] = {parity0 ? B : A, parity0 ? A : B};
 
-  // Level 0 into buf[0]: interior points from X, boundary points from the
-  // level's array; and buf[1]'s boundary points from the other array.  A
-  // buffer holds levels of one parity only (level s in buf[s & 1]) and the
-  // sweeps write interior points only, so every level finds its boundary in
-  // place.  Addresses are clamped into the grid, so the loads are
-  // unconditional (values loaded for points past the grid are never read).
-  // All of a wave's loads are issued before the first LDS store, so their
-  // latencies overlap.
-  const bool touches = oi <= 0 || oj <= 0 || oi + ri >= n || oj + rj >= n;
-  const int gjc = min(max(gj, 0), n - 1);
-  constexpr int kLoadRows = (kRI + NW - 1) / NW;
-  C v[kLoadRows];
+  // Level 0, clamped into the grid in a NARROW one (where what lies past its
+  // edge is replaced below), the two boundary values of each row (lanes 0 and
+  // 63) and the rows outside the region.
+  auto at = [&](int i, int j) {
+    return static_cast<int64_t>(min(i, n - 1)) * n + (NARROW ? min(j, n - 1) : j);
+  };
+  Rows<C, V, R> x, y;
+  C ring[2][R];
 #pragma unroll
-  for (int k = 0; k < kLoadRows; ++k) {
-    const int r = w + k * NW;
-    if (r < ri) {
-      const int gi = oi + r;
-      const int64_t at = static_cast<int64_t>(min(max(gi, 0), n - 1)) * n + gjc;
-      const bool edge = col_bnd || gi == 0 || gi == n - 1;
-      v[k] = St::load((edge ? bnd(0) : X)[at]);
-    }
+  for (int r = 0; r < R; ++r) {
+#pragma unroll
+    for (int c = 0; c < V; ++c) x.v[r][c] = St::load(X[at(gi0 + r, gj + c)]);
   }
+  // (lanes 0 and 63 use them; two addresses for the wave)
+  const int gr = lane < 32 ? sj.origin - 1 : min(sj.origin + 64 * V, n - 1);
 #pragma unroll
-  for (int k = 0; k < kLoadRows; ++k) {
-    const int r = w + k * NW;
-    if (r < ri) buf[0][r * kRJ + lane] = v[k];
+  for (int p = 0; p < 2; ++p) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      ring[p][r] = St::load(bnd[p][static_cast<int64_t>(min(gi0 + r, n - 1)) * n + gr]);
   }
-  if (touches) {
+  if (w < 4) {  // (parity, side) = (w / 2, w % 2)
+    Cols o;
+    const int i = w % 2 ? min(si.origin + R * kWaves, n - 1) : si.origin - 1;
 #pragma unroll
-    for (int k = 0; k < kLoadRows; ++k) {
-      const int r = w + k * NW;
-      if (r < ri) {
-        const int gi = oi + r;
-        const int64_t at = static_cast<int64_t>(min(max(gi, 0), n - 1)) * n + gjc;
-        v[k] = St::load(bnd(1)[at]);
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < kLoadRows; ++k) {
-      const int r = w + k * NW;
-      const int gi = oi + r;
-      if (r < ri && (col_bnd || gi == 0 || gi == n - 1)) buf[1][r * kRJ + lane] = v[k];
-    }
+    for (int c = 0; c < V; ++c) o.v[c] = St::load(bnd[w / 2][at(i, gj + c)]);
+    outer[w / 2][w % 2][lane] = o;
   }
+  // NARROW: the boundary's values at the region's points that lie on it
+  C fixed[2][NARROW ? R : 1][V];
+  if constexpr (NARROW) {
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int c = 0; c < V; ++c) fixed[p][r][c] = St::load(bnd[p][at(gi0 + r, gj + c)]);
+  }
+  auto put_boundary = [&](Rows<C, V, R>& z, int p) {
+    if constexpr (NARROW) {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int c = 0; c < V; ++c)
+          if (gi0 + r >= n - 1 || gj + c >= n - 1) z.v[r][c] = fixed[p][r][c];
+    }
+  };
+  auto publish = [&](const Rows<C, V, R>& z, int p) {
+    Cols first, last;
+#pragma unroll
+    for (int c = 0; c < V; ++c) first.v[c] = z.v[0][c], last.v[c] = z.v[R - 1][c];
+    edge[p][w][0][lane] = first;
+    edge[p][w][1][lane] = last;
+  };
+  put_boundary(x, 0);
+  publish(x, 0);
   __syncthreads();
 
-  // Each wave marches a band of consecutive rows, keeping the rows above and
-  // at its point in registers: one LDS read (the row below) per point, the
-  // west and east neighbours from the adjacent lanes (full-wave DPP shifts),
-  // and the next row's read issued before the current row is computed.
-  // Every lane takes part in the reads and shifts (lanes outside the
-  // sweep's columns supply neighbours); only lanes on interior points inside
-  // the sweep's region write.
-  for (int s = 1; s <= d; ++s) {
-    const C* __restrict__ src = buf[(s - 1) & 1];
-    C* __restrict__ dst = buf[s & 1];
-    const bool lane_on = col_in && !col_bnd && lane >= s && lane < rj - s;
-    const int rows = ri - 2 * s;
-    const int h = (rows + NW - 1) / NW;
-    // the wave's band, clipped to the grid's interior rows
-    const int r0 = max(s + w * h, 1 - oi), r1 = min(min(s + (w + 1) * h, ri - s), n - 1 - oi);
-    if (r0 < r1) {
-      C north = src[(r0 - 1) * kRJ + lane];
-      C centre = src[r0 * kRJ + lane];
-      C south = src[(r0 + 1) * kRJ + lane];
-      for (int r = r0; r < r1; ++r) {
-        const C next = src[min(r + 2, ri - 1) * kRJ + lane];  // row r+2, for the next step
-        const C west = lane_from_left(centre), east = lane_from_right(centre);
-        if (lane_on)
-          dst[r * kRJ + lane] = St::load(St::store(jacobi_point<C>(centre, west, east, south,
-                                                                   north)));
-        north = centre;
-        centre = south;
-        south = next;
-      }
+  const int useful = si.useful(w * R, w * R + R);
+  // One sweep from z (level parity p) into q.  The neighbours' edge rows are
+  // asked for first; rows that need none of them are computed meanwhile, half
+  // before and half after this wave's own edge rows are published.
+  auto sweep = [&](const Rows<C, V, R>& z, Rows<C, V, R>& q, int p, int s) {
+    if (s + 1 >= useful) {  // only halo rows that nothing valid reads any more
+      __syncthreads();
+      return;
+    }
+    const Cols a = w == 0 ? outer[p][0][lane] : edge[p][w - 1][1][lane];
+    const Cols b = w == kWaves - 1 ? outer[p][1][lane] : edge[p][w + 1][0][lane];
+    constexpr int kMid = (R + 1) / 2;
+    sweep_rows<S, V, R>(z, q, 1, R > 2 ? kMid : 1, a.v, b.v, ring[p]);
+    __builtin_amdgcn_sched_barrier(0);
+    sweep_rows<S, V, R>(z, q, 0, 1, a.v, b.v, ring[p]);
+    if (R > 1) sweep_rows<S, V, R>(z, q, R - 1, R, a.v, b.v, ring[p]);
+    if constexpr (!NARROW) publish(q, p ^ 1);
+    __builtin_amdgcn_sched_barrier(0);
+    sweep_rows<S, V, R>(z, q, R > 2 ? kMid : 1, R - 1, a.v, b.v, ring[p]);
+    if constexpr (NARROW) {
+      put_boundary(q, p ^ 1);
+      publish(q, p ^ 1);
     }
     __syncthreads();
+  };
+  int s = 0;
+  for (; s + 2 <= depth; s += 2) {
+    sweep(x, y, 0, s);
+    sweep(y, x, 1, s + 1);
+  }
+  if (s < depth) {
+    sweep(x, y, 0, s);
+    x = y;
   }
 
-  // the block's interior points of level d
-  const C* fin = buf[d & 1];
-  const bool lane_out = lane >= d && lane < d + kBJ && gj >= 1 && gj <= n - 2;
-  for (int r = d + w; r < d + kBI; r += NW) {
-    const int gi = oi + r;
-    if (!lane_out || gi < 1 || gi > n - 2) continue;
-    Y[static_cast<int64_t>(gi) * n + gj] = St::store(fin[r * kRJ + lane]);
+  // the block's points of level `depth`
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int gi = gi0 + r, k = w * R + r;
+    if (k < si.lo || k >= si.hi || gi > n - 2) continue;
+    S* to = Y + static_cast<int64_t>(gi) * n + gj;
+#pragma unroll
+    for (int c = 0; c < V; ++c) {
+      const int l = lane * V + c;
+      if (l >= sj.lo && l < sj.hi && gj + c <= n - 2) to[c] = St::store(x.v[r][c]);
+    }
   }
+}
+
+// Launch shape: columns per lane, rows per wave and sweeps per launch.
+struct Shape {
+  int v, rows, depth;
+};
+
+constexpr Shape kShapes[] = {{1, 3, 0}, {1, 4, 0}, {2, 3, 0}, {2, 4, 0},
+                             {2, 5, 0}, {2, 6, 0}, {2, 8, 0}};
+
+// The shape and depth with the smallest modelled time: 5.4 us a launch; per
+// sweep 0.06 us plus 9 ns per instruction of a wave's rows that is not idle
+// halo, times the workgroups a CU runs; and where a CU holds one workgroup at
+// a time (more than 64 VGPRs: over 8 FP64 points a lane), its loads, about
+// 10 us, for each further one.  The constants are fitted to 200 measured
+// (shape, size, type) times, 10 % off on average; the shapes of the fastest:
+// FP64 150^2 1 x 3 rows, depth 20 (52 us for 98 sweeps, 2 x 8: 167); 1000^2
+// 2 x 5, 19 (204 us for 200; 1 x 3: 626); 2800^2 2 x 4, 12 (513 us for 100;
+// 2 x 8: 717).
+Shape pick_shape(int dtype, int n, int64_t nsweeps, int cap) {
+  Shape best{2, 4, 2};
+  double best_us = INFINITY;
+  const bool fp64 = dtype == NPBX_F64;
+  for (const Shape& sh : kShapes) {
+    const int wj = 64 * sh.v, wi = kWaves * sh.rows;
+    const double issue =
+        sh.rows * (5.0 * sh.v + (fp64 ? 4 : 2) + (dtype == NPBX_BF16 ? 2.0 * sh.v : 0));
+    const int resident = fp64 && sh.rows * sh.v > 8 ? 1 : 2;
+    for (int depth = std::min(cap, 4); depth <= std::min(cap, kMaxDepth); depth += 2) {
+      if (wj - 2 * depth < 8 || wi - 2 * depth < 8) break;
+      // sweep_rounds: that many rounds and a last one of depth 1
+      int64_t rounds = cdiv(nsweeps - 1, depth);
+      rounds += (rounds ^ (nsweeps - 1)) & 1;
+      const int d = static_cast<int>(cdiv(nsweeps - 1, std::max<int64_t>(rounds, 1)));
+      const double tiles =
+          static_cast<double>(span_count(n - 2, wj, d)) * span_count(n - 2, wi, d) / 256;
+      const double shared = std::min<double>(resident, std::ceil(tiles));
+      const double turns = std::max(1.0, (tiles / shared + std::ceil(tiles / shared)) / 2);
+      const double sweep = 0.06 + 0.0091 * issue * (1.0 - static_cast<double>(d) / wi) * shared;
+      const double us = static_cast<double>(rounds) *
+                        (5.4 + turns * d * sweep + (turns - 1) * (resident == 1 ? 10 : 2.5));
+      if (us < best_us) {
+        best_us = us;
+        best = {sh.v, sh.rows, depth};
+      }
+    }
+  }
+  return best;
+}
+
+template <class S, int V, int R>
+void launch_shape(const S* X, S* Y, const S* A, const S* B, int n, int parity, int depth,
+                  hipStream_t stream) {
+  const int tj = span_count(n - 2, 64 * V, depth), ti = span_count(n - 2, R * kWaves, depth);
+  const dim3 grid(static_cast<unsigned>(int64_t(tj) * ti)), block(64 * kWaves);
+  if (n - 2 < 64 * V || n - 2 < R * kWaves)
+    hipLaunchKernelGGL((jacobi2d_block<S, V, R, true>), grid, block, 0, stream, X, Y, A, B, n,
+                       parity, depth, tj, ti);
+  else
+    hipLaunchKernelGGL((jacobi2d_block<S, V, R, false>), grid, block, 0, stream, X, Y, A, B, n,
+                       parity, depth, tj, ti);
 }
 
 }  // namespace
@@ -161,21 +271,12 @@ int jacobi_deep_waves() { return g_jacobi_deep_waves.load(); }
 void set_jacobi_deep_waves(int w) { g_jacobi_deep_waves.store(w); }
 int jacobi_deep_max() { return kDeep; }
 
-// Sweeps [first, first + nsweeps) of one grid through the LDS-blocked kernel
-// at depth <= T (2 .. kDeep) per launch.
+// Sweeps [first, first + nsweeps) of one grid in blocks, T the "jacobi.deep"
+// setting (2 .. 7: at most that many sweeps per launch; 8: by shape).
 int jacobi_deep_sweeps(int dtype, void* A, void* B, int n, int64_t first, int64_t nsweeps, int T,
                        hipStream_t stream) {
   NPBX_REQUIRE(T >= 2 && T <= kDeep, "jacobi.deep=%d outside [2, %d]", T, kDeep);
-  const int tiles_i = static_cast<int>(cdiv(n - 2, kBI));
-  const int tiles_j = static_cast<int>(cdiv(n - 2, kBJ));
-  const int64_t ntiles = int64_t(tiles_i) * tiles_j;
-  NPBX_REQUIRE(ntiles < (int64_t(1) << 31), "jacobi2d: too many tiles");
-  // By shape: 16 waves while the grid has at most two blocks per CU or the
-  // staged region is FP64 (80 KiB of LDS: two workgroups per CU), else 8
-  // (four 40 KiB workgroups per CU, so the same 32 waves in smaller barrier
-  // groups).
-  int waves = jacobi_deep_waves();
-  if (waves == 0) waves = (ntiles <= 2 * 256 || dtype == NPBX_F64) ? 16 : 8;
+  const Shape shape = pick_shape(dtype, n, nsweeps, T == kDeep ? kMaxDepth : T);
   return dispatch_dtype(dtype, [&](auto tag) -> int {
     using S = decltype(tag);
     S* a = static_cast<S*>(A);
@@ -184,20 +285,20 @@ int jacobi_deep_sweeps(int dtype, void* A, void* B, int n, int64_t first, int64_
     // the first round reads the array that holds level `first`; each round
     // writes the other array and the next reads it
     S* X = (first & 1) ? b : a;
-    for (int depth : sweep_rounds(nsweeps, T)) {
+    for (int depth : sweep_rounds(nsweeps, shape.depth)) {
       S* Y = X == a ? b : a;
       const int parity = static_cast<int>(level & 1);
-      const unsigned blocks = static_cast<unsigned>(ntiles);
-      if (waves == 4)
-        hipLaunchKernelGGL((jacobi2d_deep<S, 4>), dim3(blocks), dim3(256), 0, stream, X, Y, a, b,
-                           n, parity, depth, tiles_j);
-      else if (waves == 8)
-        hipLaunchKernelGGL((jacobi2d_deep<S, 8>), dim3(blocks), dim3(512), 0, stream, X, Y, a, b,
-                           n, parity, depth, tiles_j);
-      else
-        hipLaunchKernelGGL((jacobi2d_deep<S, 16>), dim3(blocks), dim3(1024), 0, stream, X, Y, a,
-                           b, n, parity, depth, tiles_j);
-      NPBX_LAUNCHED("jacobi2d_deep");
+      auto go = [&](auto launch) { launch(X, Y, a, b, n, parity, depth, stream); };
+      switch (shape.v * 10 + shape.rows) {
+        case 13: go(launch_shape<S, 1, 3>); break;
+        case 14: go(launch_shape<S, 1, 4>); break;
+        case 23: go(launch_shape<S, 2, 3>); break;
+        case 24: go(launch_shape<S, 2, 4>); break;
+        case 25: go(launch_shape<S, 2, 5>); break;
+        case 26: go(launch_shape<S, 2, 6>); break;
+        default: go(launch_shape<S, 2, 8>); break;
+      }
+      NPBX_LAUNCHED("jacobi2d_block");
       X = Y;
       level += depth;
     }

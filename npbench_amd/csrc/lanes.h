@@ -1,7 +1,10 @@
-// Neighbour exchange between the lanes of a wave.
+// Neighbour exchange between the lanes of a wave, and the blocks of kernels
+// that advance a grid several sweeps per launch.
 #pragma once
 
 #include <hip/hip_runtime.h>
+
+#include <climits>
 
 namespace npbx {
 
@@ -35,11 +38,44 @@ __device__ __forceinline__ double dpp_or(double edge, double x) {
       __builtin_amdgcn_update_dpp(__double2hiint(edge), __double2hiint(x), CTRL, 0xF, 0xF, false),
       __builtin_amdgcn_update_dpp(__double2loint(edge), __double2loint(x), CTRL, 0xF, 0xF, false));
 }
-__device__ __forceinline__ double lane_from_left_or(double edge, double x) {
+template <int CTRL>
+__device__ __forceinline__ float dpp_or(float edge, float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(edge), __float_as_int(x), CTRL,
+                                                    0xF, 0xF, false));
+}
+template <class C>
+__device__ __forceinline__ C lane_from_left_or(C edge, C x) {
   return dpp_or<0x138>(edge, x);
 }
-__device__ __forceinline__ double lane_from_right_or(double edge, double x) {
+template <class C>
+__device__ __forceinline__ C lane_from_right_or(C edge, C x) {
   return dpp_or<0x130>(edge, x);
+}
+
+// A direction of a grid split into blocks that advance several sweeps per
+// launch: n interior points, regions of `width` points held by a workgroup,
+// halos of `depth` points where a region ends inside the grid and none where
+// it ends with it.  Block t of `count` has its region's first interior point
+// at grid index origin (from 1) and owns the region's points [lo, hi); the
+// last region is shifted back to end with the grid.
+struct Span {
+  int origin, lo, hi;
+  int width, first, last;  // first, last: whether the region ends with the grid
+  // The sweeps, counted from 1, from which on none of the region's points
+  // [from, to) is needed: a halo is valid for one cell less each sweep.
+  __device__ __forceinline__ int useful(int from, int to) const {
+    return min(first ? INT_MAX : to, last ? INT_MAX : width - from);
+  }
+};
+__host__ __device__ inline int span_count(int n, int width, int depth) {
+  const int out = width - 2 * depth;
+  return n <= width ? 1 : (n - 2 * depth + out - 1) / out;
+}
+__device__ __forceinline__ Span span_of(int t, int count, int n, int width, int depth) {
+  const int out = width - 2 * depth;
+  const int o = t == count - 1 ? max(n - width, 0) : t * out;
+  return {1 + o, (t == 0 ? 0 : t * out + depth) - o,
+          (t == count - 1 ? n : (t + 1) * out + depth) - o, width, t == 0, t == count - 1};
 }
 
 }  // namespace npbx

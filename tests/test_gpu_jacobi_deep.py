@@ -72,3 +72,20 @@ def test_deep_fp64_1000_is_the_oracle(st, deep):
     print("jacobi deep f64 1000^2 200 sweeps", flush=True)
     a, b = run(st, A, B, "f64", 200, 0)
     assert np.array_equal(a.cpu().numpy(), ra) and np.array_equal(b.cpu().numpy(), rb)
+
+
+@pytest.mark.parametrize("dt", ["f64", "f32", "bf16"])
+@pytest.mark.parametrize("n,nsweeps,first", [(65, 60, 0), (66, 31, 1), (150, 98, 0), (351, 57, 0),
+                                             (699, 44, 1), (1001, 39, 0), (2111, 27, 0)])
+def test_deep_default_shape_matches_plain_sweeps(st, deep, dt, n, nsweeps, first):
+    """The shape and depth the size picks (a grid's blocks from one to many
+    per direction, partial halos, rows of any alignment)."""
+    from npbench_amd import device
+    rng = np.random.default_rng(n + nsweeps)
+    A, B = rng.random((n, n)), rng.random((n, n))
+    deep(0)
+    pa, pb = run(st, A, B, dt, nsweeps, first)
+    deep(8, 0)
+    print(f"jacobi default shape {dt} n={n} sweeps={nsweeps} first={first}", flush=True)
+    da, db = run(st, A, B, dt, nsweeps, first)
+    assert torch.equal(da, pa) and torch.equal(db, pb)
