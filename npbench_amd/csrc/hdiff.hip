@@ -17,8 +17,9 @@
 // Same operations in the same order as the reference, so FP64 is bitwise
 // NumPy.
 //
-// Fallback (hdiff_kernel, K not a multiple of V or unaligned arrays): one
-// output point per thread, the Laplacians rebuilt from 13 cached loads.
+// Fallback (hdiff_kernel, fields narrower than a group of columns or columns
+// shorter than a vector): one output point per thread, the Laplacians rebuilt
+// from 13 cached loads.
 // The limiter keeps the reference test "r * grad > 0 -> 0".
 //
 // Iterated form (nsteps > 1, build-defined): step n reads the previous
@@ -143,8 +144,13 @@ __global__ __launch_bounds__(256) void hdiff_copy_halo(const S* __restrict__ src
 // group is shifted left to end at column J-1 (J >= W) and stores only its
 // own columns, so every column is stored once and every load is in the
 // field.  Prefetched vectors are held as raw storage words until the row
-// that uses them.
-template <class S, int W, int STRIP, int VB>
+// that uses them.  The output is stored around the caches' allocation: kept
+// lines of it would push out the inputs that later rows and calls read (FP32
+// 256 x 256 x 160 with three operand sets in turn 29.9 -> 20.4 us, FP64 57.6
+// -> 54.8; with one set, cached inputs, FP32 20.6 -> 20.4, FP64 40.0 -> 38.5).
+// TAIL: a column's last vector is shifted back to end with it (what two lanes
+// store there is the same) and addresses are aligned to elements only.
+template <class S, int W, int STRIP, int VB, bool TAIL = false>
 __global__ __launch_bounds__(256) void hdiff_march(const S* __restrict__ in, S* __restrict__ out,
                                                    const S* __restrict__ coeff, int I, int J,
                                                    int K, int xblocks, S* __restrict__ halo_dst) {
@@ -155,19 +161,25 @@ __global__ __launch_bounds__(256) void hdiff_march(const S* __restrict__ in, S* 
   using Raw = RawVec<S, V>;
   const int b = xcd_tile(blockIdx.x, gridDim.x);
   const int xb = b % xblocks, strip = b / xblocks;
-  const int kvs = K / V;
+  const int kvs = TAIL ? (K + V - 1) / V : K / V;
   const int groups = (J + W - 1) / W;
   const int t = xb * 256 + threadIdx.x;
   if (t >= groups * kvs) return;
   const int yn = (t / kvs) * W;     // the group's first column
   const int y0 = min(yn, J - W);    // first column computed
-  const int k0 = (t % kvs) * V;
+  const int k0 = TAIL ? min((t % kvs) * V, K - V) : (t % kvs) * V;
   const int x0 = strip * STRIP, x1 = min(x0 + STRIP, I);
   const int64_t si = static_cast<int64_t>(J + 4) * K;  // in-field row stride
   // in-field column y0 + c, c = 0 .. W+3: far left, side left, the W own
   // columns, side right, far right
   const S* __restrict__ base = in + static_cast<int64_t>(y0) * K + k0;
-  auto ld = [&](int p, int c, Raw& r) { loadraw<S, V>(base + p * si + c * K, r); };
+  auto load = [](const S* p, Raw& r) {
+    if constexpr (TAIL)
+      loadraw_any<S, V>(p, r);
+    else
+      loadraw<S, V>(p, r);
+  };
+  auto ld = [&](int p, int c, Raw& r) { load(base + p * si + c * K, r); };
   auto lap = [](C c, C ip, C im, C jp, C jm) {
     C nb = ip + im;
     nb = nb + jp;
@@ -235,7 +247,7 @@ __global__ __launch_bounds__(256) void hdiff_march(const S* __restrict__ in, S* 
   ld(p0, W + 3, nfar[1]);
   const S* __restrict__ cfp = coeff + (static_cast<int64_t>(x0) * J + y0) * K + k0;
 #pragma unroll
-  for (int w = 0; w < W; ++w) loadraw<S, V>(cfp + w * K, ncf[w]);
+  for (int w = 0; w < W; ++w) load(cfp + w * K, ncf[w]);
 
   // One output row x (in-field row p = x + 2): o0/o1/o2 hold the own rows
   // p, p+1, p+2 (o2 filled here), s0/s1/s2 the side rows p-1, p, p+1 (s2
@@ -265,7 +277,7 @@ __global__ __launch_bounds__(256) void hdiff_march(const S* __restrict__ in, S* 
       ld(pn, W + 3, nfar[1]);
       const S* nc = cfp + static_cast<int64_t>(pn - 2 - x0) * J * K;
 #pragma unroll
-      for (int w = 0; w < W; ++w) loadraw<S, V>(nc + w * K, ncf[w]);
+      for (int w = 0; w < W; ++w) load(nc + w * K, ncf[w]);
     }
     C res[W][V];
 #pragma unroll
@@ -304,10 +316,15 @@ __global__ __launch_bounds__(256) void hdiff_march(const S* __restrict__ in, S* 
 #pragma unroll
     for (int w = 0; w < W; ++w) {
       if (y0 + w < yn) continue;  // stored by the group to the left
-      if (halo_dst)
-        storev<S, V>(halo_dst + p * si + static_cast<int64_t>(y0 + w + 2) * K + k0, res[w]);
-      else
-        storev<S, V>(out + (static_cast<int64_t>(x) * J + y0 + w) * K + k0, res[w]);
+      if (halo_dst) {  // the next step's input
+        S* to = halo_dst + p * si + static_cast<int64_t>(y0 + w + 2) * K + k0;
+        if constexpr (TAIL)
+          storev_any<S, V>(to, res[w]);
+        else
+          storev<S, V>(to, res[w]);
+      } else {
+        storev_stream<S, V, TAIL>(out + (static_cast<int64_t>(x) * J + y0 + w) * K + k0, res[w]);
+      }
     }
   };
   // Fully unrolled: the slots rotate and the carried values change
@@ -324,26 +341,34 @@ __global__ __launch_bounds__(256) void hdiff_march(const S* __restrict__ in, S* 
   }
 }
 
-// Marching shapes (tuning knob "hdiff.shape"): {W columns per lane, STRIP
-// rows per thread, VB bytes of k per lane}; a shape whose vector is
-// narrower than one element (4 bytes of FP64) runs the storage type's
-// default.
+// Marching shapes (tuning knob "hdiff.shape", 1 .. 13; 14 is the FP64
+// default): {W columns per lane, STRIP rows per thread, VB bytes of k per
+// lane}.
 struct MarchShape {
   int w, strip, vb;
 };
 constexpr MarchShape kMarchShapes[] = {{0, 0, 0},   {1, 12, 16}, {1, 6, 16}, {2, 6, 16},
                                        {2, 12, 16}, {1, 18, 16}, {4, 6, 8},  {2, 6, 8},
                                        {4, 12, 8},  {4, 6, 4},   {4, 12, 4}, {2, 12, 8},
-                                       {2, 12, 4},  {3, 6, 8}};
-constexpr int kMarchShapeCount = sizeof(kMarchShapes) / sizeof(kMarchShapes[0]);
+                                       {2, 12, 4},  {3, 6, 8},   {4, 4, 8}};
+constexpr int kMarchShapeCount = 14;  // of the knob
 std::atomic<int> g_hdiff_shape{0};
 
-// Default shape per storage type (knob value 0), the fastest at 256 x 256 x
-// 160 on the MI355X: FP64 and FP32 2 columns x 6 rows with 8-byte vectors,
-// BF16 4 x 6 with 4-byte vectors (two elements: the four columns' window
-// then fits in 110 VGPRs, four waves per SIMD).
+// The shapes a call tries in turn; the first that fits runs: no wider than J,
+// columns of k whole vectors, arrays aligned to them.  The first of each type
+// is the fastest of 22 shapes on the MI355X over calls whose operands change
+// (three sets in turn; us, streaming stores): 256 x 256 x 160 FP64 4 x 4 x 8 B
+// 50.2 (2 x 6 x 8: 54.8, 4 x 6 x 8: 51.2), FP32 2 x 6 x 8 20.4 (4 x 4 x 8:
+// 21.5, 4 x 6 x 4: 27.0), BF16 4 x 6 x 4 14.8 (2 x 6 x 8: 15.0).  An odd K
+// leaves FP32 the 4-byte vectors (190 x 203 x 137: 13.4; a point per thread
+// 28.8) and BF16 the tail form of its own.
 template <class S>
-constexpr int default_march_shape() { return sizeof(S) == 2 ? 9 : 7; }
+constexpr int march_order(int n) {
+  constexpr int f64[] = {14, 7, 1}, f32[] = {7, 9, 12, 1}, b16[] = {9, 12, 1};
+  if (sizeof(S) == 8) return n < 3 ? f64[n] : 0;
+  if (sizeof(S) == 4) return n < 4 ? f32[n] : 0;
+  return n < 3 ? b16[n] : 0;
+}
 
 // ---------------------------------------------------------------- fused steps
 // hdiff_tb<S, TB>: up to TB iterated steps in one HBM round trip.  A
@@ -766,15 +791,30 @@ constexpr int hdiff_tb_max() { return sizeof(S) == 2 ? 2 : 4; }  // BF16 x4 exce
 template <class S>
 int run_hdiff(const S* in, S* out, const S* coeff, int I, int J, int K, int64_t nsteps,
               hipStream_t stream) {
+  auto aligned_to = [&](int bytes) {
+    auto ok = [&](const void* p) { return reinterpret_cast<uintptr_t>(p) % bytes == 0; };
+    return ok(in) && ok(out) && ok(coeff);
+  };
+  auto fits = [&](int sh) {
+    const MarchShape& m = kMarchShapes[sh];
+    return m.w <= J && m.vb >= int(sizeof(S)) && K * int64_t(sizeof(S)) % m.vb == 0 &&
+           aligned_to(m.vb);
+  };
   int shape = g_hdiff_shape.load();
-  if (shape <= 0 || shape >= kMarchShapeCount || kMarchShapes[shape].vb < int(sizeof(S)))
-    shape = default_march_shape<S>();
-  if (kMarchShapes[shape].w > J) shape = 1;  // a group needs J >= W columns
-  const int W = kMarchShapes[shape].w, strip = kMarchShapes[shape].strip;
-  const int V = kMarchShapes[shape].vb / static_cast<int>(sizeof(S));
-  const bool aligned = aligned16(in) && aligned16(out) && aligned16(coeff);
-  const bool vec = K % V == 0 && aligned;
-  const int64_t lanes = cdiv(J, W) * (K / V);
+  if (shape <= 0 || shape >= kMarchShapeCount || !fits(shape)) {
+    int n = 0;
+    do shape = march_order<S>(n++);
+    while (shape && !fits(shape));
+  }
+  // BF16 columns that no 4-byte vector divides: the last vector of a column is
+  // shifted back to end with it, and addresses are aligned to elements only.
+  const bool tail = sizeof(S) == 2 && !shape && J >= 4 && K >= 2;
+  if (tail) shape = 9;
+  const bool vec = shape != 0;
+  const bool aligned = aligned_to(16);
+  const int W = vec ? kMarchShapes[shape].w : 1, strip = vec ? kMarchShapes[shape].strip : 1;
+  const int V = vec ? kMarchShapes[shape].vb / static_cast<int>(sizeof(S)) : 1;
+  const int64_t lanes = cdiv(J, W) * cdiv(K, V);
   const int xblocks = static_cast<int>(cdiv(lanes, 256));
   const int64_t mblocks = int64_t(xblocks) * cdiv(I, strip);
   NPBX_REQUIRE(!vec || (lanes < (int64_t(1) << 31) && mblocks < (int64_t(1) << 31)),
@@ -787,6 +827,13 @@ int run_hdiff(const S* in, S* out, const S* coeff, int I, int J, int K, int64_t 
                            next);
       };
       constexpr int b4 = sizeof(S) <= 4 ? 4 : 8;  // FP64 has no 4-byte vector
+      if constexpr (sizeof(S) == 2) {
+        if (tail) {
+          go(hdiff_march<S, 4, 6, 4, true>);
+          NPBX_LAUNCHED("hdiff_march");
+          return NPBX_OK;
+        }
+      }
       switch (shape) {
         case 1: go(hdiff_march<S, 1, 12, 16>); break;
         case 2: go(hdiff_march<S, 1, 6, 16>); break;
@@ -800,7 +847,8 @@ int run_hdiff(const S* in, S* out, const S* coeff, int I, int J, int K, int64_t 
         case 10: go(hdiff_march<S, 4, 12, b4>); break;
         case 11: go(hdiff_march<S, 2, 12, 8>); break;
         case 12: go(hdiff_march<S, 2, 12, b4>); break;
-        default: go(hdiff_march<S, 3, 6, 8>); break;
+        case 13: go(hdiff_march<S, 3, 6, 8>); break;
+        default: go(hdiff_march<S, 4, 4, 8>); break;
       }
       NPBX_LAUNCHED("hdiff_march");
     } else {

@@ -89,6 +89,13 @@ __device__ __forceinline__ void loadraw(const S* __restrict__ p, RawVec<S, V>& r
   }
 }
 
+// The same from an address aligned only to its elements (the hardware takes
+// global accesses of any alignment; what crosses a line costs a second one).
+template <class S, int V>
+__device__ __forceinline__ void loadraw_any(const S* __restrict__ p, RawVec<S, V>& r) {
+  __builtin_memcpy(r.w, p, sizeof(r.w));
+}
+
 template <class S, int V>
 __device__ __forceinline__ void unpackv(const RawVec<S, V>& r, typename Storage<S>::C (&out)[V]) {
   S tmp[V];
@@ -113,6 +120,29 @@ __device__ __forceinline__ void storev(S* __restrict__ p,
     pack_words<S, V>(in, w);
     *reinterpret_cast<uint32_t*>(p) = w[0];
   }
+}
+
+// storev to an address aligned only to its elements.
+template <class S, int V>
+__device__ __forceinline__ void storev_any(S* __restrict__ p,
+                                           const typename Storage<S>::C (&in)[V]) {
+  uint32_t w[V * sizeof(S) / 4];
+  pack_words<S, V>(in, w);
+  __builtin_memcpy(p, w, sizeof(w));
+}
+
+// storev without keeping the line in the caches for a later read (a streaming
+// output), from an address aligned to the vector or, ANY, to its elements.
+template <class S, int V, bool ANY>
+__device__ __forceinline__ void storev_stream(S* __restrict__ p,
+                                              const typename Storage<S>::C (&in)[V]) {
+  constexpr int kWords = V * static_cast<int>(sizeof(S)) / 4;
+  constexpr int kAlign = ANY ? static_cast<int>(sizeof(S)) : 4 * kWords;
+  typedef uint32_t vec_t __attribute__((ext_vector_type(kWords)));
+  typedef vec_t at_t __attribute__((aligned(kAlign)));
+  uint32_t w[kWords];
+  pack_words<S, V>(in, w);
+  __builtin_nontemporal_store(__builtin_bit_cast(vec_t, w), reinterpret_cast<at_t*>(p));
 }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }

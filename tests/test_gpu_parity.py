@@ -229,6 +229,29 @@ def test_hdiff_two_step_strips(st, hdiff_tblock, precision, rows, I, J, K):
         _native.set_tuning("hdiff.fuse_rows", old)
 
 
+@pytest.mark.parametrize("precision", ["fp64", "fp32", "bf16"])
+@pytest.mark.parametrize("I,J,K", [(3, 1, 5), (4, 2, 3), (6, 3, 7), (5, 4, 2), (7, 5, 1),
+                                   (9, 6, 41), (13, 33, 22), (6, 70, 137)])
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("nsteps", [1, 2])
+def test_hdiff_any_level_count_and_alignment(st, precision, I, J, K, offset, nsteps):
+    """Columns that vectors do not divide and arrays aligned to one element:
+    every k is independent, so the result is bitwise that of the same columns
+    padded to whole 16-byte vectors (narrow fields, J < 4, included)."""
+    dt = {"fp64": torch.float64, "fp32": torch.float32, "bf16": torch.bfloat16}[precision]
+    inf, out, coeff = _hdiff_inputs(I, J, K, 7 * I + J + K)
+    pad = lambda a: np.concatenate([a, np.zeros(a.shape[:2] + (-K % 16,))], axis=2)  # noqa: E731
+    want = dev(pad(out), dt)
+    st.hdiff(dev(pad(inf), dt), want, dev(pad(coeff), dt), nsteps=nsteps)
+    put = _unaligned if offset else dev
+    got = put(out, dt)
+    print(f"hdiff {precision} {I}x{J}x{K} offset={offset} nsteps={nsteps}", flush=True)
+    st.hdiff(put(inf, dt), got, put(coeff, dt), nsteps=nsteps)
+    torch.cuda.synchronize()
+    assert torch.equal(got.contiguous().view(torch.uint8),
+                       want[:, :, :K].contiguous().view(torch.uint8))
+
+
 @pytest.fixture
 def hdiff_shape():
     """Sets the library's hdiff.shape knob for one test and restores it."""
