@@ -218,8 +218,8 @@ int npbx_pack_cols(int dtype, const void *A, const void *B, int64_t n,
  * select the wave-private heat tile: rows per wave including its own 2T halo
  * rows),
  * "heat.seg" = default planes per heat tile, "sweep.shape" = the plain
- * sweep's planes per workgroup / planes loaded ahead (0: 16/4, 1: 16/8,
- * 2: 32/8, 3: 8/4), "hdiff.tblock" = iterated hdiff steps fused per HBM round
+ * heat sweep's planes per workgroup / planes loaded ahead (0: by size and
+ * type, 1: 16/8, 2: 32/8, 3: 8/4), "hdiff.tblock" = iterated hdiff steps fused per HBM round
  * trip (1, the default, 2: the two-step register march with strips of
  * "hdiff.fuse_rows" output rows (0, the default: 16 for BF16, 32
  * otherwise), or 4: LDS blocks; BF16 at most 2), "adi.path" = ADI launches

@@ -138,9 +138,9 @@ int jacobi_deep_max();
 int jacobi_deep_sweeps(int dtype, void* A, void* B, int n, int64_t first, int64_t nsweeps, int T,
                        hipStream_t stream);
 
-// Plain-sweep shape chosen by the tuning knob "sweep.shape" (0 = 16 planes
-// per workgroup with loads of 4 planes in flight, 1 = 16/8, 2 = 32/8,
-// 3 = 8/4).
+// Plain heat-sweep shape chosen by the tuning knob "sweep.shape" (0 = by size
+// and type, heat3d.hip; 1, 2, 3 = 16-byte vectors, 16, 32, 8 planes per
+// workgroup with loads of 8, 8, 4 planes in flight).
 int sweep_shape();
 // Fused hdiff steps per round ("hdiff.tblock"; 1 = one launch per step).
 int hdiff_tblock();

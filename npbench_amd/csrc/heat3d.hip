@@ -3,21 +3,20 @@
 // Layout: N x N x N, C order (i slowest, k contiguous).  A sweep writes the
 // interior [1, N-2]^3 of dst from src; boundary faces are never written.
 //
-// Plain sweep (2.5-D), vector form: each lane owns V consecutive k (one
-// 16-byte load: 4 FP32, 2 FP64, 8 BF16), a wave spans 64*V k, a 256-thread
-// workgroup is one wave-row x 4 j-rows, and each thread marches along i over
-// kPlanes planes carrying the i-1 / i / i+1 vectors in registers.  Loads for
-// kUnroll planes (i+1, j+-1 vectors and the two k-edge scalars) are issued
-// before any of them is used, so every lane keeps several 16-byte HBM
-// requests in flight.  The j+-1 rows and k edges are L1/L2 hits.  Tiles are
-// numbered XCD by XCD (xcd_tile) so neighbours share an L2.  Each src element
-// crosses HBM about once per sweep.
-//
-// Scalar form (rows not 16-byte aligned): one k per lane, same marching.
+// Plain sweep (2.5-D): each lane owns V consecutive k, a wave spans 64*V k, a
+// 256-thread workgroup is one wave-row x 4 j-rows, and each thread marches
+// along i over kPlanes planes carrying the i-1 / i / i+1 vectors in registers.
+// Loads for kUnroll planes (i+1, j+-1 vectors and the two k-edge scalars) are
+// issued before any of them is used.  The j+-1 rows and k edges are L1/L2
+// hits.  Tiles are numbered XCD by XCD (xcd_tile) so neighbours share an L2.
+// Each src element crosses HBM about once per sweep.  Accesses ask only for
+// the elements' own alignment, so any side and any base take this form.
 //
 // Arithmetic (points.h): the FP64 drop-in follows the reference order, per
 // axis 0.125*((x[+1] - 2*c) + x[-1]), the axis terms summed i, j, k left to
 // right, then + c; FP32 arithmetic uses the 7-operation form of the same map.
+#include <type_traits>
+
 #include "common.h"
 #include "points.h"
 #include "vecio.h"
@@ -29,6 +28,8 @@ constexpr int kLanes = 64;
 constexpr int kCols = 4;
 constexpr int kRows = 16;
 
+// One point a lane, 16 planes, the grid's own block order: the best BF16 form
+// for sides of 129 to 192 (run_sweeps).
 template <class S>
 __global__ __launch_bounds__(kLanes* kCols) void heat3d_sweep(const S* __restrict__ src,
                                                              S* __restrict__ dst, int n) {
@@ -56,41 +57,48 @@ __global__ __launch_bounds__(kLanes* kCols) void heat3d_sweep(const S* __restric
 }
 
 // kPlanes = planes per workgroup (i segment); kUnroll = planes whose loads
-// are issued together.  Both are picked per call from the tuning knob
-// "sweep.shape" (sweep_shape below).
-template <class S, int kPlanes, int kUnroll>
+// are issued together (run_sweeps below).  A row's last vector is shifted
+// back to end with it where vectors do not divide the row; it shares points,
+// with the same values, with the one before.
+template <class S, int V, int kPlanes, int kUnroll>
 __global__ __launch_bounds__(kLanes* kCols) void heat3d_sweep_vec(const S* __restrict__ src,
                                                                  S* __restrict__ dst, int n,
                                                                  int tiles_k, int tiles_j) {
   using T = Storage<S>;
   using C = typename T::C;
-  constexpr int V = Vec16<S>::N;
   const int t = xcd_tile(blockIdx.x, gridDim.x);
   const int tk = t % tiles_k;
   const int tj = (t / tiles_k) % tiles_j;
   const int ti = t / (tiles_k * tiles_j);
-  const int k0 = (tk * kLanes + threadIdx.x) * V;
+  const int kv = (tk * kLanes + threadIdx.x) * V;
   const int j = 1 + tj * kCols + threadIdx.y;
   const int i0 = 1 + ti * kPlanes;
-  if (k0 >= n || j > n - 2) return;
+  if (kv >= n || j > n - 2) return;
+  const int k0 = min(kv, n - V);
   const int i_end = min(i0 + kPlanes, n - 1);
   const int64_t plane = static_cast<int64_t>(n) * n;
   const int64_t col = static_cast<int64_t>(j) * n + k0;
   const bool has_km = k0 > 0, has_kp = k0 + V < n;
   const bool full = k0 >= 1 && k0 + V <= n - 1;  // all V points interior in k
+  auto load = [&](const S* p, C(&x)[V]) {
+    S raw[V];
+    __builtin_memcpy(raw, p, sizeof(raw));
+#pragma unroll
+    for (int v = 0; v < V; ++v) x[v] = T::load(raw[v]);
+  };
 
   C below[V], centre[V];
-  load16(src + col + (i0 - 1) * plane, below);
-  load16(src + col + i0 * plane, centre);
+  load(src + col + (i0 - 1) * plane, below);
+  load(src + col + i0 * plane, centre);
   for (int i = i0; i < i_end; i += kUnroll) {
     C above[kUnroll][V], jp[kUnroll][V], jm[kUnroll][V], km[kUnroll], kp[kUnroll];
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
       // clamp so the loads of planes past the segment end stay in bounds
       const int64_t q = col + min(i + u, n - 2) * plane;
-      load16(src + q + plane, above[u]);
-      load16(src + q + n, jp[u]);
-      load16(src + q - n, jm[u]);
+      load(src + q + plane, above[u]);
+      load(src + q + n, jp[u]);
+      load(src + q - n, jm[u]);
       km[u] = has_km ? T::load(src[q - 1]) : C(0);
       kp[u] = has_kp ? T::load(src[q + V]) : C(0);
     }
@@ -106,7 +114,10 @@ __global__ __launch_bounds__(kLanes* kCols) void heat3d_sweep_vec(const S* __res
       }
       S* o = dst + col + static_cast<int64_t>(i + u) * plane;
       if (full) {
-        store16(o, out);
+        S raw[V];
+#pragma unroll
+        for (int v = 0; v < V; ++v) raw[v] = T::store(out[v]);
+        __builtin_memcpy(o, raw, sizeof(raw));
       } else {
 #pragma unroll
         for (int v = 0; v < V; ++v)
@@ -121,9 +132,8 @@ __global__ __launch_bounds__(kLanes* kCols) void heat3d_sweep_vec(const S* __res
   }
 }
 
-template <class S, int kPlanes, int kUnroll>
+template <class S, int V, int kPlanes, int kUnroll>
 int run_vec(S* A, S* B, int n, int64_t first, int64_t nsweeps, hipStream_t stream) {
-  constexpr int V = Vec16<S>::N;
   const dim3 block(kLanes, kCols);
   const int tiles_k = static_cast<int>(cdiv(n, kLanes * V));
   const int tiles_j = static_cast<int>(cdiv(n - 2, kCols));
@@ -132,7 +142,7 @@ int run_vec(S* A, S* B, int n, int64_t first, int64_t nsweeps, hipStream_t strea
   NPBX_REQUIRE(nblocks < (int64_t(1) << 31), "heat3d: grid too large");
   for (int64_t s = first; s < first + nsweeps; ++s) {
     const bool even = (s % 2) == 0;
-    hipLaunchKernelGGL((heat3d_sweep_vec<S, kPlanes, kUnroll>),
+    hipLaunchKernelGGL((heat3d_sweep_vec<S, V, kPlanes, kUnroll>),
                        dim3(static_cast<unsigned>(nblocks)), block, 0, stream, even ? A : B,
                        even ? B : A, n, tiles_k, tiles_j);
     NPBX_LAUNCHED("heat3d_sweep_vec");
@@ -141,16 +151,7 @@ int run_vec(S* A, S* B, int n, int64_t first, int64_t nsweeps, hipStream_t strea
 }
 
 template <class S>
-int run_sweeps(S* A, S* B, int n, int64_t first, int64_t nsweeps, hipStream_t stream) {
-  constexpr int V = Vec16<S>::N;
-  if (n % V == 0 && aligned16(A) && aligned16(B)) {
-    switch (sweep_shape()) {
-      case 1: return run_vec<S, 16, 8>(A, B, n, first, nsweeps, stream);
-      case 2: return run_vec<S, 32, 8>(A, B, n, first, nsweeps, stream);
-      case 3: return run_vec<S, 8, 4>(A, B, n, first, nsweeps, stream);
-      default: return run_vec<S, 16, 4>(A, B, n, first, nsweeps, stream);
-    }
-  }
+int run_points(S* A, S* B, int n, int64_t first, int64_t nsweeps, hipStream_t stream) {
   const dim3 block(kLanes, kCols);
   const dim3 grid(static_cast<unsigned>(cdiv(n - 2, kLanes)),
                   static_cast<unsigned>(cdiv(n - 2, kCols)),
@@ -161,6 +162,52 @@ int run_sweeps(S* A, S* B, int n, int64_t first, int64_t nsweeps, hipStream_t st
     NPBX_LAUNCHED("heat3d_sweep");
   }
   return NPBX_OK;
+}
+
+// The sweeps in the launch shape of the setting "sweep.shape" where that is
+// not 0, else by size.  A march over planes is a chain of load latencies, so
+// it is as short as leaves the chip some waves to switch between; from about
+// 128^3 on it saves loads of planes i-1 and i.  Narrow vectors fill a wave's
+// lanes on short rows, and FP32 keeps them: with one point a lane a row's
+// accesses are whole lines and the k-edge scalars hit the same ones.
+// Measured, us per sweep, V points a lane x planes / ahead:
+//   FP64       2x1/1  2x2/2  2x4/4  2x8/4  2x16/4     BF16  2x1/1  2x2/2  4x2/2  8x4/2  1x16
+//     64^3       3.7    3.7    3.7    4.9    7.6       64^3   3.5    3.5    4.0    7.0    5.2
+//     101^3      6.3    6.1    6.3    7.1    8.4      101^3   5.0    4.8    5.5    7.5    7.1
+//     160^3     18.3   17.4   16.8   17.5   19.6      177^3  16.3   13.7   12.1   13.9   10.6
+//     201^3     29.1   27.6   25.8   25.7   29.8      201^3  20.3   17.9   15.3   17.5   16.2
+//     512^3      723    678    626    615    622      512^3   329    268    200    176    234
+//   FP32       2x1/1  1x4/4  1x8/4  4x4/4  4x16/4
+//     64^3       3.5    3.2    3.8    3.9    8.5
+//     101^3      5.2    4.7    5.1    5.5    8.5
+//     201^3     20.9   18.4   14.8   15.6   18.2
+//     256^3     32.0   27.5   22.2   24.7   25.7
+//     512^3      384    289    284    317    314
+template <class S>
+int run_sweeps(S* A, S* B, int n, int64_t first, int64_t nsweeps, hipStream_t stream) {
+  constexpr int N = Vec16<S>::N;
+  if (n >= N) {
+    switch (sweep_shape()) {
+      case 1: return run_vec<S, N, 16, 8>(A, B, n, first, nsweeps, stream);
+      case 2: return run_vec<S, N, 32, 8>(A, B, n, first, nsweeps, stream);
+      case 3: return run_vec<S, N, 8, 4>(A, B, n, first, nsweeps, stream);
+      default: break;
+    }
+  }
+  if (n <= 88) return run_vec<S, 2, 1, 1>(A, B, n, first, nsweeps, stream);
+  if constexpr (std::is_same_v<S, double>) {
+    if (n <= 112) return run_vec<S, 2, 2, 2>(A, B, n, first, nsweeps, stream);
+    if (n <= 176) return run_vec<S, 2, 4, 4>(A, B, n, first, nsweeps, stream);
+    return run_vec<S, 2, 8, 4>(A, B, n, first, nsweeps, stream);
+  } else if constexpr (std::is_same_v<S, float>) {
+    if (n <= 112) return run_vec<S, 1, 4, 4>(A, B, n, first, nsweeps, stream);
+    return run_vec<S, 1, 8, 4>(A, B, n, first, nsweeps, stream);
+  } else {
+    if (n <= 128) return run_vec<S, 2, 2, 2>(A, B, n, first, nsweeps, stream);
+    if (n <= 192) return run_points<S>(A, B, n, first, nsweeps, stream);
+    if (n <= 280) return run_vec<S, 4, 2, 2>(A, B, n, first, nsweeps, stream);
+    return run_vec<S, 8, 4, 2>(A, B, n, first, nsweeps, stream);
+  }
 }
 
 int heat_entry(int dtype, void* A, void* B, int64_t N, int64_t first, int64_t nsweeps, int tblock,

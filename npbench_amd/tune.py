@@ -38,7 +38,7 @@ SHAPES = {
     torch.bfloat16: [(2, 2), (2, 4)],
 }
 SEGS = (32, 64, 128)
-SWEEP_SHAPES = (0, 1, 2, 3)  # libnpbx "sweep.shape": 16/4, 16/8, 32/8, 8/4
+SWEEP_SHAPES = (0, 1, 2, 3)  # libnpbx "sweep.shape": by size, 16/8, 32/8, 8/4
 VEC = {torch.float64: 2, torch.float32: 4, torch.bfloat16: 8}
 
 _memo = {}

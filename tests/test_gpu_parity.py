@@ -131,6 +131,52 @@ def test_heat3d_reduced_precision(st, precision, tol):
     assert err <= tol
 
 
+def _heat_exactly(x, y):
+    """One sweep of the library's arithmetic: FP64 the reference's; FP32 (and
+    BF16 storage) 0.125 * (six neighbours, plane i-1 first, i+1 last) +
+    0.25 * c in one rounding, which FP64 holds exactly for values of [0.25, 1)."""
+    if x.dtype == torch.float64:
+        a, b = x.numpy(), y.numpy()
+        m = slice(1, -1)
+        c = a[m, m, m]
+        b[m, m, m] = (0.125 * (a[2:, m, m] - 2.0 * c + a[:-2, m, m]) +
+                      0.125 * (a[m, 2:, m] - 2.0 * c + a[m, :-2, m]) +
+                      0.125 * (a[m, m, 2:] - 2.0 * c + a[m, m, :-2]) + c)
+        return
+    a = x.float()
+    m = slice(1, -1)
+    s = a[:-2, m, m] + a[m, :-2, m] + a[m, 2:, m] + a[m, m, :-2] + a[m, m, 2:] + a[2:, m, m]
+    y[m, m, m] = (0.125 * s.double() + 0.25 * a[m, m, m].double()).float().to(x.dtype)
+
+
+# the sides where the launch shape changes, the smallest ones, and remainders
+# of the vectors; bases that are aligned to their elements alone
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,off", [(3, 1), (4, 0), (7, 1), (9, 0), (64, 1), (88, 0), (89, 1),
+                                   (112, 1), (113, 0), (128, 1), (129, 0), (176, 1), (177, 0),
+                                   (192, 0), (193, 1), (257, 0), (280, 1), (281, 0)])
+def test_heat3d_sweep_shapes_bitwise(st, dtype, n, off):
+    print(f"heat3d shapes {dtype} n={n} off={off}", flush=True)
+    gen = torch.Generator().manual_seed(31 * n + off)
+    a, b = (torch.empty(n, n, n).uniform_(0.25, 1.0, generator=gen).to(dtype) for _ in range(2))
+
+    def on_device(x):
+        buf = torch.full((n ** 3 + 2 * off + 1,), 0.5, dtype=dtype, device="cuda")
+        view = buf[off:off + n ** 3].view(n, n, n)
+        view.copy_(x)
+        return buf, view
+
+    (fa, da), (fb, db) = on_device(a), on_device(b)
+    st.heat3d_sweeps(da, db, 2)
+    _heat_exactly(a, b)
+    _heat_exactly(b, a)
+    torch.cuda.synchronize()
+    for buf, view, want in ((fa, da, a), (fb, db, b)):
+        assert torch.equal(view.cpu(), want)
+        out = torch.cat([buf[:off], buf[off + n ** 3:]]).cpu()
+        assert torch.equal(out, torch.full_like(out, 0.5))  # nothing written around it
+
+
 # ---------------------------------------------------------------- hdiff
 def _hdiff_inputs(I, J, K, seed):
     rng = np.random.default_rng(seed)
