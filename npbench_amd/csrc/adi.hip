@@ -11,7 +11,8 @@
 // do not depend on the data and are the same for every line, so they are
 // computed once per call (adi_tables) with the reference's own operations.
 //
-// One thread owns one line (a column in the first half, a row in the
+// Sides up to 1842 run as split half sweeps (adi_split below).  In the other
+// forms one thread owns one line (a column in the first half, a row in the
 // second).  A line is a serial chain of divisions, so the time is the
 // chain's latency.  Three things keep the chain short:
 //  * the steps of a 16-step chunk have no branches between them, so the
@@ -503,6 +504,276 @@ __global__ __launch_bounds__(NT) void adi_rows(AdiArgs g) {
   row_sweep<NT, QLDS>(g, static_cast<int>(blockIdx.x) * NT, lds, qlds);
 }
 
+// ------------------------------------------------------- split half sweep
+// One half sweep of L lines per workgroup, its chain alone on one wave.
+//
+// Both halves are the same computation on a matrix `in` laid out [step][line]:
+// the column sweep reads u, the row sweep reads the column sweep's result,
+// which is therefore written transposed ([line][step]).  A workgroup keeps one
+// array s[step][line] in LDS: helper waves (1 .. 3) fill it with right-hand
+// sides, wave 0 runs the forward recurrence over it in place (q) and then the
+// back substitution (x), and the helpers check q and store x as the chunks are
+// finished.  Wave 0 so issues what the recurrence itself consists of -- five
+// dependent FP64 operations a step forward, two back, at 7.4 cycles each --
+// and its LDS accesses; with right-hand sides, checks and staging on the same
+// wave (adi_columns, adi_rows) it was bound by issuing those.  Chunks are
+// handed over by flags in LDS, so no wave waits for another but for data.
+//
+// The check of the short division (division.h) looks at q where that kernel
+// looks at the estimate m: the two agree to a few units of the last place, so
+// 2 lo <= |q| < hi / 2 implies lo <= |m| < hi (an m out of range leaves a q
+// that is subnormal-sized, infinite or NaN).  From a line's first NaN
+// right-hand side on, q is NaN in either form and is not looked at, so a grid
+// that has overflowed costs no more.  If a value fails, the workgroup
+// forms its right-hand sides again and runs the forward pass with the
+// division operator.
+//
+// Time per half sweep against one-wave workgroups that do it all (path 3):
+// N = 50 7.4 -> 5.4 us, 100 14.6 -> 8.8, 200 23.8 -> 13.6, 300 40.9 -> 18.5,
+// 1000 133 -> 61, 1800 226 -> 103: 58 ns a step, 7 dependent FP64 operations
+// at about 8.3 ns, and 2 us for the launch and the first loads.
+constexpr int kSplitLines = 8;  // L; 16 is 2 % slower, 32 8 %, 64 20 % (N = 200)
+constexpr int kHelpers = 3;     // 7 are level
+constexpr int kAhead = 2;       // chunks a helper loads ahead; 4 are level
+
+struct AdiHalf {
+  const double* in;  // [step][line], pitch ldi
+  double* out;       // [line][step], pitch ldo
+  int ldi, ldo;
+  SweepTab tab;
+  double wm, wc, wp;  // right-hand side (wm in[.][i-1] + wc in[.][i]) - wp in[.][i+1]
+  double wq;          // weight of q[j-1]
+  int n;
+};
+
+// LDS of a workgroup: s (chunks * kCW rows of L + 1: odd, so that both a row's
+// lines and a line's steps spread over the banks), the steps' (den, y) pairs,
+// three flags a chunk, the verdict, and each line's first NaN right-hand side.
+struct SplitLds {
+  static constexpr int L = kSplitLines;
+  static constexpr int P = L + 1;
+  static constexpr int chunks(int n) { return (n - 2 + kCW - 1) / kCW; }
+  static constexpr size_t bytes(int n) {
+    return static_cast<size_t>(chunks(n)) * (kCW * (P + 2) * sizeof(double) + 3 * sizeof(int)) +
+           (1 + L) * sizeof(int);
+  }
+};
+
+// Flags between the waves of a workgroup: LDS accesses of a wave are done in
+// order, so a flag stored after the data is seen after it; the fences order
+// them for the compiler.
+__device__ __forceinline__ void raise_flag(int* flag) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void wait_flag(int* flag) {
+  while (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == 0)
+    __builtin_amdgcn_s_sleep(1);
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+__global__ __launch_bounds__(64 * (kHelpers + 1)) void adi_split(AdiHalf g) {
+  using Lds = SplitLds;
+  constexpr int L = Lds::L, P = Lds::P;
+  constexpr int kPer = kCW * L / 64;  // elements of a chunk per lane of a wave
+  extern __shared__ __align__(16) double shared_mem[];
+  const int n = g.n, nc = Lds::chunks(n), steps = n - 2;
+  double2* dy = reinterpret_cast<double2*>(shared_mem);
+  double* s = shared_mem + 2 * kCW * nc;
+  int* rhs_done = reinterpret_cast<int*>(s + kCW * nc * P);
+  int* q_done = rhs_done + nc;
+  int* x_done = q_done + nc;
+  int* bad = x_done + nc;
+  int* nan_from = bad + 1;
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lb = static_cast<int>(blockIdx.x) * L;  // lines lb+1 .. lb+L
+  for (int e = threadIdx.x; e <= 3 * nc; e += 64 * (kHelpers + 1)) rhs_done[e] = 0;
+  if (threadIdx.x < L) nan_from[threadIdx.x] = steps;
+  __syncthreads();
+
+  // Chunk c's right-hand sides, by one wave: lane l % L's line, steps past
+  // the last and lines past the last clamped into the grid.
+  const int li = lane % L, lr = lane / L;
+  const int gi = min(lb + 1 + li, n - 2);
+  struct Raw {
+    double m[kPer], c[kPer], p[kPer], tab;
+  };
+  auto fetch = [&](int c, Raw& r) {
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int j = min(1 + c * kCW + k * (64 / L) + lr, n - 2);
+      const double* a = g.in + static_cast<int64_t>(j) * g.ldi + gi;
+      r.m[k] = a[-1];
+      r.c[k] = a[0];
+      r.p[k] = a[1];
+    }
+    r.tab = (lane & kCW ? g.tab.y : g.tab.den)[1 + c * kCW + (lane & (kCW - 1))];
+  };
+  auto form = [&](int c, const Raw& r) {
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int j = c * kCW + k * (64 / L) + lr;
+      const double v = (g.wm * r.m[k] + g.wc * r.c[k]) - g.wp * r.p[k];
+      s[j * P + li] = v;
+      if (v != v) atomicMin(nan_from + li, j);
+    }
+    if (lane < 2 * kCW)
+      reinterpret_cast<double*>(dy)[2 * (c * kCW + (lane & (kCW - 1))) + (lane >> 4)] = r.tab;
+  };
+
+  const bool fast = g.tab.ok[0] != 0.0;
+  if (w == 0) {
+    if (fast) {
+      __builtin_amdgcn_s_setprio(3);
+      double q = 1.0;
+      double rv[2][kCW];
+      double2 t[2][kCW];
+      auto read = [&](int c, double(&r)[kCW], double2(&d)[kCW]) {
+#pragma unroll
+        for (int k = 0; k < kCW; ++k) {
+          r[k] = s[(c * kCW + k) * P + li];
+          d[k] = dy[c * kCW + k];
+        }
+      };
+      auto run = [&](int c, const double(&r)[kCW], const double2(&d)[kCW]) {
+#pragma unroll
+        for (int k = 0; k < kCW; ++k) {
+          double m;
+          q = short_division(r[k] - g.wq * q, d[k].x, d[k].y, m);
+          s[(c * kCW + k) * P + li] = q;
+        }
+        raise_flag(q_done + c);
+      };
+      if (lane < L) {
+        wait_flag(rhs_done);
+        read(0, rv[0], t[0]);
+        for (int c = 0; c < nc; c += 2) {
+          if (c + 1 < nc) {
+            wait_flag(rhs_done + c + 1);
+            read(c + 1, rv[1], t[1]);
+          }
+          run(c, rv[0], t[0]);
+          if (c + 1 >= nc) break;
+          if (c + 2 < nc) {
+            wait_flag(rhs_done + c + 2);
+            read(c + 2, rv[0], t[0]);
+          }
+          run(c + 1, rv[1], t[1]);
+        }
+      }
+    }
+  } else {
+    if (w == 1) {  // x[0] = x[n-1] = 1
+      for (int l = lane; l < 2 * L; l += 64) {
+        const int i = lb + 1 + l / 2;
+        if (i <= n - 2) g.out[static_cast<int64_t>(i) * g.ldo + (l & 1 ? n - 1 : 0)] = 1.0;
+      }
+    }
+    // kAhead chunks loaded ahead, so that the loads' latency is paid once
+    Raw raw[kAhead];
+    auto each = [&](auto&& f) {
+#pragma unroll
+      for (int d = 0; d < kAhead; ++d) f(d);
+    };
+    each([&](int d) {
+      if (w - 1 + d * kHelpers < nc) fetch(w - 1 + d * kHelpers, raw[d]);
+    });
+    for (int c0 = w - 1; c0 < nc; c0 += kAhead * kHelpers)
+      each([&](int d) {
+        const int c = c0 + d * kHelpers, next = c + kAhead * kHelpers;
+        if (c >= nc) return;
+        form(c, raw[d]);
+        raise_flag(rhs_done + c);
+        if (next < nc) fetch(next, raw[d]);
+      });
+    if (fast) {
+      const double lo = 2.0 * g.tab.ok[1], hi = 0.5 * g.tab.ok[2];
+      bool ok = true;
+      for (int c = w - 1; c < nc; c += kHelpers) {
+        wait_flag(q_done + c);
+        const int checked = nan_from[li];  // at most `steps`; final for this chunk's steps
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+          const int j = c * kCW + k * (64 / L) + lr;
+          const double q = fabs(s[j * P + li]);
+          ok = ok && (j >= checked || (q >= lo && q < hi));
+        }
+      }
+      if (!ok) *bad = 1;
+    }
+  }
+  __syncthreads();
+  if (!fast || *bad) {
+    for (int c = w; c < nc; c += kHelpers + 1) {
+      Raw a;
+      fetch(c, a);
+      form(c, a);
+    }
+    __syncthreads();
+    if (w == 0 && lane < L) {
+      double q = 1.0;
+      for (int j = 0; j < steps; ++j) {
+        q = (s[j * P + li] - g.wq * q) / dy[j].x;
+        s[j * P + li] = q;
+      }
+    }
+    __syncthreads();
+  }
+
+  // back substitution, and the helpers' stores of finished chunks
+  if (w == 0) {
+    if (lane < L) {
+      const ConstTab ptab = as_const(g.tab.p);
+      double x = 1.0;
+      double qv[2][kCW], pv[2][kCW];
+      auto read = [&](int c, double(&q)[kCW], double(&p)[kCW]) {
+#pragma unroll
+        for (int k = 0; k < kCW; ++k) q[k] = s[(c * kCW + k) * P + li];
+        table_chunk(ptab, 1 + c * kCW, p);
+      };
+      auto run = [&](int c, const double(&q)[kCW], const double(&p)[kCW]) {
+#pragma unroll
+        for (int k = kCW - 1; k >= 0; --k) {
+          x = p[k] * x + q[k];
+          s[(c * kCW + k) * P + li] = x;
+        }
+        raise_flag(x_done + c);
+      };
+      int c = nc - 1;
+      read(c, qv[0], pv[0]);
+      if (c > 0) read(c - 1, qv[1], pv[1]);
+#pragma unroll
+      for (int k = kCW - 1; k >= 0; --k) {  // the chunk that may run past the last step
+        const double nx = pv[0][k] * x + qv[0][k];
+        x = c * kCW + k < steps ? nx : x;
+        s[(c * kCW + k) * P + li] = x;
+      }
+      raise_flag(x_done + c);
+      for (c -= 1; c >= 0; c -= 2) {
+        if (c > 0) read(c - 1, qv[0], pv[0]);
+        run(c, qv[1], pv[1]);
+        if (c == 0) break;
+        if (c > 1) read(c - 2, qv[1], pv[1]);
+        run(c - 1, qv[0], pv[0]);
+      }
+    }
+  } else {
+    const int jj = lane & (kCW - 1);
+    for (int c = nc - w; c >= 0; c -= kHelpers) {
+      wait_flag(x_done + c);
+      const int j = c * kCW + jj;
+#pragma unroll
+      for (int k = 0; k < L / 4; ++k) {
+        const int l = k * 4 + (lane >> 4);
+        const int i = lb + 1 + l;
+        if (j < steps && i <= n - 2)
+          g.out[static_cast<int64_t>(i) * g.ldo + 1 + j] = s[j * P + l];
+      }
+    }
+  }
+}
+
 // Self-check of the short division: random (n, den) pairs, half of them with
 // n / den next to a rounding midpoint (the cases a wrong rounding would
 // show), compared bit for bit with the division operator wherever the
@@ -555,11 +826,10 @@ __global__ __launch_bounds__(256) void adi_division_check(uint64_t seed, int64_t
   atomicAdd(&counts[1], wrong);
 }
 
-// 0: the default (3), 1: every time step in one single-workgroup launch, 2:
+// 0: the default (split half sweeps, else 3), 1: every time step in one single-workgroup launch, 2:
 // a launch per half step over 256-line workgroups, 3: the same over one-wave
-// workgroups.  Measured on the MI355X, one wave per CU is the fastest: a
-// line's chain leaves the SIMD idle most of the time, and waves sharing a CU
-// queue behind each other's memory instructions.
+// workgroups, the fastest of 1 to 3: waves sharing a CU queue behind each
+// other's memory instructions.
 std::atomic<int> g_adi_path{0};
 
 template <int NT, bool QLDS>
@@ -573,10 +843,29 @@ int launch_halves(const AdiArgs& g, int nb, int64_t tsteps, hipStream_t stream) 
   return NPBX_OK;
 }
 
+// The split half sweeps take sides whose kSplitLines lines fit a CU's LDS (up
+// to 1842); they are the faster form for all of them.
+constexpr size_t kLdsBytes = 160 * 1024;
+int launch_split(const AdiArgs& g, double* v, int ldv, int64_t tsteps, hipStream_t stream) {
+  const int n = g.n;
+  const size_t lds = SplitLds::bytes(n);
+  const dim3 grid(static_cast<unsigned>(cdiv(n - 2, SplitLds::L)));
+  const AdiHalf cols{g.u, v, n, ldv, g.cols, g.nd, g.c1, g.f, g.a, n};
+  const AdiHalf rows{v, g.u, ldv, n, g.rows, g.na, g.c2, g.c, g.d, n};
+  for (int64_t s = 0; s < tsteps; ++s) {
+    hipLaunchKernelGGL((adi_split), grid, dim3(64 * (kHelpers + 1)), lds, stream, cols);
+    NPBX_LAUNCHED("adi_split (columns)");
+    hipLaunchKernelGGL((adi_split), grid, dim3(64 * (kHelpers + 1)), lds, stream, rows);
+    NPBX_LAUNCHED("adi_split (rows)");
+  }
+  return NPBX_OK;
+}
+
 // Launch shape and scratch layout of one call: v (the column sweep's output,
 // (n + 16) rows of ldv), q ([step][line], qrows x ld) and the eight tables.
 struct AdiPlan {
   int path, nt, nb;
+  bool split;
   int64_t ld, ldv, qrows, tl, vel, qel, tel;
   size_t bytes() const { return static_cast<size_t>(vel + qel + tel) * sizeof(double); }
 };
@@ -585,6 +874,7 @@ int plan_adi(int64_t n64, AdiPlan& pl) {
   const int n = static_cast<int>(n64);
   const int lines = n - 2;
   pl.path = g_adi_path.load();
+  pl.split = pl.path == 0 && SplitLds::bytes(n) <= kLdsBytes;
   if (pl.path == 0) pl.path = 3;
   NPBX_REQUIRE(pl.path != 1 || lines <= 512,
                "adi: one-launch path holds at most 512 lines (N=%d)", n);
@@ -632,6 +922,7 @@ int run_adi(double* u, int64_t n64, int64_t tsteps, const AdiPlan& pl, void* ws,
   g.ld = static_cast<int>(ld);
   g.ldv = static_cast<int>(ldv);
   g.tsteps = static_cast<int>(tsteps);
+  if (pl.split) return launch_split(g, v, g.ldv, tsteps, stream);
   if (path == 1) {
     if (nt == 256)
       hipLaunchKernelGGL(adi_fused<256>, dim3(1), dim3(256), 0, stream, g);

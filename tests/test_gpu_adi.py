@@ -68,6 +68,18 @@ def test_adi_fp64_bitwise(st, adi_path, n, tsteps, path):
     assert_bitwise(run_gpu(st, u, tsteps), want, f"adi n={n} tsteps={tsteps} path={path}")
 
 
+# split half sweeps: one chunk and one step more or less, eight lines and one
+# more or less, and the last side whose lines fit LDS beside the first beyond
+@pytest.mark.parametrize("n", [10, 11, 49, 50, 51, 1842, 1843])
+def test_adi_split_edges_bitwise(st, adi_path, n):
+    u = np.random.default_rng(n).random((n, n))
+    tsteps = 3 if n < 100 else 1
+    want = ref.adi_kernel(tsteps, n, u.copy())
+    adi_path(0)
+    print(f"adi split n={n}", flush=True)
+    assert_bitwise(run_gpu(st, u, tsteps), want, f"adi split n={n}")
+
+
 @pytest.mark.parametrize("tsteps,n", [(5, 100), (100, 200)])
 def test_adi_reference_presets_bitwise(st, tsteps, n):
     """The reference's initialisation at its S and paper presets; values grow
@@ -126,6 +138,21 @@ def test_adi_wide_range_inputs_take_the_division_operator(st):
     u[9, 11] = 5e-324  # subnormal
     want = ref.adi_kernel(tsteps, n, u.copy())
     assert_bitwise(run_gpu(st, u, tsteps), want, "adi wide range")
+
+
+def test_adi_nan_and_overflow_match_the_oracle(st):
+    """NaN, infinities and values that overflow on the way: split half sweeps
+    leave the short division exactly where it would rescale."""
+    n, tsteps = 40, 2
+    for name, at, val in (("nan", (20, 30), np.nan), ("inf", (3, 4), np.inf),
+                          ("overflow", (slice(None), slice(1, -1)), 1e307)):
+        u = np.random.default_rng(12).random((n, n)) + 0.5
+        u[at] *= val
+        with np.errstate(all="ignore"):
+            want = ref.adi_kernel(tsteps, n, u.copy())
+        print(f"adi {name}", flush=True)
+        got = run_gpu(st, u, tsteps)
+        assert np.array_equal(got, want, equal_nan=True), name
 
 
 def test_adi_argument_checks(st, adi_path):
