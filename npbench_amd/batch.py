@@ -1,9 +1,10 @@
 """Batched grids: many independent Jacobi 2-D / heat 3-D grids of uneven size
-advanced together by persistent tile-queue launches (libnpbx plans).
+advanced together (libnpbx plans): 2-D grids in register blocks, heat grids on
+tiles of ``tblock`` sweeps or by single sweeps, whichever suits their sizes.
 
 A ``Plan`` fixes the grids (device tensors A, B of one storage dtype), each
-grid's sweep range and the temporal-blocking depth.  ``launch()`` enqueues
-every round; ``capture()`` records them into a HIP graph on a side stream so
+grid's sweep range, the temporal-blocking depth and the most planes of a heat
+tile (``seg``).  ``launch()`` enqueues every round; ``capture()`` records them into a HIP graph on a side stream so
 later launches replay the graph.  Results are bitwise those of running each
 grid alone with the per-grid entry points.
 """

@@ -514,7 +514,7 @@ __global__ __launch_bounds__(NT) void adi_rows(AdiArgs g) {
 // sides, wave 0 runs the forward recurrence over it in place (q) and then the
 // back substitution (x), and the helpers check q and store x as the chunks are
 // finished.  Wave 0 so issues what the recurrence itself consists of -- five
-// dependent FP64 operations a step forward, two back, at 7.4 cycles each --
+// dependent FP64 operations a step forward, two back, about 8.3 ns each --
 // and its LDS accesses; with right-hand sides, checks and staging on the same
 // wave (adi_columns, adi_rows) it was bound by issuing those.  Chunks are
 // handed over by flags in LDS, so no wave waits for another but for data.

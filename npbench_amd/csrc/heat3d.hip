@@ -15,10 +15,12 @@
 // Arithmetic (points.h): the FP64 drop-in follows the reference order, per
 // axis 0.125*((x[+1] - 2*c) + x[-1]), the axis terms summed i, j, k left to
 // right, then + c; FP32 arithmetic uses the 7-operation form of the same map.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
 #include "points.h"
+#include "tiles.h"
 #include "vecio.h"
 
 namespace npbx {
@@ -61,12 +63,10 @@ __global__ __launch_bounds__(kLanes* kCols) void heat3d_sweep(const S* __restric
 // back to end with it where vectors do not divide the row; it shares points,
 // with the same values, with the one before.
 template <class S, int V, int kPlanes, int kUnroll>
-__global__ __launch_bounds__(kLanes* kCols) void heat3d_sweep_vec(const S* __restrict__ src,
-                                                                 S* __restrict__ dst, int n,
-                                                                 int tiles_k, int tiles_j) {
+__device__ __forceinline__ void sweep_tile(const S* __restrict__ src, S* __restrict__ dst, int n,
+                                           int tiles_k, int tiles_j, int t) {
   using T = Storage<S>;
   using C = typename T::C;
-  const int t = xcd_tile(blockIdx.x, gridDim.x);
   const int tk = t % tiles_k;
   const int tj = (t / tiles_k) % tiles_j;
   const int ti = t / (tiles_k * tiles_j);
@@ -130,6 +130,147 @@ __global__ __launch_bounds__(kLanes* kCols) void heat3d_sweep_vec(const S* __res
       }
     }
   }
+}
+
+template <class S, int V, int kPlanes, int kUnroll>
+__global__ __launch_bounds__(kLanes* kCols) void heat3d_sweep_vec(const S* __restrict__ src,
+                                                                 S* __restrict__ dst, int n,
+                                                                 int tiles_k, int tiles_j) {
+  sweep_tile<S, V, kPlanes, kUnroll>(src, dst, n, tiles_k, tiles_j,
+                                     xcd_tile(blockIdx.x, gridDim.x));
+}
+
+// One sweep of up to kMaxBatch grids: tile t of the launch belongs to the grid
+// g with cum[g] <= t < cum[g+1].  `form` is the grid's kernel form (batch_form).
+struct HeatBatch {
+  int32_t count;
+  int32_t cum[kMaxBatch + 1];
+  struct {
+    const void* src;
+    void* dst;
+    int32_t n, tiles_k, tiles_j, form;
+  } grid[kMaxBatch];
+};
+
+// The forms of a batch's grids by type: points a lane, planes, planes ahead.
+struct Form {
+  int v, planes;
+};
+template <class S>
+struct BatchForms;
+template <>
+struct BatchForms<double> {
+  static constexpr Form form[3] = {{2, 2}, {2, 4}, {2, 8}};
+  static constexpr int ahead[3] = {2, 4, 4};
+};
+template <>
+struct BatchForms<float> {
+  static constexpr Form form[3] = {{1, 1}, {1, 4}, {1, 8}};
+  static constexpr int ahead[3] = {1, 4, 4};
+};
+template <>
+struct BatchForms<bf16> {
+  static constexpr Form form[3] = {{2, 2}, {4, 2}, {8, 4}};
+  static constexpr int ahead[3] = {2, 2, 2};
+};
+
+template <class S>
+__global__ __launch_bounds__(kLanes* kCols) void heat3d_sweep_batch(const HeatBatch b) {
+  using F = BatchForms<S>;
+  const int t = xcd_tile(blockIdx.x, gridDim.x);
+  int lo = 0, hi = b.count - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (b.cum[mid] <= t) lo = mid; else hi = mid - 1;
+  }
+  const auto& g = b.grid[lo];
+  const S* src = static_cast<const S*>(g.src);
+  S* dst = static_cast<S*>(g.dst);
+  const int tile = t - b.cum[lo];
+  if (g.form == 0)
+    sweep_tile<S, F::form[0].v, F::form[0].planes, F::ahead[0]>(src, dst, g.n, g.tiles_k,
+                                                                g.tiles_j, tile);
+  else if (g.form == 1)
+    sweep_tile<S, F::form[1].v, F::form[1].planes, F::ahead[1]>(src, dst, g.n, g.tiles_k,
+                                                                g.tiles_j, tile);
+  else
+    sweep_tile<S, F::form[2].v, F::form[2].planes, F::ahead[2]>(src, dst, g.n, g.tiles_k,
+                                                                g.tiles_j, tile);
+}
+
+// A batch's grids take the forms that a single grid of as many points takes
+// (run_sweeps); BF16's follow the row length, which its vectors have to fill.
+int batch_form(int dtype, int n, int64_t points) {
+  if (dtype == NPBX_BF16) return n <= 128 ? 0 : n <= 280 ? 1 : 2;
+  const int64_t lo = dtype == NPBX_F64 ? 112 : 56, hi = dtype == NPBX_F64 ? 176 : 112;
+  return points <= lo * lo * lo ? 0 : points <= hi * hi * hi ? 1 : 2;
+}
+
+// Grids are swept in groups that fit the Infinity Cache with both arrays, one
+// group after the other: a sweep of more runs at HBM's rate (FP32, 256^3 grids:
+// 8 in one launch 303 us a sweep, 1 at a time 25).
+constexpr int64_t kGroupBytes = int64_t(256) << 20;
+
+template <class S>
+int group_sweeps(int dtype, const SweepGrid* grids, size_t count, bool enqueue,
+                 hipStream_t stream, int64_t* launches, int64_t* tiles) {
+  int64_t sweeps = 0;
+  for (size_t i = 0; i < count; ++i) sweeps = std::max(sweeps, grids[i].nsweeps);
+  for (int64_t s = 0; s < sweeps; ++s) {
+    int64_t points = 0;
+    for (size_t i = 0; i < count; ++i)
+      if (s < grids[i].nsweeps) points += int64_t(grids[i].n) * grids[i].n * grids[i].n;
+    HeatBatch b;
+    b.count = 0;
+    b.cum[0] = 0;
+    for (size_t i = 0; i <= count; ++i) {
+      if (b.count == kMaxBatch || (i == count && b.count > 0)) {
+        const int blocks = b.cum[b.count];
+        *launches += 1;
+        *tiles += blocks;
+        if (enqueue) {
+          hipLaunchKernelGGL(heat3d_sweep_batch<S>, dim3(static_cast<unsigned>(blocks)),
+                             dim3(kLanes, kCols), 0, stream, b);
+          NPBX_LAUNCHED("heat3d_sweep_batch");
+        }
+        b.count = 0;
+      }
+      if (i == count || s >= grids[i].nsweeps) continue;
+      const SweepGrid& g = grids[i];
+      const int form = batch_form(dtype, g.n, points);
+      const Form f = BatchForms<S>::form[form];
+      const bool even = ((g.first + s) & 1) == 0;
+      auto& d = b.grid[b.count];
+      d.src = even ? g.A : g.B;
+      d.dst = even ? g.B : g.A;
+      d.n = g.n;
+      d.form = form;
+      d.tiles_k = static_cast<int32_t>(cdiv(g.n, kLanes * f.v));
+      d.tiles_j = static_cast<int32_t>(cdiv(g.n - 2, kCols));
+      const int64_t nt = int64_t(d.tiles_k) * d.tiles_j * cdiv(g.n - 2, f.planes);
+      NPBX_REQUIRE(b.cum[b.count] + nt < (int64_t(1) << 31), "heat batch: too many tiles");
+      b.cum[b.count + 1] = b.cum[b.count] + static_cast<int32_t>(nt);
+      ++b.count;
+    }
+  }
+  return NPBX_OK;
+}
+
+template <class S>
+int batch_sweeps(int dtype, const std::vector<SweepGrid>& grids, bool enqueue,
+                 hipStream_t stream, int64_t* launches, int64_t* tiles) {
+  auto bytes = [](const SweepGrid& g) {
+    return 2 * int64_t(sizeof(S)) * g.n * g.n * g.n;
+  };
+  for (size_t i = 0; i < grids.size();) {
+    int64_t total = bytes(grids[i]);
+    size_t end = i + 1;
+    while (end < grids.size() && total + bytes(grids[end]) <= kGroupBytes)
+      total += bytes(grids[end++]);
+    NPBX_TRY(group_sweeps<S>(dtype, &grids[i], end - i, enqueue, stream, launches, tiles));
+    i = end;
+  }
+  return NPBX_OK;
 }
 
 template <class S, int V, int kPlanes, int kUnroll>
@@ -229,6 +370,14 @@ int heat_entry(int dtype, void* A, void* B, int64_t N, int64_t first, int64_t ns
 }
 
 }  // namespace
+
+int heat_batch_sweeps(int dtype, const std::vector<SweepGrid>& grids, bool enqueue,
+                      hipStream_t stream, int64_t* launches, int64_t* tiles) {
+  return dispatch_dtype(dtype, [&](auto tag) {
+    return batch_sweeps<decltype(tag)>(dtype, grids, enqueue, stream, launches, tiles);
+  });
+}
+
 }  // namespace npbx
 
 extern "C" int npbx_heat3d(int dtype, void* A, void* B, int64_t N, int64_t tsteps, int tblock,

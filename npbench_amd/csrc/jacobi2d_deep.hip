@@ -31,11 +31,13 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
 #include "lanes.h"
 #include "points.h"
+#include "tiles.h"
 #include "vecio.h"
 
 namespace npbx {
@@ -73,23 +75,29 @@ __device__ __forceinline__ void sweep_rows(const Rows<C, V, R>& x, Rows<C, V, R>
   }
 }
 
-template <class S, int V, int R, bool NARROW>
-__global__ __launch_bounds__(64 * kWaves) void jacobi2d_block(const S* __restrict__ X,
-                                                              S* __restrict__ Y,
-                                                              const S* __restrict__ A,
-                                                              const S* __restrict__ B, int n,
-                                                              int parity0, int depth, int tiles_j,
-                                                              int tiles_i) {
-  using St = Storage<S>;
-  using C = typename St::C;
+// LDS of a workgroup.
+template <class C, int V>
+struct BlockLds {
   struct alignas(sizeof(C) * V) Cols {
     C v[V];
   };
-  __shared__ Cols edge[2][kWaves][2][64];  // per level parity: each wave's first and last row
-  __shared__ Cols outer[2][2][64];         // per level parity: the rows above and below the region
+  Cols edge[2][kWaves][2][64];  // per level parity: each wave's first and last row
+  Cols outer[2][2][64];         // per level parity: the rows above and below the region
+};
+
+template <class S, int V, int R, bool NARROW>
+__device__ __forceinline__ void block_sweeps(const S* __restrict__ X, S* __restrict__ Y,
+                                             const S* __restrict__ A, const S* __restrict__ B,
+                                             int n, int parity0, int depth, int tiles_j,
+                                             int tiles_i, int tile,
+                                             BlockLds<typename Storage<S>::C, V>& lds) {
+  using St = Storage<S>;
+  using C = typename St::C;
+  using Cols = typename BlockLds<C, V>::Cols;
+  auto& edge = lds.edge;
+  auto& outer = lds.outer;
   const int lane = threadIdx.x % 64;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-  const int tile = xcd_tile(blockIdx.x, gridDim.x);
   const Span sj = span_of(tile % tiles_j, tiles_j, n - 2, 64 * V, depth);
   const Span si = span_of(tile / tiles_j, tiles_i, n - 2, R * kWaves, depth);
   const int gj = sj.origin + lane * V, gi0 = si.origin + w * R;
@@ -202,6 +210,47 @@ __global__ __launch_bounds__(64 * kWaves) void jacobi2d_block(const S* __restric
   }
 }
 
+template <class S, int V, int R, bool NARROW>
+__global__ __launch_bounds__(64 * kWaves) void jacobi2d_block(const S* __restrict__ X,
+                                                              S* __restrict__ Y,
+                                                              const S* __restrict__ A,
+                                                              const S* __restrict__ B, int n,
+                                                              int parity0, int depth, int tiles_j,
+                                                              int tiles_i) {
+  __shared__ BlockLds<typename Storage<S>::C, V> lds;
+  block_sweeps<S, V, R, NARROW>(X, Y, A, B, n, parity0, depth, tiles_j, tiles_i,
+                                xcd_tile(blockIdx.x, gridDim.x), lds);
+}
+
+// Whether a side's grid is smaller than a region.
+__host__ __device__ constexpr bool narrow(int n, int v, int rows) {
+  return n - 2 < 64 * v || n - 2 < rows * kWaves;
+}
+
+// The rounds of several grids: block t belongs to the round g with cum[g] <= t
+// < cum[g+1].
+template <class S, int V, int R>
+__global__ __launch_bounds__(64 * kWaves) void jacobi2d_blocks(const BlockBatch b) {
+  __shared__ BlockLds<typename Storage<S>::C, V> lds;
+  const int t = xcd_tile(blockIdx.x, gridDim.x);
+  int lo = 0, hi = b.count - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (b.cum[mid] <= t) lo = mid; else hi = mid - 1;
+  }
+  const BlockRound& g = b.round[lo];
+  auto run = [&](auto is_narrow) {
+    block_sweeps<S, V, R, decltype(is_narrow)::value>(
+        static_cast<const S*>(g.X), static_cast<S*>(g.Y), static_cast<const S*>(g.A),
+        static_cast<const S*>(g.B), g.n, g.parity0, g.depth, g.tiles_j, g.tiles_i,
+        t - b.cum[lo], lds);
+  };
+  if (narrow(g.n, V, R))
+    run(std::true_type{});
+  else
+    run(std::false_type{});
+}
+
 // Launch shape: columns per lane, rows per wave and sweeps per launch.
 struct Shape {
   int v, rows, depth;
@@ -219,28 +268,39 @@ constexpr Shape kShapes[] = {{1, 3, 0}, {1, 4, 0}, {2, 3, 0}, {2, 4, 0},
 // FP64 150^2 1 x 3 rows, depth 20 (52 us for 98 sweeps, 2 x 8: 167); 1000^2
 // 2 x 5, 19 (204 us for 200; 1 x 3: 626); 2800^2 2 x 4, 12 (513 us for 100;
 // 2 x 8: 717).
-Shape pick_shape(int dtype, int n, int64_t nsweeps, int cap) {
+// Several grids advance by a round each per launch: as many launches as the
+// grid with the most rounds has, and their mean number of workgroups.
+Shape pick_shape(int dtype, const std::vector<SweepGrid>& grids, int cap, int max_points = 16) {
   Shape best{2, 4, 2};
   double best_us = INFINITY;
   const bool fp64 = dtype == NPBX_F64;
   for (const Shape& sh : kShapes) {
+    if (sh.v * sh.rows > max_points) continue;
     const int wj = 64 * sh.v, wi = kWaves * sh.rows;
     const double issue =
         sh.rows * (5.0 * sh.v + (fp64 ? 4 : 2) + (dtype == NPBX_BF16 ? 2.0 * sh.v : 0));
     const int resident = fp64 && sh.rows * sh.v > 8 ? 1 : 2;
     for (int depth = std::min(cap, 4); depth <= std::min(cap, kMaxDepth); depth += 2) {
       if (wj - 2 * depth < 8 || wi - 2 * depth < 8) break;
-      // sweep_rounds: that many rounds and a last one of depth 1
-      int64_t rounds = cdiv(nsweeps - 1, depth);
-      rounds += (rounds ^ (nsweeps - 1)) & 1;
-      const int d = static_cast<int>(cdiv(nsweeps - 1, std::max<int64_t>(rounds, 1)));
-      const double tiles =
-          static_cast<double>(span_count(n - 2, wj, d)) * span_count(n - 2, wi, d) / 256;
-      const double shared = std::min<double>(resident, std::ceil(tiles));
+      double launches = 0, blocks = 0, d = 1;
+      for (const SweepGrid& g : grids) {
+        // sweep_rounds: that many rounds and a last one of depth 1
+        int64_t rounds = cdiv(g.nsweeps - 1, depth);
+        rounds += (rounds ^ (g.nsweeps - 1)) & 1;
+        const int dg = static_cast<int>(cdiv(g.nsweeps - 1, std::max<int64_t>(rounds, 1)));
+        blocks += static_cast<double>(rounds) * span_count(g.n - 2, wj, dg) *
+                  span_count(g.n - 2, wi, dg);
+        if (static_cast<double>(rounds) > launches) {
+          launches = static_cast<double>(rounds);
+          d = dg;
+        }
+      }
+      const double tiles = blocks / std::max(launches, 1.0) / 256;
+      const double shared = std::max(1.0, std::min<double>(resident, std::ceil(tiles)));
       const double turns = std::max(1.0, (tiles / shared + std::ceil(tiles / shared)) / 2);
-      const double sweep = 0.06 + 0.0091 * issue * (1.0 - static_cast<double>(d) / wi) * shared;
-      const double us = static_cast<double>(rounds) *
-                        (5.4 + turns * d * sweep + (turns - 1) * (resident == 1 ? 10 : 2.5));
+      const double sweep = 0.06 + 0.0091 * issue * (1.0 - d / wi) * shared;
+      const double us =
+          launches * (5.4 + turns * d * sweep + (turns - 1) * (resident == 1 ? 10 : 2.5));
       if (us < best_us) {
         best_us = us;
         best = {sh.v, sh.rows, depth};
@@ -255,12 +315,26 @@ void launch_shape(const S* X, S* Y, const S* A, const S* B, int n, int parity, i
                   hipStream_t stream) {
   const int tj = span_count(n - 2, 64 * V, depth), ti = span_count(n - 2, R * kWaves, depth);
   const dim3 grid(static_cast<unsigned>(int64_t(tj) * ti)), block(64 * kWaves);
-  if (n - 2 < 64 * V || n - 2 < R * kWaves)
+  if (narrow(n, V, R))
     hipLaunchKernelGGL((jacobi2d_block<S, V, R, true>), grid, block, 0, stream, X, Y, A, B, n,
                        parity, depth, tj, ti);
   else
     hipLaunchKernelGGL((jacobi2d_block<S, V, R, false>), grid, block, 0, stream, X, Y, A, B, n,
                        parity, depth, tj, ti);
+}
+
+// Calls f.template operator()<V, R>() for a shape of kShapes.
+template <class F>
+int with_shape(int v, int rows, F&& f) {
+  switch (v * 10 + rows) {
+    case 13: return f.template operator()<1, 3>();
+    case 14: return f.template operator()<1, 4>();
+    case 23: return f.template operator()<2, 3>();
+    case 24: return f.template operator()<2, 4>();
+    case 25: return f.template operator()<2, 5>();
+    case 26: return f.template operator()<2, 6>();
+    default: return f.template operator()<2, 8>();
+  }
 }
 
 }  // namespace
@@ -276,7 +350,8 @@ int jacobi_deep_max() { return kDeep; }
 int jacobi_deep_sweeps(int dtype, void* A, void* B, int n, int64_t first, int64_t nsweeps, int T,
                        hipStream_t stream) {
   NPBX_REQUIRE(T >= 2 && T <= kDeep, "jacobi.deep=%d outside [2, %d]", T, kDeep);
-  const Shape shape = pick_shape(dtype, n, nsweeps, T == kDeep ? kMaxDepth : T);
+  const Shape shape =
+      pick_shape(dtype, {{A, B, n, first, nsweeps}}, T == kDeep ? kMaxDepth : T);
   return dispatch_dtype(dtype, [&](auto tag) -> int {
     using S = decltype(tag);
     S* a = static_cast<S*>(A);
@@ -288,20 +363,72 @@ int jacobi_deep_sweeps(int dtype, void* A, void* B, int n, int64_t first, int64_
     for (int depth : sweep_rounds(nsweeps, shape.depth)) {
       S* Y = X == a ? b : a;
       const int parity = static_cast<int>(level & 1);
-      auto go = [&](auto launch) { launch(X, Y, a, b, n, parity, depth, stream); };
-      switch (shape.v * 10 + shape.rows) {
-        case 13: go(launch_shape<S, 1, 3>); break;
-        case 14: go(launch_shape<S, 1, 4>); break;
-        case 23: go(launch_shape<S, 2, 3>); break;
-        case 24: go(launch_shape<S, 2, 4>); break;
-        case 25: go(launch_shape<S, 2, 5>); break;
-        case 26: go(launch_shape<S, 2, 6>); break;
-        default: go(launch_shape<S, 2, 8>); break;
-      }
+      with_shape(shape.v, shape.rows, [&]<int V, int R>() {
+        launch_shape<S, V, R>(X, Y, a, b, n, parity, depth, stream);
+        return NPBX_OK;
+      });
       NPBX_LAUNCHED("jacobi2d_block");
       X = Y;
       level += depth;
     }
+    return NPBX_OK;
+  });
+}
+
+// Launch r runs round r of every grid that has one.
+int jacobi_batch_plan(int dtype, const std::vector<SweepGrid>& grids, BlockPlan& plan) {
+  // more than 10 FP64 points a lane spill beside the NARROW form
+  const Shape shape = pick_shape(dtype, grids, kMaxDepth, dtype == NPBX_F64 ? 10 : 16);
+  plan.v = shape.v;
+  plan.rows = shape.rows;
+  std::vector<std::vector<int>> depths;
+  size_t nrounds = 0;
+  for (const SweepGrid& g : grids) {
+    depths.push_back(sweep_rounds(g.nsweeps, shape.depth));
+    nrounds = std::max(nrounds, depths.back().size());
+  }
+  std::vector<int64_t> level;
+  for (const SweepGrid& g : grids) level.push_back(g.first);
+  // round r reads the array that holds its first level: A or B by the parity
+  // of `first`, then in turn
+  for (size_t r = 0; r < nrounds; ++r) {
+    bool open = false;
+    for (size_t i = 0; i < grids.size(); ++i) {
+      if (r >= depths[i].size()) continue;
+      if (!open || plan.launches.back().count == kMaxBatch) {
+        plan.launches.emplace_back();
+        plan.launches.back().count = 0;
+        plan.launches.back().cum[0] = 0;
+        open = true;
+      }
+      const SweepGrid& g = grids[i];
+      BlockBatch& b = plan.launches.back();
+      const bool from_a = ((g.first + static_cast<int64_t>(r)) & 1) == 0;
+      const int depth = depths[i][r];
+      const int tj = span_count(g.n - 2, 64 * shape.v, depth);
+      const int ti = span_count(g.n - 2, shape.rows * kWaves, depth);
+      const int64_t end = b.cum[b.count] + int64_t(tj) * ti;
+      NPBX_REQUIRE(end < (int64_t(1) << 31), "jacobi batch: too many blocks");
+      b.round[b.count] = {g.A, g.B, from_a ? g.A : g.B, from_a ? g.B : g.A, g.n,
+                          static_cast<int32_t>(level[i] & 1), depth, tj, ti};
+      b.cum[++b.count] = static_cast<int32_t>(end);
+      level[i] += depth;
+    }
+  }
+  return NPBX_OK;
+}
+
+int jacobi_batch_launch(int dtype, const BlockPlan& plan, hipStream_t stream) {
+  return dispatch_dtype(dtype, [&](auto tag) -> int {
+    using S = decltype(tag);
+    for (const BlockBatch& b : plan.launches)
+      NPBX_TRY(with_shape(plan.v, plan.rows, [&]<int V, int R>() -> int {
+        hipLaunchKernelGGL((jacobi2d_blocks<S, V, R>),
+                           dim3(static_cast<unsigned>(b.cum[b.count])), dim3(64 * kWaves), 0,
+                           stream, b);
+        NPBX_LAUNCHED("jacobi2d_blocks");
+        return NPBX_OK;
+      }));
     return NPBX_OK;
   });
 }

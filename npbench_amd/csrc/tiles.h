@@ -2,7 +2,10 @@
 // host-side planner.
 #pragma once
 
+#include <hip/hip_runtime.h>
+
 #include <cstdint>
+#include <vector>
 
 namespace npbx {
 
@@ -40,6 +43,42 @@ struct RoundBatch {
   int32_t cum[kMaxBatch + 1];
   GridRound round[kMaxBatch];
 };
+
+// A grid of a plan that runs outside the tile kernels: sweeps [first,
+// first + nsweeps) between A and B.
+struct SweepGrid {
+  void* A;
+  void* B;
+  int n;
+  int64_t first, nsweeps;
+};
+
+// One 2-D grid in one launch of register blocks (jacobi2d_deep.hip), as
+// GridRound without the tiles.
+struct BlockRound {
+  const void* A;
+  const void* B;
+  const void* X;
+  void* Y;
+  int32_t n, parity0, depth, tiles_j, tiles_i;
+};
+struct BlockBatch {
+  int32_t count;
+  int32_t cum[kMaxBatch + 1];
+  BlockRound round[kMaxBatch];
+};
+// A batch's launches and the shape they share: columns per lane, rows per wave.
+struct BlockPlan {
+  int v = 0, rows = 0;
+  std::vector<BlockBatch> launches;
+};
+int jacobi_batch_plan(int dtype, const std::vector<SweepGrid>& grids, BlockPlan& plan);
+int jacobi_batch_launch(int dtype, const BlockPlan& plan, hipStream_t stream);
+
+// The plain sweeps of several heat grids, one launch per sweep of all of them
+// (heat3d.hip); with `enqueue` false only counts launches and workgroups.
+int heat_batch_sweeps(int dtype, const std::vector<SweepGrid>& grids, bool enqueue,
+                      hipStream_t stream, int64_t* launches, int64_t* tiles);
 
 // Per-launch queue state, self-resetting: `next` hands out tile indices and
 // `done` counts workgroups that found the queue empty; the last one resets

@@ -36,6 +36,7 @@
 // launches and graph replays need no memset and no device-side tile list.
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstring>
 #include <type_traits>
 #include <vector>
@@ -1170,7 +1171,10 @@ struct Plan {
   int T = 0;
   int rows = 4;
   int nblocks = 0;
-  std::vector<RoundBatch> launches;
+  std::vector<RoundBatch> launches;  // heat grids on tiles
+  std::vector<SweepGrid> sweeps;     // heat grids on plain sweeps
+  BlockPlan blocks;                  // 2-D grids
+  int64_t nlaunches = 0;
   std::vector<ColsPack> packs;  // grids whose boundary columns each launch packs
   float* d_cols = nullptr;
   QueueState* d_queue = nullptr;
@@ -1190,7 +1194,19 @@ int plan_free(Plan* p) {
   return NPBX_OK;
 }
 
+// EUNSUPPORTED unless the tile kernel is built for (T, rows), whichever form
+// the plan then takes.
+int built_shape(int dtype, int T, int rows) {
+  return dispatch_dtype(dtype, [&](auto tag) {
+    return with_shape<decltype(tag)>(T, rows, []<int, int>() { return NPBX_OK; });
+  });
+}
+
 int plan_enqueue(Plan* p, hipStream_t s) {
+  if (p->nlaunches > 0) NPBX_TRY(built_shape(p->dtype, p->T, p->rows));
+  NPBX_TRY(jacobi_batch_launch(p->dtype, p->blocks, s));
+  int64_t unused = 0;
+  NPBX_TRY(heat_batch_sweeps(p->dtype, p->sweeps, true, s, &unused, &unused));
   // A and B may have been rewritten since the last launch: pack their
   // boundary columns afresh (one small kernel per grid, before the rounds).
   for (const ColsPack& c : p->packs) NPBX_TRY(pack_cols(c.A, c.B, c.n, p->d_cols + c.off, s));
@@ -1200,6 +1216,50 @@ int plan_enqueue(Plan* p, hipStream_t s) {
     NPBX_TRY(launch_any(p->dtype, p->T, p->rows, b, p->d_queue, std::min(nt, p->nblocks), s));
   }
   return NPBX_OK;
+}
+
+// The planes per tile for a plan's heat grids (at most `seg`), or 0 where one
+// launch per plain sweep of all of them (heat_batch_sweeps) is faster: a
+// tile's march is a chain of some 2 us a plane, so tiles pay where there are
+// enough for the chip with many planes each, and only the wave-private ones
+// (the shared tile never did).  The shorter of, in us a sweep, fitted to
+// measured times of 1 to 8 grids of 64^3 to 256^3 (FP32, B = A.copy()):
+//   plain  3.5 + 1.45e-6 per point
+//   tiles  turns of 256 workgroups * (8.6 + 1.06 seg at T = 3, 7 + 0.92 seg at
+//          T = 2) + 0.19e-6 per point
+// Measured at T = 3, 14 rows, plain | 8, 22, 64 planes a tile:
+//   64^3 x 8     7.1 | 21  36  81      192^3 x 4   43 | 51  37  84
+//   128^3 x 4   16.1 | 21  35  81      256^3 x 2   53 | 38  36  83
+//   256^3 x 1   25.5 | 21  35  83      256^3 x 8  303 | 140 116 102
+int heat_tile_seg(int dtype, const std::vector<SweepGrid>& grids, int T, int rows, int seg) {
+  if (!uses_cols(kHeat3D, dtype, rows)) return 0;
+  int64_t longest = 0;
+  double points = 0;  // swept, over all sweeps
+  for (const SweepGrid& g : grids) {
+    longest = std::max(longest, g.nsweeps);
+    points += static_cast<double>(g.nsweeps) * g.n * g.n * g.n;
+  }
+  double best_us = 3.5 * static_cast<double>(longest) + 1.45e-6 * points;
+  int best = 0;
+  for (int s = seg; s >= 1; s = s > 8 ? s * 3 / 4 : s - 2) {
+    double tiles = 0;
+    for (const SweepGrid& g : grids) {
+      GridRound r{};
+      r.n = g.n;
+      r.kind = kHeat3D;
+      tile_grid(r, kHeat3D, g.n, dtype, T, s);
+      tiles += static_cast<double>(g.nsweeps) * static_cast<double>(tiles_per_round(r));
+    }
+    const double turns = std::ceil(tiles / static_cast<double>(longest) / 256);
+    const double us = static_cast<double>(longest) * turns *
+                          (T == 3 ? 8.6 + 1.06 * s : 7 + 0.92 * s) +
+                      0.19e-6 * points;
+    if (us < best_us) {
+      best_us = us;
+      best = s;
+    }
+  }
+  return best;
 }
 
 int new_queue(QueueState** q) {
@@ -1222,40 +1282,65 @@ extern "C" int npbx_plan_create(const npbx_grid_spec* specs, int32_t count, int3
                tblock, tmax, dtype_name(dtype));
   if (seg <= 0) seg = g_heat_seg.load();
   std::vector<GridRound> base(count);
-  std::vector<std::vector<int>> depths(count);
-  size_t nrounds = 0;
+  std::vector<SweepGrid> flat, heat;
   int64_t lups = 0;
   for (int i = 0; i < count; ++i) {
     const npbx_grid_spec& s = specs[i];
     NPBX_TRY(check_grid("plan_create", i, s.kind, s.dtype, s.n, s.A, s.B, dtype, base[i]));
     NPBX_REQUIRE(s.first >= 0 && s.nsweeps >= 0, "plan_create: grid %d negative sweeps", i);
-    tile_grid(base[i], base[i].kind, base[i].n, dtype, tblock, seg);
-    depths[i] = round_depths(s.nsweeps, tblock);
-    nrounds = std::max(nrounds, depths[i].size());
     lups += grid_lups(base[i], s.nsweeps);
+    if (s.nsweeps > 0)
+      (base[i].kind == kHeat3D ? heat : flat)
+          .push_back({s.A, s.B, base[i].n, s.first, s.nsweeps});
   }
-  // Launch group r runs round r of every grid that has one.
+  const int rows = g_heat_rows.load();
   auto p = new Plan();
   p->dtype = dtype;
   p->T = tblock;
+  p->rows = rows;
   p->lups = lups;
-  int64_t cols_total = 0;
-  for (int i = 0; i < count; ++i)
-    if (uses_cols(base[i].kind, dtype, base[i].rows)) {
-      p->packs.push_back({specs[i].A, specs[i].B, base[i].n, cols_total});
-      cols_total += (cols_elems(base[i].n) + 63) / 64 * 64;  // 256-byte aligned
-    }
-  if (cols_total > 0) {
-    const hipError_t e = hipMalloc(reinterpret_cast<void**>(&p->d_cols),
-                                   static_cast<size_t>(cols_total) * sizeof(float));
-    if (e != hipSuccess) {
-      plan_free(p);
-      return fail(NPBX_ENOMEM, "plan_create: %s", hipGetErrorString(e));
-    }
-    size_t k = 0;
-    for (int i = 0; i < count; ++i)
-      if (uses_cols(base[i].kind, dtype, base[i].rows)) base[i].cols = p->d_cols + p->packs[k++].off;
+  auto built = [&](int rc) {
+    if (rc != NPBX_OK) plan_free(p);
+    return rc;
+  };
+  if (!flat.empty()) {
+    NPBX_TRY(built(jacobi_batch_plan(dtype, flat, p->blocks)));
+    p->nlaunches += static_cast<int64_t>(p->blocks.launches.size());
+    for (const BlockBatch& b : p->blocks.launches) p->ntiles += b.cum[b.count];
   }
+  const int tile_seg = heat.empty() ? 0 : heat_tile_seg(dtype, heat, tblock, rows, seg);
+  if (tile_seg == 0) {
+    p->sweeps = heat;
+    NPBX_TRY(built(heat_batch_sweeps(dtype, heat, false, nullptr, &p->nlaunches, &p->ntiles)));
+    *plan = p;
+    return NPBX_OK;
+  }
+  // Heat grids on tiles: launch group r runs round r of every grid that has one.
+  std::erase_if(base, [](const GridRound& g) { return g.kind != kHeat3D; });
+  count = static_cast<int32_t>(base.size());
+  std::vector<npbx_grid_spec> heat_specs;
+  for (const npbx_grid_spec* s = specs; heat_specs.size() < base.size(); ++s)
+    if (s->kind == NPBX_KIND_HEAT3D) heat_specs.push_back(*s);
+  specs = heat_specs.data();
+  std::vector<std::vector<int>> depths(count);
+  size_t nrounds = 0;
+  for (int i = 0; i < count; ++i) {
+    tile_grid(base[i], base[i].kind, base[i].n, dtype, tblock, tile_seg);
+    depths[i] = round_depths(specs[i].nsweeps, tblock);
+    nrounds = std::max(nrounds, depths[i].size());
+  }
+  int64_t cols_total = 0;
+  for (int i = 0; i < count; ++i) {
+    p->packs.push_back({specs[i].A, specs[i].B, base[i].n, cols_total});
+    cols_total += (cols_elems(base[i].n) + 63) / 64 * 64;  // 256-byte aligned
+  }
+  const hipError_t e = hipMalloc(reinterpret_cast<void**>(&p->d_cols),
+                                 static_cast<size_t>(cols_total) * sizeof(float));
+  if (e != hipSuccess) {
+    plan_free(p);
+    return fail(NPBX_ENOMEM, "plan_create: %s", hipGetErrorString(e));
+  }
+  for (int i = 0; i < count; ++i) base[i].cols = p->d_cols + p->packs[i].off;
   std::vector<int64_t> level(count);
   std::vector<void*> X(count);
   for (int i = 0; i < count; ++i) {
@@ -1278,13 +1363,9 @@ extern "C" int npbx_plan_create(const npbx_grid_spec* specs, int32_t count, int3
     for (auto& b : pk.out) p->launches.push_back(b);
     p->ntiles += pk.tiles;
   }
-  p->rows = base[0].rows;
+  p->nlaunches += static_cast<int64_t>(p->launches.size());
   p->nblocks = resident_blocks(dtype, tblock, p->rows);
-  const int rc = new_queue(&p->d_queue);
-  if (rc != NPBX_OK) {
-    plan_free(p);
-    return rc;
-  }
+  NPBX_TRY(built(new_queue(&p->d_queue)));
   *plan = p;
   return NPBX_OK;
 }
@@ -1320,7 +1401,7 @@ extern "C" int npbx_plan_capture(void* plan, void* stream) {
 extern "C" int npbx_plan_info(void* plan, int64_t* launches, int64_t* tiles, int64_t* lups) {
   NPBX_REQUIRE(plan, "plan_info: null plan");
   const Plan* p = static_cast<const Plan*>(plan);
-  if (launches) *launches = static_cast<int64_t>(p->launches.size());
+  if (launches) *launches = p->nlaunches;
   if (tiles) *tiles = p->ntiles;
   if (lups) *lups = p->lups;
   return NPBX_OK;

@@ -272,6 +272,47 @@ def test_plan_batch_wave_tiles(st, heat_rows, T, rows):
         plan.close()
 
 
+def _device_batch(dtype, specs):
+    """(kind, n, nsweeps, first) -> the grids of a plan and copies of them."""
+    from npbench_amd import batch
+    gen = torch.Generator(device="cuda").manual_seed(len(specs))
+    gs, alone = [], []
+    for kind, n, ns, first in specs:
+        shape = (n,) * (2 if kind == "jacobi_2d" else 3)
+        a, b = (torch.rand(shape, generator=gen, device="cuda").to(DT[dtype]) for _ in range(2))
+        gs.append(batch.Grid(kind, a, b, ns, first))
+        alone.append((a.clone(), b.clone()))
+    return gs, alone
+
+
+# more grids than one launch takes, regions wider and narrower than a grid,
+# every row form of the heat sweeps; FP64: heat grids of two cache groups;
+# FP32: heat grids on tiles, with fewer planes a tile than asked for
+@pytest.mark.parametrize("dtype,T,rows,specs", [
+    ("f32", 2, 4, [("jacobi_2d", 8 * (1 + i % 40), 1 + i % 23, i) for i in range(60)] +
+     [("heat_3d", 8 * (1 + i % 5), 1 + i % 9, i) for i in range(55)]),
+    ("f64", 2, 4, [("jacobi_2d", n, 41, n // 8) for n in (4, 64, 128, 130, 258, 1000)] +
+     [("heat_3d", n, 3, n // 2) for n in (4, 114, 180, 232, 240)]),
+    ("bf16", 2, 4, [("jacobi_2d", n, 30, 0) for n in (8, 136, 1024)] +
+     [("heat_3d", n, 4, 1) for n in (8, 128, 136, 280, 288)]),
+    ("f32", 3, 14, [("heat_3d", 256, 8, i) for i in range(4)] +
+     [("heat_3d", 36, 20, 1), ("jacobi_2d", 520, 9, 1)]),
+    ("f32", 2, 12, [("heat_3d", 264, 5, i) for i in range(3)]),
+])
+def test_plan_forms_match_each_grid_alone(st, heat_rows, dtype, T, rows, specs):
+    from npbench_amd import batch
+    heat_rows(rows)
+    gs, alone = _device_batch(dtype, specs)
+    print(f"plan forms {dtype} T={T} rows={rows} grids={len(specs)}", flush=True)
+    plan = batch.Plan(gs, tblock=T, seg=64)
+    plan.launch()
+    for g, (a, b), (kind, n, ns, first) in zip(gs, alone, specs):
+        f = st.jacobi2d_sweeps if kind == "jacobi_2d" else st.heat3d_sweeps
+        f(a, b, ns, first=first)
+        assert torch.equal(g.A, a) and torch.equal(g.B, b), f"{kind} n={n} first={first}"
+    plan.close()
+
+
 def test_pack_cols_layout(st):
     """npbx_pack_cols: cols[a][q][j][s] = (A, B)[a][q][j][(0, n-1)[s]], then
     one word that is 1 exactly when A's and B's boundaries are equal (each
