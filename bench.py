@@ -147,8 +147,7 @@ def batched_fp32(st, dev, batch, tune, torch, clock, args, A64):
             plan.capture(side)
             clock = type(clock)(dev, side)
         launches = plan.info()["launches"]
-        kind = "wave-private" if cfg["rows"] >= 10 else "shared"
-        kernel = f"stencil_tiles<float,T={cfg['T']},R={cfg['rows']}> ({kind} heat tile)"
+        kernel = "heat_march"
 
         def step():
             plan.launch(clock.stream)
@@ -156,7 +155,8 @@ def batched_fp32(st, dev, batch, tune, torch, clock, args, A64):
         step()
     wall, ev = clock.run(step, args.steps)
     # algorithmic bytes: one read and one write of every grid per round trip
-    bytes_per_lup = 2 * SIZE["f32"] / cfg["T"]
+    round_trips = SWEEPS if plan is None else launches
+    bytes_per_lup = 2 * SIZE["f32"] * round_trips / SWEEPS
     glups = lup_step * args.steps / wall / 1e9
     rl = roofline(bytes_per_lup * lup_step / launches, ev / (args.steps * launches), kernel)
     # T-independent view: the bandwidth a plain sweep would need for this rate

@@ -139,13 +139,13 @@ int npbx_heat3d_sweeps(int dtype, void *A, void *B, int64_t N, int64_t first,
 /* ---- batched grids: many independent grids in shared launches -------------
  * No reference counterpart: the batched and serving forms of the two
  * explicit kernels.  A plan fixes a list of grids (each with its own side,
- * arrays and sweep range, all of one dtype) and a temporal-blocking depth
- * `tblock` (2..4 FP32, 2 FP64/BF16).  Its launches advance all grids of a
- * kind together: 2-D grids by blocks of up to 28 sweeps, heat grids by rounds
- * of up to `tblock` sweeps as one persistent kernel over a device work-tile
- * queue, or, where the plan expects that to be faster, by single sweeps.
- * Results are bitwise those of the per-grid entry points.  `seg` = most heat
- * planes per tile (0 = default).  Each grid's side must be a multiple of 16
+ * arrays and sweep range, all of one dtype).  Its launches advance all grids
+ * of a kind together: 2-D grids by register blocks of up to 28 sweeps, heat
+ * grids by rounds of up to 4 sweeps (FP32) or by single sweeps, whichever the
+ * plan expects to be faster.  Results are bitwise those of the per-grid entry
+ * points.  `tblock` (2..4 FP32, 2 FP64/BF16) and `seg` describe the tiles of
+ * the serving form below; a plan checks `tblock` and "heat.rows" as that does
+ * and chooses its own depths.  Each grid's side must be a multiple of 16
  * bytes of elements.
  * npbx_plan_capture records the plan's launches into a HIP graph on a
  * non-default stream; later npbx_plan_launch calls replay the graph. */

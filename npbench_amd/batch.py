@@ -1,12 +1,13 @@
 """Batched grids: many independent Jacobi 2-D / heat 3-D grids of uneven size
-advanced together (libnpbx plans): 2-D grids in register blocks, heat grids on
-tiles of ``tblock`` sweeps or by single sweeps, whichever suits their sizes.
+advanced together (libnpbx plans): 2-D grids in register blocks, heat grids in
+rounds of up to four sweeps or by single sweeps, whichever suits their sizes.
 
-A ``Plan`` fixes the grids (device tensors A, B of one storage dtype), each
-grid's sweep range, the temporal-blocking depth and the most planes of a heat
-tile (``seg``).  ``launch()`` enqueues every round; ``capture()`` records them into a HIP graph on a side stream so
-later launches replay the graph.  Results are bitwise those of running each
-grid alone with the per-grid entry points.
+A ``Plan`` fixes the grids (device tensors A, B of one storage dtype) and each
+grid's sweep range; ``tblock`` and ``seg`` name a tile shape of the serving
+rounds and do not bind a plan.  ``launch()`` enqueues every round;
+``capture()`` records them into a HIP graph on a side stream so later launches
+replay the graph.  Results are bitwise those of running each grid alone with
+the per-grid entry points.
 """
 
 import ctypes

@@ -45,6 +45,7 @@
 
 #include "common.h"
 #include "division.h"
+#include "lanes.h"
 
 namespace npbx {
 namespace {
@@ -186,16 +187,6 @@ constexpr int kQRows = 280;
 __device__ __forceinline__ void opaque(int& t, int& n, int& lb) {
   asm volatile("" : "+v"(t));
   asm volatile("" : "+s"(n), "+s"(lb));
-}
-
-// A workgroup barrier that orders LDS only.  The chunk loops' barriers guard
-// the LDS tiles; with __syncthreads they would also wait for every global
-// store in flight (the per-step stores of q and v), which the other threads
-// never read within the sweep.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // Per-sweep constants of the forward pass.

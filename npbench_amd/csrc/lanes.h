@@ -52,6 +52,15 @@ __device__ __forceinline__ C lane_from_right_or(C edge, C x) {
   return dpp_or<0x130>(edge, x);
 }
 
+// A workgroup barrier that orders LDS only: with __syncthreads the waves would
+// also wait for every global load and store in flight, which the other threads
+// do not touch.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // A direction of a grid split into blocks that advance several sweeps per
 // launch: n interior points, regions of `width` points held by a workgroup,
 // halos of `depth` points where a region ends inside the grid and none where

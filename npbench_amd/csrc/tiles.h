@@ -80,6 +80,14 @@ int jacobi_batch_launch(int dtype, const BlockPlan& plan, hipStream_t stream);
 int heat_batch_sweeps(int dtype, const std::vector<SweepGrid>& grids, bool enqueue,
                       hipStream_t stream, int64_t* launches, int64_t* tiles);
 
+// Rounds of FP32 heat grids on wave-stacked tiles (heatmarch.hip): depths up
+// to kHeatMarchDepth, sides of at least kHeatMarchRows.  A batch's cum counts
+// planes of tile columns: (columns of a round) * (n - 2) each.
+constexpr int kHeatMarchDepth = 4;
+constexpr int kHeatMarchRows = 33;
+int heat_march_columns(int n, int depth, int* tiles_k, int* tiles_j);
+int heat_march_launch(const RoundBatch& b, int blocks, hipStream_t stream);
+
 // Per-launch queue state, self-resetting: `next` hands out tile indices and
 // `done` counts workgroups that found the queue empty; the last one resets
 // both to zero for the next launch.

@@ -327,26 +327,6 @@ __device__ __forceinline__ void heat_tile(const GridRound g, int tile,
 constexpr int kPrivateRows = 10;  // heat.rows >= this selects the wave-private tile
 constexpr bool wave_private(int rows) { return rows >= kPrivateRows; }
 
-// Raw buffer loads from one plane (num_records = the plane's bytes; the
-// descriptor's third word is the gfx9 raw-buffer format).  The 32-bit vector
-// offset is the lane's, the scalar offset the wave's row.
-struct Rsrc {
-  __amdgpu_buffer_rsrc_t r;
-};
-__device__ __forceinline__ Rsrc plane_rsrc(const float* base, int64_t elems) {
-  return {__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), static_cast<short>(0),
-                                            static_cast<int>(elems * 4), 0x00020000)};
-}
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ void buf_load16(Rsrc rs, uint32_t voff, uint32_t soff, float (&d)[4]) {
-  const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rs.r, voff, soff, 0);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) d[i] = __uint_as_float(v[i]);
-}
-__device__ __forceinline__ float buf_load1(Rsrc rs, uint32_t voff, uint32_t soff) {
-  return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs.r, voff, soff, 0));
-}
-
 // Full-wave DPP shifts (wave_shr:1, wave_shl:1): lane l receives lane l-1's
 // (from_left) or lane l+1's (from_right) value; lane 0 / lane 63 receive 0,
 // which only ever reaches halo or global-boundary points.
@@ -880,11 +860,30 @@ std::atomic<int> g_sweep_shape{0};
 // when A's and B's global boundaries (all six faces) are bitwise equal, as
 // when B = A.copy(); the tile then takes every boundary value from its own
 // registers (the value of any level there is the same).
-__global__ void pack_flag_kernel(int* __restrict__ flag) { *flag = 1; }
+// Grids share launches (grid.y): one at a time they took 71 us each at 256^3,
+// too few loads in flight for a line per value.
+struct PackBatch {
+  int32_t count;
+  struct {
+    const float* A;
+    const float* B;
+    float* cols;
+    int32_t n;
+  } grid[kMaxBatch];
+};
 
-__global__ __launch_bounds__(256) void pack_cols_kernel(const float* __restrict__ A,
-                                                        const float* __restrict__ B,
-                                                        float* __restrict__ cols, int n) {
+__global__ void pack_flag_kernel(const PackBatch b) {
+  const int i = threadIdx.x;
+  if (i < b.count)
+    *reinterpret_cast<int*>(b.grid[i].cols + 4 * static_cast<int64_t>(b.grid[i].n) * b.grid[i].n) =
+        1;
+}
+
+__global__ __launch_bounds__(256) void pack_cols_kernel(const PackBatch b) {
+  const float* __restrict__ A = b.grid[blockIdx.y].A;
+  const float* __restrict__ B = b.grid[blockIdx.y].B;
+  float* __restrict__ cols = b.grid[blockIdx.y].cols;
+  const int n = b.grid[blockIdx.y].n;
   const int64_t nn = static_cast<int64_t>(n) * n;
   int* flag = reinterpret_cast<int*>(cols + 4 * nn);
   unsigned same = 1;  // bitwise and of every comparison: no branch between the loads
@@ -920,17 +919,24 @@ __global__ __launch_bounds__(256) void pack_cols_kernel(const float* __restrict_
 
 int64_t cols_elems(int64_t n) { return 4 * n * n + 1; }
 
-int pack_cols(const void* A, const void* B, int n, void* cols, hipStream_t stream) {
-  const int64_t nn = static_cast<int64_t>(n) * n;
-  int* flag = reinterpret_cast<int*>(static_cast<float*>(cols) + 4 * nn);
-  hipLaunchKernelGGL(pack_flag_kernel, dim3(1), dim3(1), 0, stream, flag);
+int pack_batch(const PackBatch& b, hipStream_t stream) {
+  int64_t n = 0;
+  for (int i = 0; i < b.count; ++i) n = std::max<int64_t>(n, b.grid[i].n);
+  hipLaunchKernelGGL(pack_flag_kernel, dim3(1), dim3(64), 0, stream, b);
   NPBX_LAUNCHED("pack_flag");
-  const unsigned blocks = static_cast<unsigned>(std::min<int64_t>(cdiv(4 * nn, 256), 4096));
-  hipLaunchKernelGGL(pack_cols_kernel, dim3(blocks), dim3(256), 0, stream,
-                     static_cast<const float*>(A), static_cast<const float*>(B),
-                     static_cast<float*>(cols), n);
+  const unsigned blocks = static_cast<unsigned>(std::min<int64_t>(cdiv(4 * n * n, 256), 4096));
+  hipLaunchKernelGGL(pack_cols_kernel, dim3(blocks, static_cast<unsigned>(b.count)), dim3(256), 0,
+                     stream, b);
   NPBX_LAUNCHED("pack_cols");
   return NPBX_OK;
+}
+
+int pack_cols(const void* A, const void* B, int n, void* cols, hipStream_t stream) {
+  PackBatch b;
+  b.count = 1;
+  b.grid[0] = {static_cast<const float*>(A), static_cast<const float*>(B),
+               static_cast<float*>(cols), n};
+  return pack_batch(b, stream);
 }
 
 // Whether a grid's rounds run the wave-private tile (and so use packed columns).
@@ -1037,12 +1043,17 @@ int launch_any(int dtype, int T, int RH, const RoundBatch& b, QueueState* queue,
   });
 }
 
+int compute_units() {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return 256;
+  return cus;
+}
+
 // Workgroups that fit on the device at once for the persistent grid.
 int resident_blocks(int dtype, int T, int RH) {
-  int dev = 0, cus = 0, per_cu = 1;
-  if (hipGetDevice(&dev) != hipSuccess) return 1024;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    cus = 256;
+  int per_cu = 1;
   dispatch_dtype(dtype, [&](auto tag) {
     using S = decltype(tag);
     return with_shape<S>(T, RH, [&]<int TT, int RR>() {
@@ -1054,7 +1065,7 @@ int resident_blocks(int dtype, int T, int RH) {
       return NPBX_OK;
     });
   });
-  return cus * per_cu;
+  return compute_units() * per_cu;
 }
 
 }  // namespace
@@ -1171,13 +1182,12 @@ struct Plan {
   int T = 0;
   int rows = 4;
   int nblocks = 0;
-  std::vector<RoundBatch> launches;  // heat grids on tiles
+  std::vector<RoundBatch> launches;  // heat grids' rounds (heatmarch.hip)
   std::vector<SweepGrid> sweeps;     // heat grids on plain sweeps
   BlockPlan blocks;                  // 2-D grids
   int64_t nlaunches = 0;
   std::vector<ColsPack> packs;  // grids whose boundary columns each launch packs
   float* d_cols = nullptr;
-  QueueState* d_queue = nullptr;
   int64_t ntiles = 0, lups = 0;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -1188,7 +1198,6 @@ int plan_free(Plan* p) {
   // Release paths ignore errors: the plan is gone either way.
   if (p->exec) (void)hipGraphExecDestroy(p->exec);
   if (p->graph) (void)hipGraphDestroy(p->graph);
-  if (p->d_queue) (void)hipFree(p->d_queue);
   if (p->d_cols) (void)hipFree(p->d_cols);
   delete p;
   return NPBX_OK;
@@ -1208,58 +1217,53 @@ int plan_enqueue(Plan* p, hipStream_t s) {
   int64_t unused = 0;
   NPBX_TRY(heat_batch_sweeps(p->dtype, p->sweeps, true, s, &unused, &unused));
   // A and B may have been rewritten since the last launch: pack their
-  // boundary columns afresh (one small kernel per grid, before the rounds).
-  for (const ColsPack& c : p->packs) NPBX_TRY(pack_cols(c.A, c.B, c.n, p->d_cols + c.off, s));
+  // boundary columns afresh (before the rounds).
+  PackBatch pack;
+  pack.count = 0;
+  for (const ColsPack& c : p->packs) {
+    pack.grid[pack.count++] = {static_cast<const float*>(c.A), static_cast<const float*>(c.B),
+                               p->d_cols + c.off, c.n};
+    if (pack.count == kMaxBatch || &c == &p->packs.back()) {
+      NPBX_TRY(pack_batch(pack, s));
+      pack.count = 0;
+    }
+  }
   for (const RoundBatch& b : p->launches) {
-    const int nt = b.cum[b.count];
-    if (nt == 0) continue;
-    NPBX_TRY(launch_any(p->dtype, p->T, p->rows, b, p->d_queue, std::min(nt, p->nblocks), s));
+    NPBX_TRY(heat_march_launch(b, p->nblocks, s));
   }
   return NPBX_OK;
 }
 
-// The planes per tile for a plan's heat grids (at most `seg`), or 0 where one
-// launch per plain sweep of all of them (heat_batch_sweeps) is faster: a
-// tile's march is a chain of some 2 us a plane, so tiles pay where there are
-// enough for the chip with many planes each, and only the wave-private ones
-// (the shared tile never did).  The shorter of, in us a sweep, fitted to
-// measured times of 1 to 8 grids of 64^3 to 256^3 (FP32, B = A.copy()):
-//   plain  3.5 + 1.45e-6 per point
-//   tiles  turns of 256 workgroups * (8.6 + 1.06 seg at T = 3, 7 + 0.92 seg at
-//          T = 2) + 0.19e-6 per point
-// Measured at T = 3, 14 rows, plain | 8, 22, 64 planes a tile:
-//   64^3 x 8     7.1 | 21  36  81      192^3 x 4   43 | 51  37  84
-//   128^3 x 4   16.1 | 21  35  81      256^3 x 2   53 | 38  36  83
-//   256^3 x 1   25.5 | 21  35  83      256^3 x 8  303 | 140 116 102
-int heat_tile_seg(int dtype, const std::vector<SweepGrid>& grids, int T, int rows, int seg) {
-  if (!uses_cols(kHeat3D, dtype, rows)) return 0;
+// The depth of the rounds that a plan's heat grids take on wave-stacked tiles
+// (heatmarch.hip, FP32), or 0 where one launch per plain sweep of all of them
+// is faster.  A march is a chain of some 2.3 us a plane with 2 D planes of
+// filling, so it pays where a workgroup has planes enough.  The shorter of, in
+// us a sweep, fitted to measured times of 1 to 8 grids of 64^3 to 256^3:
+//   plain  3.3 + 1.42e-6 per point
+//   march  1.25 (5 + 2.3 (planes a workgroup + 10)) / 4, the factor for grids
+//          whose A and B have different boundaries
+// Measured, plain | march, B = A.copy() | march, other boundaries:
+//   64^3 x 8    6.3 | 10.9 | 13.9       128^3 x 8   25 | 18 | 25
+//   128^3 x 1   6.5 |  6.7 |  8.5       192^3 x 2   21 | 14 | 20
+//   128^3 x 4    15 |   14 |   18       256^3 x 1   24 | 15 | 20
+//   192^3 x 1    13 |   11 |   16       256^3 x 8  179 | 64 | 92
+// (Tiles of the serving rounds: 256^3 x 1 83, 256^3 x 8 102 | 133.)
+int heat_round_depth(int dtype, const std::vector<SweepGrid>& grids) {
+  if (dtype != NPBX_F32) return 0;
   int64_t longest = 0;
-  double points = 0;  // swept, over all sweeps
+  double points = 0, planes = 0;  // over all sweeps
   for (const SweepGrid& g : grids) {
+    if (g.n < kHeatMarchRows) return 0;
+    int tk, tj;
+    const double sweeps = static_cast<double>(g.nsweeps);
     longest = std::max(longest, g.nsweeps);
-    points += static_cast<double>(g.nsweeps) * g.n * g.n * g.n;
+    points += sweeps * g.n * g.n * g.n;
+    planes += sweeps * heat_march_columns(g.n, kHeatMarchDepth, &tk, &tj) * (g.n - 2);
   }
-  double best_us = 3.5 * static_cast<double>(longest) + 1.45e-6 * points;
-  int best = 0;
-  for (int s = seg; s >= 1; s = s > 8 ? s * 3 / 4 : s - 2) {
-    double tiles = 0;
-    for (const SweepGrid& g : grids) {
-      GridRound r{};
-      r.n = g.n;
-      r.kind = kHeat3D;
-      tile_grid(r, kHeat3D, g.n, dtype, T, s);
-      tiles += static_cast<double>(g.nsweeps) * static_cast<double>(tiles_per_round(r));
-    }
-    const double turns = std::ceil(tiles / static_cast<double>(longest) / 256);
-    const double us = static_cast<double>(longest) * turns *
-                          (T == 3 ? 8.6 + 1.06 * s : 7 + 0.92 * s) +
-                      0.19e-6 * points;
-    if (us < best_us) {
-      best_us = us;
-      best = s;
-    }
-  }
-  return best;
+  const double sweeps = static_cast<double>(longest);
+  const double part = std::ceil(planes / sweeps / compute_units());
+  const double march = sweeps * 1.25 * (5 + 2.3 * (part + 10)) / kHeatMarchDepth;
+  return march < sweeps * 3.3 + 1.42e-6 * points ? kHeatMarchDepth : 0;
 }
 
 int new_queue(QueueState** q) {
@@ -1271,7 +1275,7 @@ int new_queue(QueueState** q) {
 }  // namespace
 
 extern "C" int npbx_plan_create(const npbx_grid_spec* specs, int32_t count, int32_t tblock,
-                                int32_t seg, void** plan) {
+                                int32_t /*seg*/, void** plan) {
   NPBX_REQUIRE(plan, "plan_create: null output pointer");
   *plan = nullptr;
   NPBX_REQUIRE(specs && count > 0, "plan_create: no grids");
@@ -1280,7 +1284,6 @@ extern "C" int npbx_plan_create(const npbx_grid_spec* specs, int32_t count, int3
   const int tmax = max_depth(dtype);
   NPBX_REQUIRE(tblock >= 2 && tblock <= tmax, "plan_create: tblock=%d outside [2, %d] for %s",
                tblock, tmax, dtype_name(dtype));
-  if (seg <= 0) seg = g_heat_seg.load();
   std::vector<GridRound> base(count);
   std::vector<SweepGrid> flat, heat;
   int64_t lups = 0;
@@ -1308,8 +1311,8 @@ extern "C" int npbx_plan_create(const npbx_grid_spec* specs, int32_t count, int3
     p->nlaunches += static_cast<int64_t>(p->blocks.launches.size());
     for (const BlockBatch& b : p->blocks.launches) p->ntiles += b.cum[b.count];
   }
-  const int tile_seg = heat.empty() ? 0 : heat_tile_seg(dtype, heat, tblock, rows, seg);
-  if (tile_seg == 0) {
+  const int depth = heat.empty() ? 0 : heat_round_depth(dtype, heat);
+  if (depth == 0) {
     p->sweeps = heat;
     NPBX_TRY(built(heat_batch_sweeps(dtype, heat, false, nullptr, &p->nlaunches, &p->ntiles)));
     *plan = p;
@@ -1325,8 +1328,7 @@ extern "C" int npbx_plan_create(const npbx_grid_spec* specs, int32_t count, int3
   std::vector<std::vector<int>> depths(count);
   size_t nrounds = 0;
   for (int i = 0; i < count; ++i) {
-    tile_grid(base[i], base[i].kind, base[i].n, dtype, tblock, tile_seg);
-    depths[i] = round_depths(specs[i].nsweeps, tblock);
+    depths[i] = round_depths(specs[i].nsweeps, depth);
     nrounds = std::max(nrounds, depths[i].size());
   }
   int64_t cols_total = 0;
@@ -1348,24 +1350,32 @@ extern "C" int npbx_plan_create(const npbx_grid_spec* specs, int32_t count, int3
     X[i] = (level[i] & 1) ? specs[i].B : specs[i].A;
   }
   for (size_t r = 0; r < nrounds; ++r) {
-    Packer pk;
+    bool open = false;
     for (int i = 0; i < count; ++i) {
       if (r >= depths[i].size()) continue;
+      if (!open || p->launches.back().count == kMaxBatch) {
+        p->launches.emplace_back();
+        std::memset(&p->launches.back(), 0, sizeof(RoundBatch));
+        open = true;
+      }
       GridRound g = base[i];
       g.X = X[i];
       g.Y = X[i] == specs[i].A ? specs[i].B : specs[i].A;
       g.parity0 = static_cast<int32_t>(level[i] & 1);
       g.depth = depths[i][r];
-      pk.add(g);
+      const int64_t columns = heat_march_columns(g.n, g.depth, &g.tiles_k, &g.tiles_j);
+      RoundBatch& b = p->launches.back();
+      const int64_t end = b.cum[b.count] + columns * (g.n - 2);
+      if (end >= (int64_t(1) << 31)) return built(fail(NPBX_EINVAL, "plan_create: too many tiles"));
+      b.round[b.count] = g;
+      b.cum[++b.count] = static_cast<int32_t>(end);
       X[i] = g.Y;
       level[i] += g.depth;
+      p->ntiles += columns;
     }
-    for (auto& b : pk.out) p->launches.push_back(b);
-    p->ntiles += pk.tiles;
   }
   p->nlaunches += static_cast<int64_t>(p->launches.size());
-  p->nblocks = resident_blocks(dtype, tblock, p->rows);
-  NPBX_TRY(built(new_queue(&p->d_queue)));
+  p->nblocks = compute_units();
   *plan = p;
   return NPBX_OK;
 }
@@ -1409,7 +1419,7 @@ extern "C" int npbx_plan_info(void* plan, int64_t* launches, int64_t* tiles, int
 
 extern "C" int npbx_plan_destroy(void* plan) {
   if (!plan) return NPBX_OK;
-  // hipFree waits for work that may still use the queue state.
+  // hipFree waits for work that may still use the packed columns.
   return plan_free(static_cast<Plan*>(plan));
 }
 

@@ -145,6 +145,23 @@ __device__ __forceinline__ void storev_stream(S* __restrict__ p,
   __builtin_nontemporal_store(__builtin_bit_cast(vec_t, w), reinterpret_cast<at_t*>(p));
 }
 
+// Raw buffer loads from one plane (num_records = the plane's bytes; the
+// descriptor's third word is the gfx9 raw-buffer format).  The 32-bit vector
+// offset is the lane's, the scalar offset the wave's row.
+struct Rsrc {
+  __amdgpu_buffer_rsrc_t r;
+};
+__device__ __forceinline__ Rsrc plane_rsrc(const float* base, int64_t elems) {
+  return {__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), static_cast<short>(0),
+                                            static_cast<int>(elems * 4), 0x00020000)};
+}
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void buf_load16(Rsrc rs, uint32_t voff, uint32_t soff, float (&d)[4]) {
+  const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rs.r, voff, soff, 0);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) d[i] = __uint_as_float(v[i]);
+}
+
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // Workgroups of a 1-D grid are handed to the 8 XCDs round-robin (block b runs

@@ -272,7 +272,7 @@ def test_plan_batch_wave_tiles(st, heat_rows, T, rows):
         plan.close()
 
 
-def _device_batch(dtype, specs):
+def _device_batch(dtype, specs, same_boundary):
     """(kind, n, nsweeps, first) -> the grids of a plan and copies of them."""
     from npbench_amd import batch
     gen = torch.Generator(device="cuda").manual_seed(len(specs))
@@ -280,6 +280,8 @@ def _device_batch(dtype, specs):
     for kind, n, ns, first in specs:
         shape = (n,) * (2 if kind == "jacobi_2d" else 3)
         a, b = (torch.rand(shape, generator=gen, device="cuda").to(DT[dtype]) for _ in range(2))
+        if same_boundary:
+            b = a.clone()
         gs.append(batch.Grid(kind, a, b, ns, first))
         alone.append((a.clone(), b.clone()))
     return gs, alone
@@ -287,7 +289,8 @@ def _device_batch(dtype, specs):
 
 # more grids than one launch takes, regions wider and narrower than a grid,
 # every row form of the heat sweeps; FP64: heat grids of two cache groups;
-# FP32: heat grids on tiles, with fewer planes a tile than asked for
+# FP32: heat grids in rounds of every depth, parts that span columns and grids,
+# the smallest side such rounds take, and two tiles of columns
 @pytest.mark.parametrize("dtype,T,rows,specs", [
     ("f32", 2, 4, [("jacobi_2d", 8 * (1 + i % 40), 1 + i % 23, i) for i in range(60)] +
      [("heat_3d", 8 * (1 + i % 5), 1 + i % 9, i) for i in range(55)]),
@@ -295,14 +298,15 @@ def _device_batch(dtype, specs):
      [("heat_3d", n, 3, n // 2) for n in (4, 114, 180, 232, 240)]),
     ("bf16", 2, 4, [("jacobi_2d", n, 30, 0) for n in (8, 136, 1024)] +
      [("heat_3d", n, 4, 1) for n in (8, 128, 136, 280, 288)]),
-    ("f32", 3, 14, [("heat_3d", 256, 8, i) for i in range(4)] +
-     [("heat_3d", 36, 20, 1), ("jacobi_2d", 520, 9, 1)]),
-    ("f32", 2, 12, [("heat_3d", 264, 5, i) for i in range(3)]),
+    ("f32", 3, 14, [("heat_3d", 256, ns, ns) for ns in (17, 8, 6, 2)] +
+     [("heat_3d", n, 18, 1) for n in (36, 60, 132)] + [("jacobi_2d", 520, 9, 1)]),
+    ("f32", 2, 12, [("heat_3d", n, 5, i) for i, n in enumerate((264, 264, 248, 304))]),
 ])
-def test_plan_forms_match_each_grid_alone(st, heat_rows, dtype, T, rows, specs):
+@pytest.mark.parametrize("same_boundary", [False, True])
+def test_plan_forms_match_each_grid_alone(st, heat_rows, dtype, T, rows, specs, same_boundary):
     from npbench_amd import batch
     heat_rows(rows)
-    gs, alone = _device_batch(dtype, specs)
+    gs, alone = _device_batch(dtype, specs, same_boundary)
     print(f"plan forms {dtype} T={T} rows={rows} grids={len(specs)}", flush=True)
     plan = batch.Plan(gs, tblock=T, seg=64)
     plan.launch()
