@@ -32,10 +32,10 @@
 //    keep q in a scratch array laid out [step][line], read back one chunk
 //    ahead by the back substitutions.
 //
-// Grids of up to 256 lines run every time step in one workgroup and one
-// launch, a barrier between the halves; larger ones launch each half over
-// ceil(lines / 256) workgroups (one wave per SIMD either way: two waves on a
-// SIMD would share its issue slots, and the chain is issue-bound there).
+// Path 1 runs every time step in one workgroup and one launch, a barrier
+// between the halves; paths 2 and 3 launch each half over workgroups of 256 or
+// 64 lines (one wave per SIMD either way: two waves on a SIMD would share its
+// issue slots, and the chain is issue-bound there).
 #include <hip/hip_runtime.h>
 
 #include <atomic>
