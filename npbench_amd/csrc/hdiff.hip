@@ -362,11 +362,25 @@ std::atomic<int> g_hdiff_shape{0};
 // 21.5, 4 x 6 x 4: 27.0), BF16 4 x 6 x 4 14.8 (2 x 6 x 8: 15.0).  An odd K
 // leaves FP32 the 4-byte vectors (190 x 203 x 137: 13.4; a point per thread
 // 28.8) and BF16 the tail form of its own.
+// Small calls leave a march too few waves, each a chain of row loads: up to
+// kPoint points run a point per thread, and FP64 and FP32 up to
+// some millions one column x 6 rows of 16-byte vectors where these fit (us, a
+// call among others, point | 1 x 6 x 16 | the order above):
+//   FP64   60 x 60 x 40 3.7 | 4.2 | 5.5    104 x 100 x 98 11.7 | 7.3 | 9.0
+//         237 x 238 x 40 26 | 10.2 | 12.2  190 x 203 x 101 48 | - | 22.5
+//   FP32   60 x 60 x 40 2.3 | 4.6 | 5.4    147 x 126 x 64  5.4 | 5.8 | 6.1
+//         160 x 160 x 80 9.6 | 7.0 | 7.8   256 x 256 x 96  28 | 14.7 | 15.2
+//   BF16  103 x 78 x 55  3.1 | 7.9 | 7.9   147 x 126 x 64  5.0 | 6.9 | 7.5
+//         130 x 130 x 90 8.0 | 8.0 | 8.1   160 x 160 x 80  9.8 | 7.6 | 8.1
 template <class S>
-constexpr int march_order(int n) {
+constexpr int march_order(int n, int64_t points) {
   constexpr int f64[] = {14, 7, 1}, f32[] = {7, 9, 12, 1}, b16[] = {9, 12, 1};
-  if (sizeof(S) == 8) return n < 3 ? f64[n] : 0;
-  if (sizeof(S) == 4) return n < 4 ? f32[n] : 0;
+  constexpr int f64_mid[] = {2, 7, 1}, f32_mid[] = {2, 7, 9, 12, 1};
+  constexpr int64_t kPoint = sizeof(S) == 8 ? 250000 : sizeof(S) == 4 ? 900000 : 1250000;
+  if (points < kPoint) return 0;
+  if (sizeof(S) == 8) return n >= 3 ? 0 : points < 3200000 ? f64_mid[n] : f64[n];
+  if (sizeof(S) == 4)
+    return points < 5000000 ? (n < 5 ? f32_mid[n] : 0) : n < 4 ? f32[n] : 0;
   return n < 3 ? b16[n] : 0;
 }
 
@@ -800,15 +814,16 @@ int run_hdiff(const S* in, S* out, const S* coeff, int I, int J, int K, int64_t 
     return m.w <= J && m.vb >= int(sizeof(S)) && K * int64_t(sizeof(S)) % m.vb == 0 &&
            aligned_to(m.vb);
   };
+  const int64_t points = int64_t(I) * J * K;
   int shape = g_hdiff_shape.load();
   if (shape <= 0 || shape >= kMarchShapeCount || !fits(shape)) {
     int n = 0;
-    do shape = march_order<S>(n++);
+    do shape = march_order<S>(n++, points);
     while (shape && !fits(shape));
   }
   // BF16 columns that no 4-byte vector divides: the last vector of a column is
   // shifted back to end with it, and addresses are aligned to elements only.
-  const bool tail = sizeof(S) == 2 && !shape && J >= 4 && K >= 2;
+  const bool tail = sizeof(S) == 2 && !shape && J >= 4 && K >= 2 && points >= 1250000;
   if (tail) shape = 9;
   const bool vec = shape != 0;
   const bool aligned = aligned_to(16);

@@ -153,8 +153,8 @@ def _heat_exactly(x, y):
 # of the vectors; bases that are aligned to their elements alone
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n,off", [(3, 1), (4, 0), (7, 1), (9, 0), (64, 1), (88, 0), (89, 1),
-                                   (112, 1), (113, 0), (128, 1), (129, 0), (176, 1), (177, 0),
-                                   (192, 0), (193, 1), (257, 0), (280, 1), (281, 0)])
+                                   (112, 1), (113, 0), (128, 1), (129, 0), (176, 1), (177, 0), (130, 1), (131, 0),
+                                   (192, 0), (193, 1), (194, 0), (195, 1), (257, 0), (280, 1), (281, 0)])
 def test_heat3d_sweep_shapes_bitwise(st, dtype, n, off):
     print(f"heat3d shapes {dtype} n={n} off={off}", flush=True)
     gen = torch.Generator().manual_seed(31 * n + off)
@@ -314,6 +314,32 @@ def _unaligned(a, dt):
     v = buf[1:].view(a.shape)
     v.copy_(torch.from_numpy(a).to(dt))
     return v
+
+
+# both sides of the point counts where the default shape changes (250,000,
+# 900,000, 1,250,000, 3,200,000 and 5,000,000), K odd, even and whole vectors
+@pytest.mark.parametrize("precision", ["fp64", "fp32", "bf16"])
+@pytest.mark.parametrize("I,J,K", [(66, 71, 53), (71, 66, 54), (97, 96, 96), (98, 97, 95),
+                                   (104, 122, 97), (109, 120, 97), (160, 161, 123),
+                                   (163, 160, 124), (200, 193, 129), (202, 195, 128)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_hdiff_default_shapes_by_size(st, hdiff_shape, precision, I, J, K, offset):
+    """Bitwise one march shape (a column x 6 rows) on columns padded to whole
+    16-byte vectors."""
+    dt = {"fp64": torch.float64, "fp32": torch.float32, "bf16": torch.bfloat16}[precision]
+    inf, out, coeff = _hdiff_inputs(I, J, K, 5 * I + J + K)
+    pad = lambda a: np.concatenate([a, np.zeros(a.shape[:2] + (-K % 8,))], axis=2)  # noqa: E731
+    hdiff_shape(2)
+    want = dev(pad(out), dt)
+    st.hdiff(dev(pad(inf), dt), want, dev(pad(coeff), dt))
+    hdiff_shape(0)
+    put = _unaligned if offset else dev
+    got = put(out, dt)
+    print(f"hdiff by size {precision} {I}x{J}x{K} offset={offset}", flush=True)
+    st.hdiff(put(inf, dt), got, put(coeff, dt))
+    torch.cuda.synchronize()
+    assert torch.equal(got.contiguous().view(torch.uint8),
+                       want[:, :, :K].contiguous().view(torch.uint8))
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32", "bf16"])
