@@ -58,6 +58,13 @@ __global__ __launch_bounds__(kLanes* kCols) void heat3d_sweep(const S* __restric
   }
 }
 
+// The first column a wave takes: vectors start with the row, single points
+// with its interior, so that 64 m + 2 points take m waves.
+__host__ __device__ constexpr int first_column(int v) { return v == 1 ? 1 : 0; }
+int k_tiles(int n, int v) {
+  return static_cast<int>(cdiv(n - 2 * first_column(v), kLanes * v));
+}
+
 // kPlanes = planes per workgroup (i segment); kUnroll = planes whose loads
 // are issued together (run_sweeps below).  A row's last vector is shifted
 // back to end with it where vectors do not divide the row; it shares points,
@@ -70,10 +77,10 @@ __device__ __forceinline__ void sweep_tile(const S* __restrict__ src, S* __restr
   const int tk = t % tiles_k;
   const int tj = (t / tiles_k) % tiles_j;
   const int ti = t / (tiles_k * tiles_j);
-  const int kv = (tk * kLanes + threadIdx.x) * V;
+  const int kv = (tk * kLanes + threadIdx.x) * V + first_column(V);
   const int j = 1 + tj * kCols + threadIdx.y;
   const int i0 = 1 + ti * kPlanes;
-  if (kv >= n || j > n - 2) return;
+  if (kv >= n - first_column(V) || j > n - 2) return;
   const int k0 = min(kv, n - V);
   const int i_end = min(i0 + kPlanes, n - 1);
   const int64_t plane = static_cast<int64_t>(n) * n;
@@ -245,7 +252,7 @@ int group_sweeps(int dtype, const SweepGrid* grids, size_t count, bool enqueue,
       d.dst = even ? g.B : g.A;
       d.n = g.n;
       d.form = form;
-      d.tiles_k = static_cast<int32_t>(cdiv(g.n, kLanes * f.v));
+      d.tiles_k = k_tiles(g.n, f.v);
       d.tiles_j = static_cast<int32_t>(cdiv(g.n - 2, kCols));
       const int64_t nt = int64_t(d.tiles_k) * d.tiles_j * cdiv(g.n - 2, f.planes);
       NPBX_REQUIRE(b.cum[b.count] + nt < (int64_t(1) << 31), "heat batch: too many tiles");
@@ -276,7 +283,7 @@ int batch_sweeps(int dtype, const std::vector<SweepGrid>& grids, bool enqueue,
 template <class S, int V, int kPlanes, int kUnroll>
 int run_vec(S* A, S* B, int n, int64_t first, int64_t nsweeps, hipStream_t stream) {
   const dim3 block(kLanes, kCols);
-  const int tiles_k = static_cast<int>(cdiv(n, kLanes * V));
+  const int tiles_k = k_tiles(n, V);
   const int tiles_j = static_cast<int>(cdiv(n - 2, kCols));
   const int tiles_i = static_cast<int>(cdiv(n - 2, kPlanes));
   const int64_t nblocks = int64_t(tiles_k) * tiles_j * tiles_i;
@@ -338,7 +345,10 @@ int run_sweeps(S* A, S* B, int n, int64_t first, int64_t nsweeps, hipStream_t st
   if (n <= 88) return run_vec<S, 2, 1, 1>(A, B, n, first, nsweeps, stream);
   if constexpr (std::is_same_v<S, double>) {
     if (n <= 112) return run_vec<S, 2, 2, 2>(A, B, n, first, nsweeps, stream);
-    if (n <= 176) return run_vec<S, 2, 4, 4>(A, B, n, first, nsweeps, stream);
+    // rows of 129 to 194 points fill two or three waves of single points:
+    // 129^3 9.7 us (vectors of two 11.4, 16 planes a thread 10.6), 177^3 20.3 | 20.7
+    if (n <= 128) return run_vec<S, 2, 4, 4>(A, B, n, first, nsweeps, stream);
+    if (n <= 194) return run_vec<S, 1, 4, 4>(A, B, n, first, nsweeps, stream);
     return run_vec<S, 2, 8, 4>(A, B, n, first, nsweeps, stream);
   } else if constexpr (std::is_same_v<S, float>) {
     if (n <= 112) return run_vec<S, 1, 4, 4>(A, B, n, first, nsweeps, stream);
