@@ -632,7 +632,7 @@ def kernel_suite(st, dev, torch, clock, reps, copy_only=False, cpu=False):
             "ms_per_call": round(ev / reps * 1e3, 4),
             "us_per_phase": round(ev / reps / phases * 1e6, 3),
             "glups": round(NT * (NIT + 2) * (NXC - 2) * (NYC - 2) * reps / ev / 1e9, 3),
-            "bound": "latency (one workgroup, a barrier per phase)"}
+            "bound": "latency (two launches a time step)"}
         del c0, c1
 
     # channel flow (FP64) at the paper preset from the reference
@@ -674,7 +674,7 @@ def kernel_suite(st, dev, torch, clock, reps, copy_only=False, cpu=False):
     res[f"seidel_2d_paper_N{NS}_T{TS}_f64"] = {
         "ms_per_call": round(ev / reps * 1e3, 4),
         "glups": round((TS - 1) * (NS - 2) ** 2 * reps / ev / 1e9, 3),
-        "bound": "latency (a serial recurrence per row, rows in wavefront slots)"}
+        "bound": "latency (serial recurrences, points of a wavefront together)"}
     del s0, s1
     return res
 
