@@ -258,8 +258,8 @@ __device__ __forceinline__ void helper_wave(const SeidelArgs& g, const Tile& t, 
   }
   // Helper 0 waits for all.  Every wait ends, because the tiles waited for run
   // already; the bound only keeps a broken launch from hanging the device, and
-  // its result is NaN.
-  double spoil = 0.0;
+  // its result is NaN.  (-0.0, which added to any value leaves its every bit)
+  double spoil = -0.0;
   auto wait_for = [&](int tau) {
     if (!WAIT || h != 0) return;
     for (int polls = 0; !__all(seen >= tau + ahead) && spoil == 0.0; ++polls) {

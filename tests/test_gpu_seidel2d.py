@@ -191,3 +191,28 @@ def test_seidel2d_captured(st, n, tsteps):
         torch.cuda.synchronize()
         c_oracle.seidel_2d_kernel(tsteps, n, want)
         assert_bitwise(d.cpu().numpy(), want, f"eager {rep}")
+
+
+@pytest.mark.parametrize("n,tsteps", [(5, 2), (140, 10)])
+@pytest.mark.parametrize("signs", ["all negative", "half"])
+@pytest.mark.parametrize("captured", [False, True])
+def test_seidel2d_signed_zeros(st, n, tsteps, signs, captured):
+    """Zeros keep the sign that the reference's sums give them, in every bit:
+    nine -0.0 sum to -0.0, and any +0.0 among them makes a sum +0.0."""
+    from npbench_amd import device
+    want = np.full((n, n), -0.0)
+    if signs == "half":  # every other block of rows, so that whole stencils are -0.0
+        want[(np.arange(n) // 16) % 2 == 1] = 0.0
+    d = device.to_device(want, torch.float64)
+    torch.cuda.synchronize()
+    print(f"seidel2d signed zeros n={n} tsteps={tsteps} {signs} captured={captured}", flush=True)
+    if captured:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            st.seidel2d(d, tsteps)
+        graph.replay()
+    else:
+        st.seidel2d(d, tsteps)
+    torch.cuda.synchronize()
+    ref.seidel_2d_kernel(tsteps, n, want)
+    assert np.array_equal(d.cpu().numpy().view(np.uint64), want.view(np.uint64))
