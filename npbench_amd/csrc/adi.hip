@@ -852,6 +852,19 @@ int launch_split(const AdiArgs& g, double* v, int ldv, int64_t tsteps, hipStream
   return NPBX_OK;
 }
 
+// The pitch of v beside ld lines a row: ld + 1, but in split half sweeps, whose
+// lines of v are n long and written by different workgroups, at least n (sides
+// of 64 m + 2 have ld = n - 2).
+constexpr int64_t pitch_of_v(int64_t n, int64_t ld, bool split) {
+  return split && ld + 1 < n ? n : ld + 1;
+}
+constexpr bool split_lines_apart() {
+  for (int64_t n = 3; SplitLds::bytes(static_cast<int>(n)) <= kLdsBytes; ++n)
+    if (pitch_of_v(n, (n - 2 + 63) / 64 * 64, true) < n) return false;
+  return true;
+}
+static_assert(split_lines_apart());
+
 // Launch shape and scratch layout of one call: v (the column sweep's output,
 // (n + 16) rows of ldv), q ([step][line], qrows x ld) and the eight tables.
 struct AdiPlan {
@@ -872,7 +885,7 @@ int plan_adi(int64_t n64, AdiPlan& pl) {
   pl.nt = pl.path == 1 ? (lines <= 256 ? 256 : 512) : pl.path == 3 ? 64 : 256;
   pl.nb = static_cast<int>(cdiv(lines, pl.nt));
   pl.ld = static_cast<int64_t>(pl.nb) * pl.nt;
-  pl.ldv = pl.ld + 1;
+  pl.ldv = pitch_of_v(n64, pl.ld, pl.split);
   pl.qrows = cdiv(lines, kCW) * kCW + 1;
   pl.tl = pl.qrows + 1;  // table length: every chunk's block
   pl.vel = (n64 + 16) * pl.ldv;

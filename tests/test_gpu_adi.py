@@ -80,6 +80,18 @@ def test_adi_split_edges_bitwise(st, adi_path, n):
     assert_bitwise(run_gpu(st, u, tsteps), want, f"adi split n={n}")
 
 
+@pytest.mark.parametrize("n", [66, 130])
+def test_adi_split_lines_of_whole_groups_bitwise(st, adi_path, n):
+    """Sides of 64 m + 2, whose lines of the scratch v would lie n - 1 apart
+    with the other forms' pitch (a compile-time check in adi.hip covers every
+    side)."""
+    u = np.random.default_rng(n).random((n, n))
+    want = ref.adi_kernel(3, n, u.copy())
+    adi_path(0)
+    print(f"adi split n={n}", flush=True)
+    assert_bitwise(run_gpu(st, u, 3), want, f"adi split n={n}")
+
+
 @pytest.mark.parametrize("tsteps,n", [(5, 100), (100, 200)])
 def test_adi_reference_presets_bitwise(st, tsteps, n):
     """The reference's initialisation at its S and paper presets; values grow
