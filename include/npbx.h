@@ -86,7 +86,8 @@ int npbx_stream_create(void **stream);
 int npbx_stream_destroy(void *stream);
 /* Waits for `stream` until it drains or the monotonic clock passes
  * deadline_ns (CLOCK_MONOTONIC nanoseconds; 0 = no deadline).  Polls, so a
- * host-side timeout can interrupt between calls (timeout_decorator.py:46-72). */
+ * host-side timeout can interrupt between calls (timeout_decorator.py:46-72).
+ * Also reports a failed npbx_seidel2d call on the current device (see there). */
 int npbx_sync(void *stream, int64_t deadline_ns);
 int npbx_event_create(void **event);
 int npbx_event_destroy(void *event);
@@ -237,7 +238,8 @@ int npbx_pack_cols(int dtype, const void *A, const void *B, int64_t n,
  * per thread, bytes of k per lane),
  * "seidel.blocks" = tiles (64 rows of a
  * group of 4 sweeps) per seidel_2d launch (default 2048; at most 4096 take
- * effect), "jacobi.deep" = 2-D Jacobi sweeps per launch at
+ * effect), "seidel.polls" = polls after which a tile that waits for another
+ * gives up (default 2^22, some seconds), "jacobi.deep" = 2-D Jacobi sweeps per launch at
  * tblock <= 1 (8, the default: up to 28, by size and type; 2 .. 7: at most
  * that many; 0 or 1: one launch per sweep), "jacobi.deep_waves" = 0, 4, 8 or
  * 16 (no effect: its workgroups have 16 waves).  Results do not depend on them. */
@@ -320,7 +322,10 @@ int npbx_channel_flow_launch(int dtype, int64_t nit, void *u, void *v,
  * launches of at most "seidel.blocks" tiles, so a launch's duration is bounded
  * whatever N is.  Under stream capture (and on a device npbx_init was not
  * called for) each wavefront step is a launch of its own.  Calls on different
- * streams do not share state. */
+ * streams do not share state.  Tiles that wait for others give up after
+ * "seidel.polls" polls (a device that stopped serving them): the grid then holds
+ * NaN, and the next npbx_seidel2d or npbx_sync on the device returns NPBX_EHIP
+ * once. */
 int npbx_seidel2d(int dtype, void *A, int64_t N, int64_t tsteps, void *stream);
 
 /* ---- alternating-direction implicit solver (adi_numpy.py:6-52) -------------

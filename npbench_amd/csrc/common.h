@@ -167,6 +167,11 @@ void set_vadv_path(int path);
 // sweeps).
 int seidel_blocks();
 void set_seidel_blocks(int blocks);
+// Polls after which a tile gives up waiting for another ("seidel.polls"), and
+// the report of it by the next call on the device.
+int seidel_polls();
+void set_seidel_polls(int polls);
+int seidel_failure();
 
 // Resolves the current device's address of npbx_adi_noalloc's fixed scratch
 // array (once per device; npbx_init calls it).

@@ -200,7 +200,7 @@ int npbx_sync(void* stream, int64_t deadline_ns) {
   int polls = 0;
   for (;;) {
     hipError_t q = hipStreamQuery(s);
-    if (q == hipSuccess) return NPBX_OK;
+    if (q == hipSuccess) return npbx::seidel_failure();
     if (q != hipErrorNotReady) return npbx::hip_fail(q, "hipStreamQuery", __FILE__, __LINE__);
     if (deadline_ns > 0 && npbx::monotonic_ns() >= deadline_ns)
       return fail(NPBX_ETIMEDOUT, "npbx_sync: deadline passed with work still queued");

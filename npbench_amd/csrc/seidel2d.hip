@@ -65,10 +65,11 @@ static_assert(64 % (kG * kW) == 0);
 constexpr int kMaxN = 1 << 14;
 constexpr int kMaxTiles = 4096;      // tiles per launch
 constexpr int kLine = 16;            // ints per counter
-constexpr int kMaxPolls = 1 << 22;   // some seconds
 
 // Tiles per launch ("seidel.blocks").
 std::atomic<int> g_seidel_blocks{2048};
+// Polls after which a wait gives up ("seidel.polls"): some seconds.
+std::atomic<int> g_seidel_polls{1 << 22};
 
 // What the workgroups of one launch share; all zero between launches.
 struct SeidelSync {
@@ -82,6 +83,8 @@ struct SeidelArgs {
   double* A;
   int n, sweeps;      // sweeps of this launch's groups in all
   int bands, groups;  // tiles per group, groups of this launch
+  int polls;          // after which a wait gives up
+  int* gave_up;       // host memory: set where one did
 };
 
 // Tiles read each other's rows within a launch.  Every access to A is an
@@ -177,7 +180,8 @@ struct Tile {
 struct SeidelLds {
   double ring[kW + 1][2][kG][kPitch];  // [0] from the loader, [w + 1] from wave w
   double2 edges[2][kW][kG];
-  int signs;  // nonzero once a value outside [2^-800, 2^800] came from A
+  double spoil;  // added to all that comes from A: -0.0, which changes no bit, or NaN
+  int signs;     // nonzero once a value outside [2^-800, 2^800] came from A
   int taken;
 };
 
@@ -257,16 +261,21 @@ __device__ __forceinline__ void helper_wave(const SeidelArgs& g, const Tile& t, 
     if (lane == 2) watch(t.grp - 1, t.band + 1, kBelow - 128 / kG + kW);
   }
   // Helper 0 waits for all.  Every wait ends, because the tiles waited for run
-  // already; the bound only keeps a broken launch from hanging the device, and
-  // its result is NaN.  (-0.0, which added to any value leaves its every bit)
-  double spoil = -0.0;
+  // already; the bound only keeps a broken launch from hanging the device.
+  // Where it is reached, all that the tile takes from A from then on is NaN,
+  // so the grid is from there on, and the host is told.
+  bool failed = false;
   auto wait_for = [&](int tau) {
     if (!WAIT || h != 0) return;
-    for (int polls = 0; !__all(seen >= tau + ahead) && spoil == 0.0; ++polls) {
+    for (int polls = 0; !failed && !__all(seen >= tau + ahead); ++polls) {
       seen = peek(watched);
-      if (polls >= kMaxPolls || (polls % 64 == 63 && peek(&sync->failed))) {
-        poke(&sync->failed, 1);
-        spoil = NAN;
+      if (polls < g.polls && !(polls % 64 == 63 && peek(&sync->failed))) continue;
+      if (__all(seen >= tau + ahead)) break;
+      failed = true;
+      poke(&sync->failed, 1);
+      if (lane == 0) {
+        lds.spoil = NAN;  // the helpers read it behind the next barrier
+        __hip_atomic_store(g.gave_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
       }
     }
     asm volatile("" ::: "memory");
@@ -278,7 +287,7 @@ __device__ __forceinline__ void helper_wave(const SeidelArgs& g, const Tile& t, 
     from[m] = min(2 + 64 * t.band + l, n - 1) * n;
   }
   const int erow = min(max(64 * t.band - h + (q & 1), 0), n - 1) * n;
-  double v[kPart], e = 1.0;
+  double v[kPart], e = 1.0, spoil = -0.0;
   auto load = [&](int tau) {
     const int c0 = tau * kG + k;  // the column lane row 0 of wave 0 needs, s + 1
 #pragma unroll
@@ -287,6 +296,7 @@ __device__ __forceinline__ void helper_wave(const SeidelArgs& g, const Tile& t, 
       v[m] = get(g.A + from[m] + min(max(c0 - 2 * l, 0), n - 1));
     }
     if (q < 2) e = get(g.A + erow + min(max(c0 - h * (kG + 1), 0), n - 1));
+    if constexpr (WAIT) spoil = lds.spoil;
   };
   auto commit = [&](int tau) {
     auto plain = [](double a) { return a >= 0x1p-800 && a <= 0x1p800; };
@@ -298,7 +308,7 @@ __device__ __forceinline__ void helper_wave(const SeidelArgs& g, const Tile& t, 
     }
     if (!__all(all)) lds.signs = 1;
     double2* to = &lds.edges[(tau + 1) & 1][h][k];
-    if (q < 2) (q ? to->y : to->x) = e;
+    if (q < 2) (q ? to->y : to->x) = e + spoil;
   };
   auto store = [&](int tau) {  // what interval tau computed
     const int par = tau & 1, c = tau - lw, s0 = c * kG - lw - 1 + k;
@@ -343,7 +353,7 @@ __global__ __launch_bounds__(kThreads) void seidel2d_tiles(SeidelArgs g, int slo
                                                            SeidelSync* sync) {
   __shared__ SeidelLds lds;
   const int tid = threadIdx.x, lane = tid % 64;
-  if (tid == 0) lds.signs = 0;
+  if (tid == 0) lds.signs = 0, lds.spoil = -0.0;
   const int w = __builtin_amdgcn_readfirstlane(tid / 64);
   Tile t;
   if constexpr (WAIT) {
@@ -405,6 +415,7 @@ struct SyncPool {
   SeidelSync* base = nullptr;  // null until seidel_setup ran on the device
   hipEvent_t last[kSyncSlots] = {};
   int next = 0;
+  std::atomic<int*> gave_up{nullptr};  // host memory the device writes
 };
 std::mutex g_pool_mu;
 SyncPool g_pool[kMaxDevices];
@@ -420,7 +431,7 @@ bool capturing(hipStream_t stream) {
 
 // One launch for all groups of g, or `launched` false where the device has no
 // counters.
-int launch_chained(const SeidelArgs& g, hipStream_t stream, bool& launched) {
+int launch_chained(SeidelArgs g, hipStream_t stream, bool& launched) {
   int dev = 0;
   NPBX_HIP(hipGetDevice(&dev));
   launched = false;
@@ -428,6 +439,8 @@ int launch_chained(const SeidelArgs& g, hipStream_t stream, bool& launched) {
   std::lock_guard<std::mutex> lock(g_pool_mu);
   SyncPool& pool = g_pool[dev];
   if (!pool.base) return NPBX_OK;
+  g.polls = g_seidel_polls.load();
+  g.gave_up = pool.gave_up.load();
   const int k = pool.next;
   NPBX_HIP(hipStreamWaitEvent(stream, pool.last[k], 0));
   hipLaunchKernelGGL(seidel2d_tiles<true>, dim3(g.bands * g.groups), dim3(kThreads), 0, stream, g,
@@ -455,6 +468,21 @@ int launch_slots(const SeidelArgs& g, hipStream_t stream) {
 
 int seidel_blocks() { return g_seidel_blocks.load(); }
 void set_seidel_blocks(int blocks) { g_seidel_blocks.store(blocks); }
+int seidel_polls() { return g_seidel_polls.load(); }
+void set_seidel_polls(int polls) { g_seidel_polls.store(polls); }
+
+// EHIP, once, where a wait of an earlier call on the current device gave up.
+int seidel_failure() {
+  int dev = 0;
+  NPBX_HIP(hipGetDevice(&dev));
+  if (dev < 0 || dev >= kMaxDevices) return NPBX_OK;
+  int* gave_up = g_pool[dev].gave_up.load();
+  if (!gave_up || !__atomic_load_n(gave_up, __ATOMIC_RELAXED) ||
+      !__atomic_exchange_n(gave_up, 0, __ATOMIC_RELAXED))
+    return NPBX_OK;
+  return fail(NPBX_EHIP, "seidel2d: a tile of an earlier call gave up waiting for another; "
+              "that call's grid holds NaN");
+}
 
 // The current device's counters and their events, once per device.
 int seidel_setup() {
@@ -468,6 +496,10 @@ int seidel_setup() {
   NPBX_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(seidel_sync)));
   for (hipEvent_t& e : pool.last)
     if (!e) NPBX_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  void* word = nullptr;
+  NPBX_HIP(hipHostMalloc(&word, kLine * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
+  *static_cast<int*>(word) = 0;
+  pool.gave_up.store(static_cast<int*>(word));
   pool.base = static_cast<SeidelSync*>(p);
   return NPBX_OK;
 }
@@ -483,8 +515,9 @@ extern "C" int npbx_seidel2d(int dtype, void* A, int64_t N, int64_t tsteps, void
   const int64_t sweeps = tsteps - 1;  // range(0, TSTEPS - 1)
   if (N < 3 || sweeps <= 0) return NPBX_OK;
   NPBX_REQUIRE(A != nullptr, "seidel2d: null array");
+  NPBX_TRY(seidel_failure());
   const hipStream_t s = as_stream(stream);
-  SeidelArgs g;
+  SeidelArgs g{};
   g.A = static_cast<double*>(A);
   g.n = static_cast<int>(N);
   g.bands = static_cast<int>(cdiv(N - 2 + kW - 1, 64));

@@ -1566,9 +1566,15 @@ extern "C" int npbx_set_tuning(const char* key, int64_t value) {
     set_seidel_blocks(static_cast<int>(value));
     return NPBX_OK;
   }
+  if (std::strcmp(key, "seidel.polls") == 0) {
+    NPBX_REQUIRE(value >= 0 && value <= (1 << 30), "set_tuning: seidel.polls must be in [0, 2^30]");
+    set_seidel_polls(static_cast<int>(value));
+    return NPBX_OK;
+  }
   return fail(NPBX_EINVAL,
               "set_tuning: unknown key '%s' (heat.rows, heat.seg, sweep.shape, hdiff.tblock, "
-              "hdiff.shape, hdiff.fuse_rows, adi.path, vadv.path, seidel.blocks, jacobi.deep, jacobi.deep_waves)",
+              "hdiff.shape, hdiff.fuse_rows, adi.path, vadv.path, seidel.blocks, seidel.polls, "
+              "jacobi.deep, jacobi.deep_waves)",
               key);
 }
 
@@ -1616,6 +1622,10 @@ extern "C" int npbx_get_tuning(const char* key, int64_t* value) {
   }
   if (std::strcmp(key, "seidel.blocks") == 0) {
     *value = seidel_blocks();
+    return NPBX_OK;
+  }
+  if (std::strcmp(key, "seidel.polls") == 0) {
+    *value = seidel_polls();
     return NPBX_OK;
   }
   return fail(NPBX_EINVAL, "get_tuning: unknown key '%s'", key);

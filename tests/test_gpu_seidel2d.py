@@ -216,3 +216,27 @@ def test_seidel2d_signed_zeros(st, n, tsteps, signs, captured):
     torch.cuda.synchronize()
     ref.seidel_2d_kernel(tsteps, n, want)
     assert np.array_equal(d.cpu().numpy().view(np.uint64), want.view(np.uint64))
+
+
+def test_seidel2d_wait_that_gives_up_is_reported(st):
+    """A wait that may poll once only gives up: the kernel ends, every row of
+    the tile that waited is NaN, and the next synchronisation (or call) says
+    so, once."""
+    from npbench_amd import _native, device
+    from oracle import c_oracle
+    n = 200
+    A = np.random.default_rng(6).random((n, n))
+    d = device.to_device(A, torch.float64)
+    old = _native.get_tuning("seidel.polls")
+    print("seidel2d bounded wait", flush=True)
+    _native.set_tuning("seidel.polls", 0)
+    try:
+        st.seidel2d(d, 2)
+    finally:
+        _native.set_tuning("seidel.polls", old)
+    with pytest.raises(_native.NpbxError, match="gave up"):
+        device.sync()
+    # the last band of 64 rows waits before its first column
+    assert np.isnan(d.cpu().numpy()[193:-1, 1:-1]).all()
+    device.sync()
+    check(st, 5, A, "after a failed call", oracle=c_oracle.seidel_2d_kernel)
