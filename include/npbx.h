@@ -142,8 +142,8 @@ int npbx_heat3d_sweeps(int dtype, void *A, void *B, int64_t N, int64_t first,
  * explicit kernels.  A plan fixes a list of grids (each with its own side,
  * arrays and sweep range, all of one dtype).  Its launches advance all grids
  * of a kind together: 2-D grids by register blocks of up to 28 sweeps, heat
- * grids by rounds of up to 4 sweeps (FP32) or by single sweeps, whichever the
- * plan expects to be faster.  Results are bitwise those of the per-grid entry
+ * grids each by rounds of up to 4 sweeps (FP32; FP64 2) or by single sweeps,
+ * whichever the plan expects to be faster.  Results are bitwise those of the per-grid entry
  * points.  `tblock` (2..4 FP32, 2 FP64/BF16) and `seg` describe the tiles of
  * the serving form below; a plan checks `tblock` and "heat.rows" as that does
  * and chooses its own depths.  Each grid's side must be a multiple of 16

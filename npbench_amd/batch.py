@@ -1,6 +1,7 @@
 """Batched grids: many independent Jacobi 2-D / heat 3-D grids of uneven size
-advanced together (libnpbx plans): 2-D grids in register blocks, heat grids in
-rounds of up to four sweeps or by single sweeps, whichever suits their sizes.
+advanced together (libnpbx plans): 2-D grids in register blocks, heat grids
+each in rounds of several sweeps or by single sweeps, whichever suits their
+sizes.
 
 A ``Plan`` fixes the grids (device tensors A, B of one storage dtype) and each
 grid's sweep range; ``tblock`` and ``seg`` name a tile shape of the serving

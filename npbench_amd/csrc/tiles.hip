@@ -955,10 +955,11 @@ int max_depth(int dtype) {
 
 int vec_elems(int dtype) { return static_cast<int>(16 / dtype_size(dtype)); }
 
-// Fills the tiling fields of a GridRound for side n and max depth T.
-void tile_grid(GridRound& g, int kind, int n, int dtype, int T, int seg) {
+// Fills the tiling fields of a GridRound for side n, max depth T and heat tiles
+// of `rows` rows a wave.
+void tile_grid(GridRound& g, int kind, int n, int dtype, int T, int rows, int seg) {
   const int V = vec_elems(dtype);
-  g.rows = g_heat_rows.load();
+  g.rows = rows;
   const int KT = 64 * V;
   g.tiles_k = n <= KT ? 1 : static_cast<int>(cdiv(n, KT - 2 * V));
   if (kind == kHeat3D) {
@@ -1088,7 +1089,7 @@ int tiled_sweeps(int kind, int dtype, void* A, void* B, int n, int64_t first, in
   g.B = B;
   g.n = n;
   g.kind = kind;
-  tile_grid(g, kind, n, dtype, T, seg > 0 ? seg : g_heat_seg.load());
+  tile_grid(g, kind, n, dtype, T, g_heat_rows.load(), seg > 0 ? seg : g_heat_seg.load());
   if (uses_cols(kind, dtype, g.rows)) {
     void* ws = nullptr;
     NPBX_TRY(workspace(static_cast<size_t>(cols_elems(n)) * sizeof(float), &ws));
@@ -1182,7 +1183,9 @@ struct Plan {
   int T = 0;
   int rows = 4;
   int nblocks = 0;
-  std::vector<RoundBatch> launches;  // heat grids' rounds (heatmarch.hip)
+  // heat grids' rounds: FP32 on wave-stacked tiles (heatmarch.hip), FP64 on
+  // this file's
+  std::vector<RoundBatch> launches;
   std::vector<SweepGrid> sweeps;     // heat grids on plain sweeps
   BlockPlan blocks;                  // 2-D grids
   int64_t nlaunches = 0;
@@ -1211,6 +1214,9 @@ int built_shape(int dtype, int T, int rows) {
   });
 }
 
+// Depth, rows a wave and planes of the tiles that a plan's FP64 grids take.
+constexpr int kTileDepth = 2, kTileRows = 2, kTileSeg = 32;
+
 int plan_enqueue(Plan* p, hipStream_t s) {
   if (p->nlaunches > 0) NPBX_TRY(built_shape(p->dtype, p->T, p->rows));
   NPBX_TRY(jacobi_batch_launch(p->dtype, p->blocks, s));
@@ -1229,16 +1235,22 @@ int plan_enqueue(Plan* p, hipStream_t s) {
     }
   }
   for (const RoundBatch& b : p->launches) {
-    NPBX_TRY(heat_march_launch(b, p->nblocks, s));
+    if (p->dtype == NPBX_F32)
+      NPBX_TRY(heat_march_launch(b, p->nblocks, s));
+    else
+      NPBX_TRY(launch_any(p->dtype, kTileDepth, kTileRows, b, nullptr, b.cum[b.count], s));
   }
   return NPBX_OK;
 }
 
-// The depth of the rounds that a plan's heat grids take on wave-stacked tiles
-// (heatmarch.hip, FP32), or 0 where one launch per plain sweep of all of them
-// is faster.  A march is a chain of some 2.3 us a plane with 2 D planes of
-// filling, so it pays where a workgroup has planes enough.  The shorter of, in
-// us a sweep, fitted to measured times of 1 to 8 grids of 64^3 to 256^3:
+// Which of a plan's heat grids advance in rounds of several sweeps; the others
+// take one launch per plain sweep of all of them (heat3d.hip).
+//
+// FP32: rounds on wave-stacked tiles (heatmarch.hip).  A march is a chain of
+// some 2.3 us a plane with 2 D planes of filling, so it pays where a workgroup
+// has planes enough: grids from some side on.  Of all such sides, and none, the
+// one with the shortest expected time: in us a sweep, fitted to measured times
+// of 1 to 8 grids of 64^3 to 256^3, the sum of
 //   plain  3.3 + 1.42e-6 per point
 //   march  1.25 (5 + 2.3 (planes a workgroup + 10)) / 4, the factor for grids
 //          whose A and B have different boundaries
@@ -1248,22 +1260,70 @@ int plan_enqueue(Plan* p, hipStream_t s) {
 //   128^3 x 4    15 |   14 |   18       256^3 x 1   24 | 15 | 20
 //   192^3 x 1    13 |   11 |   16       256^3 x 8  179 | 64 | 92
 // (Tiles of the serving rounds: 256^3 x 1 83, 256^3 x 8 102 | 133.)
-int heat_round_depth(int dtype, const std::vector<SweepGrid>& grids) {
-  if (dtype != NPBX_F32) return 0;
-  int64_t longest = 0;
-  double points = 0, planes = 0;  // over all sweeps
+// Plain sweeps of large and small grids overlap, so parting them has to win by
+// more: 256^3 and 64^3, 20 and 200 sweeps, 1047 us in plain sweeps, 1049 | 1165
+// parted, for 1210 and 1067 by the terms above; 8 x 256^3 and a 32^3, 20 sweeps,
+// 3730 and 1640 | 2200, for 3880 and 1510.
+//
+// FP64: rounds of two sweeps on this file's tiles (2 rows a wave, segments of 32
+// planes, the best of 12 shapes) for grids past the Infinity Cache, where a
+// sweep is bound by its bytes.  Columns of a tile that no point fills cost as
+// the others, so the tile's 124 of 128 useful columns decide beside the side:
+// us a sweep, plain | tiles, 320^3 157 | 158, 336^3 178 | 166, 352^3 208 | 182,
+// 376^3 251 | 264, 400^3 356 | 303, 512^3 617 | 566, 768^3 2087 | 1791.
+// BF16 stays with plain sweeps (400^3 65 | 284, 1024^3 1617 | 4539).
+double plain_us(const std::vector<SweepGrid>& grids) {
+  double longest = 0, points = 0;
   for (const SweepGrid& g : grids) {
-    if (g.n < kHeatMarchRows) return 0;
-    int tk, tj;
-    const double sweeps = static_cast<double>(g.nsweeps);
-    longest = std::max(longest, g.nsweeps);
-    points += sweeps * g.n * g.n * g.n;
-    planes += sweeps * heat_march_columns(g.n, kHeatMarchDepth, &tk, &tj) * (g.n - 2);
+    longest = std::max(longest, static_cast<double>(g.nsweeps));
+    points += static_cast<double>(g.nsweeps) * g.n * g.n * g.n;
   }
-  const double sweeps = static_cast<double>(longest);
-  const double part = std::ceil(planes / sweeps / compute_units());
-  const double march = sweeps * 1.25 * (5 + 2.3 * (part + 10)) / kHeatMarchDepth;
-  return march < sweeps * 3.3 + 1.42e-6 * points ? kHeatMarchDepth : 0;
+  return 3.3 * longest + 1.42e-6 * points;
+}
+
+double march_us(const std::vector<SweepGrid>& grids) {
+  double longest = 0, planes = 0;
+  for (const SweepGrid& g : grids) {
+    int tk, tj;
+    longest = std::max(longest, static_cast<double>(g.nsweeps));
+    planes += static_cast<double>(g.nsweeps) *
+              heat_march_columns(g.n, kHeatMarchDepth, &tk, &tj) * (g.n - 2);
+  }
+  if (longest == 0) return 0;
+  const double part = std::ceil(planes / longest / compute_units());
+  return longest * 1.25 * (5 + 2.3 * (part + 10)) / kHeatMarchDepth;
+}
+
+void split_heat(int dtype, const std::vector<SweepGrid>& grids, std::vector<SweepGrid>& rounds,
+                std::vector<SweepGrid>& plain) {
+  auto split = [&](auto&& in_rounds) {
+    rounds.clear();
+    plain.clear();
+    for (const SweepGrid& g : grids) (in_rounds(g) ? rounds : plain).push_back(g);
+  };
+  auto from_side = [&](int side) { split([&](const SweepGrid& g) { return g.n >= side; }); };
+  if (dtype == NPBX_F64) {
+    split([](const SweepGrid& g) {
+      return g.n >= 330 && 0.78 * static_cast<double>(cdiv(g.n, 124)) <
+                               static_cast<double>(cdiv(g.n, 128));
+    });
+    return;
+  }
+  int best = INT32_MAX;
+  if (dtype == NPBX_F32) {
+    std::vector<int> sides;
+    for (const SweepGrid& g : grids)
+      if (g.n >= kHeatMarchRows) sides.push_back(g.n);
+    std::sort(sides.begin(), sides.end());
+    sides.erase(std::unique(sides.begin(), sides.end()), sides.end());
+    double best_us = plain_us(grids);
+    for (const int side : sides) {
+      from_side(side);
+      const double us = (march_us(rounds) + plain_us(plain)) * (plain.empty() ? 1 : 1.18);
+      if (us < best_us) best_us = us, best = side;
+    }
+  }
+  from_side(best);
 }
 
 int new_queue(QueueState** q) {
@@ -1284,17 +1344,16 @@ extern "C" int npbx_plan_create(const npbx_grid_spec* specs, int32_t count, int3
   const int tmax = max_depth(dtype);
   NPBX_REQUIRE(tblock >= 2 && tblock <= tmax, "plan_create: tblock=%d outside [2, %d] for %s",
                tblock, tmax, dtype_name(dtype));
-  std::vector<GridRound> base(count);
   std::vector<SweepGrid> flat, heat;
   int64_t lups = 0;
   for (int i = 0; i < count; ++i) {
     const npbx_grid_spec& s = specs[i];
-    NPBX_TRY(check_grid("plan_create", i, s.kind, s.dtype, s.n, s.A, s.B, dtype, base[i]));
+    GridRound g;
+    NPBX_TRY(check_grid("plan_create", i, s.kind, s.dtype, s.n, s.A, s.B, dtype, g));
     NPBX_REQUIRE(s.first >= 0 && s.nsweeps >= 0, "plan_create: grid %d negative sweeps", i);
-    lups += grid_lups(base[i], s.nsweeps);
+    lups += grid_lups(g, s.nsweeps);
     if (s.nsweeps > 0)
-      (base[i].kind == kHeat3D ? heat : flat)
-          .push_back({s.A, s.B, base[i].n, s.first, s.nsweeps});
+      (g.kind == kHeat3D ? heat : flat).push_back({s.A, s.B, g.n, s.first, s.nsweeps});
   }
   const int rows = g_heat_rows.load();
   auto p = new Plan();
@@ -1311,66 +1370,65 @@ extern "C" int npbx_plan_create(const npbx_grid_spec* specs, int32_t count, int3
     p->nlaunches += static_cast<int64_t>(p->blocks.launches.size());
     for (const BlockBatch& b : p->blocks.launches) p->ntiles += b.cum[b.count];
   }
-  const int depth = heat.empty() ? 0 : heat_round_depth(dtype, heat);
-  if (depth == 0) {
-    p->sweeps = heat;
-    NPBX_TRY(built(heat_batch_sweeps(dtype, heat, false, nullptr, &p->nlaunches, &p->ntiles)));
-    *plan = p;
-    return NPBX_OK;
-  }
-  // Heat grids on tiles: launch group r runs round r of every grid that has one.
-  std::erase_if(base, [](const GridRound& g) { return g.kind != kHeat3D; });
-  count = static_cast<int32_t>(base.size());
-  std::vector<npbx_grid_spec> heat_specs;
-  for (const npbx_grid_spec* s = specs; heat_specs.size() < base.size(); ++s)
-    if (s->kind == NPBX_KIND_HEAT3D) heat_specs.push_back(*s);
-  specs = heat_specs.data();
-  std::vector<std::vector<int>> depths(count);
+  std::vector<SweepGrid> in_rounds;
+  split_heat(dtype, heat, in_rounds, p->sweeps);
+  NPBX_TRY(built(heat_batch_sweeps(dtype, p->sweeps, false, nullptr, &p->nlaunches, &p->ntiles)));
+  // Launch group r runs round r of every grid that has one.
+  const bool march = dtype == NPBX_F32;
+  const size_t grids = in_rounds.size();
+  std::vector<GridRound> next(grids);
+  std::vector<std::vector<int>> depths(grids);
   size_t nrounds = 0;
-  for (int i = 0; i < count; ++i) {
-    depths[i] = round_depths(specs[i].nsweeps, depth);
-    nrounds = std::max(nrounds, depths[i].size());
-  }
   int64_t cols_total = 0;
-  for (int i = 0; i < count; ++i) {
-    p->packs.push_back({specs[i].A, specs[i].B, base[i].n, cols_total});
-    cols_total += (cols_elems(base[i].n) + 63) / 64 * 64;  // 256-byte aligned
+  for (size_t i = 0; i < grids; ++i) {
+    const SweepGrid& s = in_rounds[i];
+    depths[i] = round_depths(s.nsweeps, march ? kHeatMarchDepth : kTileDepth);
+    nrounds = std::max(nrounds, depths[i].size());
+    GridRound& g = next[i];
+    g = GridRound{};
+    g.A = s.A;
+    g.B = s.B;
+    g.X = (s.first & 1) ? s.B : s.A;
+    g.n = s.n;
+    g.kind = kHeat3D;
+    g.parity0 = static_cast<int32_t>(s.first & 1);
+    if (march) {
+      p->packs.push_back({s.A, s.B, s.n, cols_total});
+      cols_total += (cols_elems(s.n) + 63) / 64 * 64;  // 256-byte aligned
+    } else {
+      tile_grid(g, kHeat3D, s.n, dtype, kTileDepth, kTileRows, kTileSeg);
+    }
   }
-  const hipError_t e = hipMalloc(reinterpret_cast<void**>(&p->d_cols),
-                                 static_cast<size_t>(cols_total) * sizeof(float));
-  if (e != hipSuccess) {
-    plan_free(p);
-    return fail(NPBX_ENOMEM, "plan_create: %s", hipGetErrorString(e));
-  }
-  for (int i = 0; i < count; ++i) base[i].cols = p->d_cols + p->packs[i].off;
-  std::vector<int64_t> level(count);
-  std::vector<void*> X(count);
-  for (int i = 0; i < count; ++i) {
-    level[i] = specs[i].first;
-    X[i] = (level[i] & 1) ? specs[i].B : specs[i].A;
+  if (cols_total > 0) {
+    const hipError_t e = hipMalloc(reinterpret_cast<void**>(&p->d_cols),
+                                   static_cast<size_t>(cols_total) * sizeof(float));
+    if (e != hipSuccess) {
+      plan_free(p);
+      return fail(NPBX_ENOMEM, "plan_create: %s", hipGetErrorString(e));
+    }
+    for (size_t i = 0; i < grids; ++i) next[i].cols = p->d_cols + p->packs[i].off;
   }
   for (size_t r = 0; r < nrounds; ++r) {
     bool open = false;
-    for (int i = 0; i < count; ++i) {
+    for (size_t i = 0; i < grids; ++i) {
       if (r >= depths[i].size()) continue;
       if (!open || p->launches.back().count == kMaxBatch) {
         p->launches.emplace_back();
         std::memset(&p->launches.back(), 0, sizeof(RoundBatch));
         open = true;
       }
-      GridRound g = base[i];
-      g.X = X[i];
-      g.Y = X[i] == specs[i].A ? specs[i].B : specs[i].A;
-      g.parity0 = static_cast<int32_t>(level[i] & 1);
+      GridRound& g = next[i];
+      g.Y = g.X == g.A ? g.B : g.A;
       g.depth = depths[i][r];
-      const int64_t columns = heat_march_columns(g.n, g.depth, &g.tiles_k, &g.tiles_j);
+      const int64_t columns = march ? heat_march_columns(g.n, g.depth, &g.tiles_k, &g.tiles_j)
+                                    : tiles_per_round(g);
       RoundBatch& b = p->launches.back();
-      const int64_t end = b.cum[b.count] + columns * (g.n - 2);
+      const int64_t end = b.cum[b.count] + columns * (march ? g.n - 2 : 1);
       if (end >= (int64_t(1) << 31)) return built(fail(NPBX_EINVAL, "plan_create: too many tiles"));
       b.round[b.count] = g;
       b.cum[++b.count] = static_cast<int32_t>(end);
-      X[i] = g.Y;
-      level[i] += g.depth;
+      g.X = g.Y;
+      g.parity0 ^= g.depth & 1;
       p->ntiles += columns;
     }
   }
@@ -1481,7 +1539,7 @@ extern "C" int npbx_rounds_launch(const npbx_round_spec* specs, int32_t count, i
                  "rounds_launch: grid %d must read one of A, B and write the other", i);
     NPBX_REQUIRE(s.depth >= 1 && s.depth <= tblock && s.level0 >= 0,
                  "rounds_launch: grid %d depth %d outside [1, %d]", i, s.depth, tblock);
-    tile_grid(g, g.kind, g.n, dtype, tblock, seg);
+    tile_grid(g, g.kind, g.n, dtype, tblock, g_heat_rows.load(), seg);
     if (uses_cols(g.kind, dtype, g.rows)) g.cols = s.cols;
     g.X = s.X;
     g.Y = s.Y;

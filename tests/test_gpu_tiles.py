@@ -317,6 +317,30 @@ def test_plan_forms_match_each_grid_alone(st, heat_rows, dtype, T, rows, specs, 
     plan.close()
 
 
+# Grids in rounds beside grids on plain sweeps: FP32 rounds of up to four sweeps
+# (9 sweeps: 4, 4, 1) beside grids too small for them, FP64 rounds of two
+# (5 sweeps: 2, 2, 1) beside one whose tiles' columns would stay a quarter empty
+@pytest.mark.parametrize("dtype,specs,launches", [
+    ("f32", [("heat_3d", 32, 5, 0), ("heat_3d", 256, 9, 1), ("heat_3d", 256, 9, 0),
+             ("heat_3d", 24, 4, 1)], 3 + 5),
+    ("f64", [("heat_3d", 336, 5, 1), ("heat_3d", 40, 3, 0)], 3 + 3),
+    ("f64", [("heat_3d", 376, 3, 0)], 3),
+])
+@pytest.mark.parametrize("same_boundary", [False, True])
+def test_plan_chooses_per_heat_grid(st, dtype, specs, launches, same_boundary):
+    """A small grid leaves the large ones of its plan their rounds."""
+    from npbench_amd import batch
+    gs, alone = _device_batch(dtype, specs, same_boundary)
+    print(f"plan per grid {dtype} grids={len(specs)} {same_boundary}", flush=True)
+    plan = batch.Plan(gs, tblock=2)
+    assert plan.info()["launches"] == launches
+    plan.launch()
+    for g, (a, b), (kind, n, ns, first) in zip(gs, alone, specs):
+        st.heat3d_sweeps(a, b, ns, first=first)
+        assert torch.equal(g.A, a) and torch.equal(g.B, b), f"n={n} first={first}"
+    plan.close()
+
+
 def test_pack_cols_layout(st):
     """npbx_pack_cols: cols[a][q][j][s] = (A, B)[a][q][j][(0, n-1)[s]], then
     one word that is 1 exactly when A's and B's boundaries are equal (each
