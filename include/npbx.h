@@ -234,7 +234,7 @@ int npbx_pack_cols(int dtype, const void *A, const void *B, int64_t n,
  * registers, d' in LDS, 80 < K <= 160; 4: loads coalesced and staged in
  * LDS, c' and d' in registers, 80 < K <= 160 with whole 64-byte chunks of
  * levels -- the default where it applies), "hdiff.shape" = hdiff marching
- * shape (0, the default: by storage type; 1 .. 13: columns per lane, rows
+ * shape (0, the default: by type and size; 1 .. 13: columns per lane, rows
  * per thread, bytes of k per lane),
  * "seidel.blocks" = tiles (64 rows of a
  * group of 4 sweeps) per seidel_2d launch (default 2048; at most 4096 take

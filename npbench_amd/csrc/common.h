@@ -145,7 +145,7 @@ int sweep_shape();
 // Fused hdiff steps per round ("hdiff.tblock"; 1 = one launch per step).
 int hdiff_tblock();
 void set_hdiff_tblock(int tb);
-// hdiff marching shape ("hdiff.shape"; 0 = by storage type, 1 .. 13 =
+// hdiff marching shape ("hdiff.shape"; 0 = by type and size, 1 .. 13 =
 // {columns per lane, rows per thread, bytes of k per lane}, hdiff.hip).
 int hdiff_shape();
 void set_hdiff_shape(int shape);

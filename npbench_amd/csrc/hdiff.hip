@@ -144,13 +144,17 @@ __global__ __launch_bounds__(256) void hdiff_copy_halo(const S* __restrict__ src
 // group is shifted left to end at column J-1 (J >= W) and stores only its
 // own columns, so every column is stored once and every load is in the
 // field.  Prefetched vectors are held as raw storage words until the row
-// that uses them.  The output is stored around the caches' allocation: kept
-// lines of it would push out the inputs that later rows and calls read (FP32
-// 256 x 256 x 160 with three operand sets in turn 29.9 -> 20.4 us, FP64 57.6
-// -> 54.8; with one set, cached inputs, FP32 20.6 -> 20.4, FP64 40.0 -> 38.5).
+// that uses them.  STREAM: the output is stored around the caches'
+// allocation, since kept lines of it would push out the inputs that later rows
+// and calls read (FP32 256 x 256 x 160 with three operand sets in turn 29.9 ->
+// 20.4 us, FP64 57.6 -> 54.8; with one set, cached inputs, FP32 20.6 -> 20.4,
+// FP64 40.0 -> 38.5).  A store writes pieces as long as a column's k, W columns
+// apart; where those are short and end inside lines, nothing gathers them into
+// lines, and the caches keep the output (FP64 1414 x 1414 x 4, one set: 2 x 6 x
+// 8 B 46.2 us streamed, 34.5 kept).
 // TAIL: a column's last vector is shifted back to end with it (what two lanes
 // store there is the same) and addresses are aligned to elements only.
-template <class S, int W, int STRIP, int VB, bool TAIL = false>
+template <class S, int W, int STRIP, int VB, bool STREAM = true, bool TAIL = false>
 __global__ __launch_bounds__(256) void hdiff_march(const S* __restrict__ in, S* __restrict__ out,
                                                    const S* __restrict__ coeff, int I, int J,
                                                    int K, int xblocks, S* __restrict__ halo_dst) {
@@ -323,7 +327,13 @@ __global__ __launch_bounds__(256) void hdiff_march(const S* __restrict__ in, S* 
         else
           storev<S, V>(to, res[w]);
       } else {
-        storev_stream<S, V, TAIL>(out + (static_cast<int64_t>(x) * J + y0 + w) * K + k0, res[w]);
+        S* to = out + (static_cast<int64_t>(x) * J + y0 + w) * K + k0;
+        if constexpr (STREAM)
+          storev_stream<S, V, TAIL>(to, res[w]);
+        else if constexpr (TAIL)
+          storev_any<S, V>(to, res[w]);
+        else
+          storev<S, V>(to, res[w]);
       }
     }
   };
@@ -354,34 +364,77 @@ constexpr MarchShape kMarchShapes[] = {{0, 0, 0},   {1, 12, 16}, {1, 6, 16}, {2,
 constexpr int kMarchShapeCount = 14;  // of the knob
 std::atomic<int> g_hdiff_shape{0};
 
-// The shapes a call tries in turn; the first that fits runs: no wider than J,
-// columns of k whole vectors, arrays aligned to them.  The first of each type
-// is the fastest of 22 shapes on the MI355X over calls whose operands change
-// (three sets in turn; us, streaming stores): 256 x 256 x 160 FP64 4 x 4 x 8 B
-// 50.2 (2 x 6 x 8: 54.8, 4 x 6 x 8: 51.2), FP32 2 x 6 x 8 20.4 (4 x 4 x 8:
-// 21.5, 4 x 6 x 4: 27.0), BF16 4 x 6 x 4 14.8 (2 x 6 x 8: 15.0).  An odd K
-// leaves FP32 the 4-byte vectors (190 x 203 x 137: 13.4; a point per thread
-// 28.8) and BF16 the tail form of its own.
-// Small calls leave a march too few waves, each a chain of row loads: up to
-// kPoint points run a point per thread, and FP64 and FP32 up to
-// some millions one column x 6 rows of 16-byte vectors where these fit (us, a
-// call among others, point | 1 x 6 x 16 | the order above):
-//   FP64   60 x 60 x 40 3.7 | 4.2 | 5.5    104 x 100 x 98 11.7 | 7.3 | 9.0
-//         237 x 238 x 40 26 | 10.2 | 12.2  190 x 203 x 101 48 | - | 22.5
-//   FP32   60 x 60 x 40 2.3 | 4.6 | 5.4    147 x 126 x 64  5.4 | 5.8 | 6.1
-//         160 x 160 x 80 9.6 | 7.0 | 7.8   256 x 256 x 96  28 | 14.7 | 15.2
-//   BF16  103 x 78 x 55  3.1 | 7.9 | 7.9   147 x 126 x 64  5.0 | 6.9 | 7.5
-//         130 x 130 x 90 8.0 | 8.0 | 8.1   160 x 160 x 80  9.8 | 7.6 | 8.1
-template <class S>
-constexpr int march_order(int n, int64_t points) {
-  constexpr int f64[] = {14, 7, 1}, f32[] = {7, 9, 12, 1}, b16[] = {9, 12, 1};
-  constexpr int f64_mid[] = {2, 7, 1}, f32_mid[] = {2, 7, 9, 12, 1};
-  constexpr int64_t kPoint = sizeof(S) == 8 ? 250000 : sizeof(S) == 4 ? 900000 : 1250000;
-  if (points < kPoint) return 0;
-  if (sizeof(S) == 8) return n >= 3 ? 0 : points < 3200000 ? f64_mid[n] : f64[n];
-  if (sizeof(S) == 4)
-    return points < 5000000 ? (n < 5 ? f32_mid[n] : 0) : n < 4 ? f32[n] : 0;
-  return n < 3 ? b16[n] : 0;
+// How a call runs: a marching shape (0: a point per thread), whether its output
+// is streamed (shapes 7, 9 and 12 also run without), and whether a column's last
+// vector is shifted back (TAIL).
+struct March {
+  int shape;
+  bool streamed, tail;
+};
+
+// Whether columns of `bytes` fill whole lines, or so many that the two at their
+// ends do not matter.
+constexpr bool whole_lines(int64_t bytes) { return bytes % 64 == 0 || bytes >= 384; }
+
+// The default, from 1200 measured (shape, stores, size) times on the MI355X, one
+// operand set and three in turn; fits(shape): no wider than J, columns of k whole
+// vectors, arrays aligned to them.
+//
+// A point per thread takes a workgroup for 64 levels of four columns, so its time
+// goes with these (2.3 us and 2 (FP64) or 0.5 ns each, and the arithmetic): it is
+// the shortest while they are few, and an order of magnitude longer where short
+// columns leave their lanes idle.  us, point | march:
+//   FP64   61 x 61 x 32   3.8 | 4.5   122 x 122 x 16  8.7 | 4.5   489 x 489 x 1  98 | 5.0
+//   FP32  100 x 100 x 24  3.4 | 4.9   223 x 223 x 12  9.2 | 5.2   663 x 663 x 2  59 | 5.7
+//   BF16  136 x 136 x 64  5.6 | 7.2   223 x 223 x 24  9.7 | 7.1   612 x 612 x 4  54 | 7.3
+// Else a column x 6 rows of 16-byte vectors (shape 2), whose stores of adjacent
+// columns are one run whatever K is, while the call is short of waves or its
+// columns short; else two or four columns, which load the side columns less
+// often.  us, three sets in turn | one:
+//                          shape 2       2 x 6 x 8 B    4 x 4 x 8 B
+//   FP64 707 x 707 x 16   45.6 | 29.8    43.0 | 30.9    42.1 | 31.8
+//        1322 x 1322 x 2  16.8 | 16.4    24.7 | 24.4    43.9 | 43.8
+//        256 x 256 x 64   17.6 | 17.8    17.9 | 17.9    17.9 | 17.8
+//        270 x 270 x 48   15.4 | 15.2    15.5 | 15.5    16.3 | 16.2
+//        256 x 256 x 160  62.8 | 39.1    54.7 | 38.9    50.7 | 38.8
+//   FP32 200 x 200 x 100  10.2 |  9.0    11.0 |  9.9    10.8 |  9.9
+//        816 x 816 x 12   17.7 | 17.6    26.8 | 26.8    32.4 | 32.5
+//        256 x 256 x 160  26.2 | 21.1    26.4 | 20.9    26.0 | 22.1
+// FP64 columns that end inside lines: 2 x 6 x 8 B kept (1000 x 1000 x 3 14.9,
+// streamed 20.0).  FP32 with odd K has 4-byte vectors only (190 x 203 x 137, 4 x 6
+// streamed 14.6, kept 14.0; a point per thread 29.3).  BF16 4 x 6 x 4 B 15.2 at 256 x 256 x 160
+// (2 x 6 x 8 B 15.4), with columns of K = 8 m that end inside lines shape 2
+// (1000 x 1000 x 8 13.1; 4 x 6 x 4 B 25.7 streamed, 13.8 kept), of K = 4 m 2 x 6 x
+// 8 B kept; odd K the tail form (190 x 203 x 137 10.6; a point per thread 21.9).
+template <class S, class Fits>
+March default_march(int I, int J, int K, Fits&& fits) {
+  const int64_t points = int64_t(I) * J * K, bytes = int64_t(K) * sizeof(S);
+  const int64_t groups = cdiv(K, kLanes) * cdiv(J, kCols) * I;
+  const bool whole = whole_lines(bytes);
+  const March point{0, false, false}, one_column{1, true, false};
+  if constexpr (sizeof(S) == 8) {
+    if (groups <= 1200) return point;
+    const bool large = points >= (K % 2 ? 9000000 : 5500000);
+    if (large && (bytes >= 256 ? whole : bytes % 64 == 0 && bytes >= 128) && fits(14))
+      return {14, true, false};
+    if (fits(2) && (points < 3200000 || bytes < 256)) return {2, true, false};
+    if (fits(7)) return {7, whole, false};
+  } else if constexpr (sizeof(S) == 4) {
+    if (groups <= (fits(2) ? 4000 : 6000) && points <= (fits(2) ? 650000 : 900000)) return point;
+    if (fits(2) && (points < 5000000 || bytes < 256)) return {2, true, false};
+    if (fits(7)) return {7, bytes >= 200, false};
+    if (bytes >= 200 && fits(9)) return {9, false, false};
+    if (fits(12)) return {12, false, false};
+  } else {
+    if (groups <= (K % 2 ? 12000 : 8000) && points <= 1250000) return point;
+    const bool stream = bytes % 64 == 0 || bytes >= 96;
+    if (!stream && fits(2)) return {2, true, false};
+    if (!stream && fits(7)) return {7, false, false};
+    if (fits(9)) return {9, stream, false};
+    if (fits(12)) return {12, stream, false};
+    if (J >= kMarchShapes[9].w && K >= 2 && !fits(1)) return {9, bytes >= 96, true};
+  }
+  return fits(1) ? one_column : point;
 }
 
 // ---------------------------------------------------------------- fused steps
@@ -814,17 +867,12 @@ int run_hdiff(const S* in, S* out, const S* coeff, int I, int J, int K, int64_t 
     return m.w <= J && m.vb >= int(sizeof(S)) && K * int64_t(sizeof(S)) % m.vb == 0 &&
            aligned_to(m.vb);
   };
-  const int64_t points = int64_t(I) * J * K;
-  int shape = g_hdiff_shape.load();
-  if (shape <= 0 || shape >= kMarchShapeCount || !fits(shape)) {
-    int n = 0;
-    do shape = march_order<S>(n++, points);
-    while (shape && !fits(shape));
-  }
-  // BF16 columns that no 4-byte vector divides: the last vector of a column is
-  // shifted back to end with it, and addresses are aligned to elements only.
-  const bool tail = sizeof(S) == 2 && !shape && J >= 4 && K >= 2 && points >= 1250000;
-  if (tail) shape = 9;
+  const int knob = g_hdiff_shape.load();
+  const March march =
+      knob > 0 && knob < kMarchShapeCount && fits(knob)
+          ? March{knob, true, false}
+          : default_march<S>(I, J, K, fits);
+  const int shape = march.shape;
   const bool vec = shape != 0;
   const bool aligned = aligned_to(16);
   const int W = vec ? kMarchShapes[shape].w : 1, strip = vec ? kMarchShapes[shape].strip : 1;
@@ -843,11 +891,23 @@ int run_hdiff(const S* in, S* out, const S* coeff, int I, int J, int K, int64_t 
       };
       constexpr int b4 = sizeof(S) <= 4 ? 4 : 8;  // FP64 has no 4-byte vector
       if constexpr (sizeof(S) == 2) {
-        if (tail) {
-          go(hdiff_march<S, 4, 6, 4, true>);
+        if (march.tail) {
+          if (march.streamed)
+            go(hdiff_march<S, 4, 6, 4, true, true>);
+          else
+            go(hdiff_march<S, 4, 6, 4, false, true>);
           NPBX_LAUNCHED("hdiff_march");
           return NPBX_OK;
         }
+      }
+      if (!march.streamed) {
+        switch (shape) {
+          case 7: go(hdiff_march<S, 2, 6, 8, false>); break;
+          case 9: go(hdiff_march<S, 4, 6, b4, false>); break;
+          default: go(hdiff_march<S, 2, 12, b4, false>); break;
+        }
+        NPBX_LAUNCHED("hdiff_march");
+        return NPBX_OK;
       }
       switch (shape) {
         case 1: go(hdiff_march<S, 1, 12, 16>); break;

@@ -316,6 +316,30 @@ def _unaligned(a, dt):
     return v
 
 
+# short columns, whose output the caches keep: every vector width of every type
+@pytest.mark.parametrize("precision,I,J,K", [
+    ("fp64", 110, 109, 16), ("fp64", 200, 201, 3), ("fp64", 1000, 70, 1),
+    ("fp32", 251, 250, 12), ("fp32", 250, 251, 6), ("fp32", 250, 251, 5), ("fp32", 210, 213, 67),
+    ("bf16", 301, 302, 8), ("bf16", 301, 302, 12), ("bf16", 300, 303, 6), ("bf16", 400, 401, 7)])
+@pytest.mark.parametrize("nsteps", [1, 2])
+def test_hdiff_short_columns(st, hdiff_shape, precision, I, J, K, nsteps):
+    """Bitwise one march shape (a column x 6 rows) on columns padded to whole
+    16-byte vectors."""
+    dt = {"fp64": torch.float64, "fp32": torch.float32, "bf16": torch.bfloat16}[precision]
+    inf, out, coeff = _hdiff_inputs(I, J, K, 5 * I + J + K)
+    pad = lambda a: np.concatenate([a, np.zeros(a.shape[:2] + (-K % 8,))], axis=2)  # noqa: E731
+    hdiff_shape(2)
+    want = dev(pad(out), dt)
+    st.hdiff(dev(pad(inf), dt), want, dev(pad(coeff), dt), nsteps=nsteps)
+    hdiff_shape(0)
+    got = dev(out, dt)
+    print(f"hdiff short columns {precision} {I}x{J}x{K} nsteps={nsteps}", flush=True)
+    st.hdiff(dev(inf, dt), got, dev(coeff, dt), nsteps=nsteps)
+    torch.cuda.synchronize()
+    assert torch.equal(got.contiguous().view(torch.uint8),
+                       want[:, :, :K].contiguous().view(torch.uint8))
+
+
 # both sides of the point counts where the default shape changes (250,000,
 # 900,000, 1,250,000, 3,200,000 and 5,000,000), K odd, even and whole vectors
 @pytest.mark.parametrize("precision", ["fp64", "fp32", "bf16"])

@@ -1,0 +1,51 @@
+"""Calls of neighbouring sizes cost alike: no launch shape is chosen where it is
+many times slower than one that the call could take.  Each pair does the same
+work, and the bounds leave room for several times the spread of such timings."""
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+DT = {"f64": torch.float64, "f32": torch.float32, "bf16": torch.bfloat16}
+
+
+@pytest.fixture(scope="module")
+def st():
+    from npbench_amd import device, stencils
+    device.require_device()
+    return stencils
+
+
+def fastest(call, reps=20, rounds=5):
+    """us a call, the best of several rounds of calls."""
+    call()
+    torch.cuda.synchronize()
+    start, stop = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    best = float("inf")
+    for _ in range(rounds):
+        start.record()
+        for _ in range(reps):
+            call()
+        stop.record()
+        torch.cuda.synchronize()
+        best = min(best, start.elapsed_time(stop) / reps * 1e3)
+    return best
+
+
+def compare(what, call, like, bound):
+    a, b = fastest(call), fastest(like)
+    print(f"{what}: {a:.1f} us, like {b:.1f} us", flush=True)
+    assert a < bound * b
+
+
+@pytest.mark.parametrize("dtype,shape,like", [
+    ("f64", (489, 489, 1), (122, 122, 16)), ("f64", (1732, 1732, 2), (433, 433, 32)),
+    ("f32", (663, 663, 2), (166, 166, 32)), ("bf16", (500, 500, 4), (125, 125, 64))])
+def test_hdiff_short_columns_cost_as_long_ones(st, dtype, shape, like):
+    def call(I, J, K):
+        gen = torch.Generator(device="cuda").manual_seed(I + K)
+        f = [torch.rand(s, generator=gen, device="cuda").to(DT[dtype])
+             for s in ((I + 4, J + 4, K), (I, J, K), (I, J, K))]
+        return lambda: st.hdiff(*f)
+    compare(f"hdiff {dtype} {shape} {like}", call(*shape), call(*like), 2)
