@@ -30,8 +30,8 @@ constexpr int kLanes = 64;
 constexpr int kCols = 4;
 constexpr int kRows = 16;
 
-// One point a lane, 16 planes, the grid's own block order: the best BF16 form
-// for sides of 129 to 192 (run_sweeps).
+// One point a lane, 16 planes, the grid's own block order: BF16 sides of 129 to
+// 194 and sides whose rows leave much of the last vectors empty (run_sweeps).
 template <class S>
 __global__ __launch_bounds__(kLanes* kCols) void heat3d_sweep(const S* __restrict__ src,
                                                              S* __restrict__ dst, int n) {
@@ -121,10 +121,10 @@ __device__ __forceinline__ void sweep_tile(const S* __restrict__ src, S* __restr
       }
       S* o = dst + col + static_cast<int64_t>(i + u) * plane;
       if (full) {
-        S raw[V];
-#pragma unroll
-        for (int v = 0; v < V; ++v) raw[v] = T::store(out[v]);
-        __builtin_memcpy(o, raw, sizeof(raw));
+        if constexpr (V == 1)
+          *o = T::store(out[0]);
+        else  // (BF16: two conversions an instruction; 512^3 204 -> 177 us a sweep)
+          storev_any<S, V>(o, out);
       } else {
 #pragma unroll
         for (int v = 0; v < V; ++v)
@@ -208,7 +208,7 @@ __global__ __launch_bounds__(kLanes* kCols) void heat3d_sweep_batch(const HeatBa
 // A batch's grids take the forms that a single grid of as many points takes
 // (run_sweeps); BF16's follow the row length, which its vectors have to fill.
 int batch_form(int dtype, int n, int64_t points) {
-  if (dtype == NPBX_BF16) return n <= 128 ? 0 : n <= 280 ? 1 : 2;
+  if (dtype == NPBX_BF16) return n <= 128 ? 0 : n <= 256 ? 1 : 2;
   const int64_t lo = dtype == NPBX_F64 ? 112 : 56, hi = dtype == NPBX_F64 ? 176 : 112;
   return points <= lo * lo * lo ? 0 : points <= hi * hi * hi ? 1 : 2;
 }
@@ -318,19 +318,26 @@ int run_points(S* A, S* B, int n, int64_t first, int64_t nsweeps, hipStream_t st
 // 128^3 on it saves loads of planes i-1 and i.  Narrow vectors fill a wave's
 // lanes on short rows, and FP32 keeps them: with one point a lane a row's
 // accesses are whole lines and the k-edge scalars hit the same ones.
+// Past the Infinity Cache a sweep's time goes with the waves a row takes, whether
+// or not points fill them, so there the count decides between vectors and single
+// points: FP64 385^3 takes four waves of vectors or six of points, 348 | 283 us;
+// FP32 keeps points but where rows are whole multiples of 256, whose planes then
+// fall on few channels (512^3 350 | 4x8/4 314).
 // Measured, us per sweep, V points a lane x planes / ahead:
-//   FP64       2x1/1  2x2/2  2x4/4  2x8/4  2x16/4     BF16  2x1/1  2x2/2  4x2/2  8x4/2  1x16
-//     64^3       3.7    3.7    3.7    4.9    7.6       64^3   3.5    3.5    4.0    7.0    5.2
-//     101^3      6.3    6.1    6.3    7.1    8.4      101^3   5.0    4.8    5.5    7.5    7.1
-//     160^3     18.3   17.4   16.8   17.5   19.6      177^3  16.3   13.7   12.1   13.9   10.6
-//     201^3     29.1   27.6   25.8   25.7   29.8      201^3  20.3   17.9   15.3   17.5   16.2
-//     512^3      723    678    626    615    622      512^3   329    268    200    176    234
-//   FP32       2x1/1  1x4/4  1x8/4  4x4/4  4x16/4
-//     64^3       3.5    3.2    3.8    3.9    8.5
-//     101^3      5.2    4.7    5.1    5.5    8.5
-//     201^3     20.9   18.4   14.8   15.6   18.2
+//   FP64       2x1/1  2x2/2  2x4/4  2x8/4  2x16/4   1x16    BF16  2x2/2  4x2/2  8x4/2  8x8/4  1x16
+//     64^3       3.7    3.7    3.7    4.9    7.6             64^3   3.5    4.0    7.0
+//     101^3      6.3    6.1    6.3    7.1    8.4            101^3   4.8    5.5    7.5            7.1
+//     160^3     18.3   17.4   16.8   17.5   19.6   19.8     176^3          11.3                 10.9
+//     201^3     29.1   27.6   25.8   25.7   29.8            200^3          13.0                 16.7
+//     385^3                           348           283     258^3          34.7   23.1   26     26.6
+//     400^3                           358           344     400^3                 54.0   57     88
+//     512^3      723    678    626    612    626    669     512^3                  176   176    237
+//   FP32       2x1/1  1x4/4  1x8/4  4x4/4  4x16/4           513^3                  330          199
+//     64^3       3.5    3.2    3.8    3.9    8.5           1024^3                 1393  1289   2122
+//     101^3      5.2    4.7    5.1    5.5    8.5    (4x8/4 512^3 .. 768^3: 513^3 247, 700^3 500,
+//     201^3     20.9   18.4   14.8   15.6   18.2    1x16 562)
 //     256^3     32.0   27.5   22.2   24.7   25.7
-//     512^3      384    289    284    317    314
+//     384^3             125    123    137    139
 template <class S>
 int run_sweeps(S* A, S* B, int n, int64_t first, int64_t nsweeps, hipStream_t stream) {
   constexpr int N = Vec16<S>::N;
@@ -342,6 +349,7 @@ int run_sweeps(S* A, S* B, int n, int64_t first, int64_t nsweeps, hipStream_t st
       default: break;
     }
   }
+  const auto waves = [n](int v) { return k_tiles(n, v); };  // a row's
   if (n <= 88) return run_vec<S, 2, 1, 1>(A, B, n, first, nsweeps, stream);
   if constexpr (std::is_same_v<S, double>) {
     if (n <= 112) return run_vec<S, 2, 2, 2>(A, B, n, first, nsweeps, stream);
@@ -349,15 +357,24 @@ int run_sweeps(S* A, S* B, int n, int64_t first, int64_t nsweeps, hipStream_t st
     // 129^3 9.7 us (vectors of two 11.4, 16 planes a thread 10.6), 177^3 20.3 | 20.7
     if (n <= 128) return run_vec<S, 2, 4, 4>(A, B, n, first, nsweeps, stream);
     if (n <= 194) return run_vec<S, 1, 4, 4>(A, B, n, first, nsweeps, stream);
+    if (n >= 330 && 3.2 * waves(1) < 5.7 * waves(2))
+      return run_points<S>(A, B, n, first, nsweeps, stream);
     return run_vec<S, 2, 8, 4>(A, B, n, first, nsweeps, stream);
   } else if constexpr (std::is_same_v<S, float>) {
     if (n <= 112) return run_vec<S, 1, 4, 4>(A, B, n, first, nsweeps, stream);
+    if (n >= 512 && n % 256 == 0) return run_vec<S, 4, 8, 4>(A, B, n, first, nsweeps, stream);
     return run_vec<S, 1, 8, 4>(A, B, n, first, nsweeps, stream);
   } else {
     if (n <= 128) return run_vec<S, 2, 2, 2>(A, B, n, first, nsweeps, stream);
-    if (n <= 192) return run_points<S>(A, B, n, first, nsweeps, stream);
-    if (n <= 280) return run_vec<S, 4, 2, 2>(A, B, n, first, nsweeps, stream);
-    return run_vec<S, 8, 4, 2>(A, B, n, first, nsweeps, stream);
+    if (n <= 194) return run_points<S>(A, B, n, first, nsweeps, stream);
+    if (n <= 256) return run_vec<S, 4, 2, 2>(A, B, n, first, nsweeps, stream);
+    if (n <= 448) return run_vec<S, 8, 4, 2>(A, B, n, first, nsweeps, stream);
+    // odd rows put vectors across lines
+    const double v8 = (n % 2 ? 7.3 : 6.5) * waves(8), v4 = (n % 2 ? 3.6 : 3.35) * waves(4);
+    const double v1 = 1.03 * waves(1);
+    if (v1 < std::min(v4, v8)) return run_points<S>(A, B, n, first, nsweeps, stream);
+    if (v4 < v8) return run_vec<S, 4, 8, 4>(A, B, n, first, nsweeps, stream);
+    return run_vec<S, 8, 8, 4>(A, B, n, first, nsweeps, stream);
   }
 }
 

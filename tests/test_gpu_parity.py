@@ -275,6 +275,31 @@ def test_hdiff_two_step_strips(st, hdiff_tblock, precision, rows, I, J, K):
         _native.set_tuning("hdiff.fuse_rows", old)
 
 
+# where rows leave the last vectors empty, and multiples of 256
+@pytest.mark.parametrize("dtype,n,off", [
+    (torch.float64, 385, 1), (torch.float64, 400, 0), (torch.float32, 512, 1),
+    (torch.bfloat16, 258, 1), (torch.bfloat16, 449, 0), (torch.bfloat16, 513, 1),
+    (torch.bfloat16, 700, 1), (torch.bfloat16, 800, 0)])
+def test_heat3d_sweep_shapes_of_large_grids_bitwise(st, dtype, n, off):
+    """Bitwise the sweep of one launch shape (16-byte vectors, 8 planes)."""
+    from npbench_amd import _native
+    print(f"heat3d large shapes {dtype} n={n} off={off}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    A, B, a, b = (torch.full((n ** 3 + 2,), 0.5, dtype=dtype, device="cuda") for _ in range(4))
+    for x, y in ((A, a), (B, b)):
+        x[off:off + n ** 3] = torch.rand(n ** 3, generator=gen, device="cuda").to(dtype)
+        y.copy_(x)
+    views = [x[off:off + n ** 3].view(n, n, n) for x in (A, B, a, b)]
+    st.heat3d_sweeps(views[0], views[1], 2)
+    _native.set_tuning("sweep.shape", 3)
+    try:
+        st.heat3d_sweeps(views[2], views[3], 2)
+    finally:
+        _native.set_tuning("sweep.shape", 0)
+    torch.cuda.synchronize()
+    assert torch.equal(A, a) and torch.equal(B, b)
+
+
 @pytest.mark.parametrize("precision", ["fp64", "fp32", "bf16"])
 @pytest.mark.parametrize("I,J,K", [(3, 1, 5), (4, 2, 3), (6, 3, 7), (5, 4, 2), (7, 5, 1),
                                    (9, 6, 41), (13, 33, 22), (6, 70, 137)])

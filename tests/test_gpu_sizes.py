@@ -49,3 +49,16 @@ def test_hdiff_short_columns_cost_as_long_ones(st, dtype, shape, like):
              for s in ((I + 4, J + 4, K), (I, J, K), (I, J, K))]
         return lambda: st.hdiff(*f)
     compare(f"hdiff {dtype} {shape} {like}", call(*shape), call(*like), 2)
+
+
+@pytest.mark.parametrize("dtype,n,like", [("bf16", 264, 256), ("bf16", 513, 512),
+                                          ("f64", 385, 384)])
+def test_heat3d_side_just_past_a_vectors_multiple(st, dtype, n, like):
+    def call(n):
+        gen = torch.Generator(device="cuda").manual_seed(n)
+        a = torch.rand((n,) * 3, generator=gen, device="cuda").to(DT[dtype])
+        b = a.clone()
+        return lambda: st.heat3d_sweeps(a, b, 8)
+    a, b = fastest(call(n), 2), fastest(call(like), 2)
+    print(f"heat3d {dtype} {n}^3 {a:.1f} us, {like}^3 {b:.1f} us", flush=True)
+    assert a < 1.3 * (n / like) ** 3 * b
