@@ -41,7 +41,7 @@ namespace npbx {
 namespace {
 
 constexpr int kThreadsC = 1024;
-constexpr int kLdsPoints = 1024;  // most points of the one-workgroup form
+constexpr int kLdsPoints = 10240;  // two FP64 pressure buffers: all 160 KiB of LDS
 
 // The reference's scalar expressions, computed on the host as Python computes
 // them (x**2 is the C library's pow, which CPython's float power calls).
@@ -489,8 +489,8 @@ __global__ __launch_bounds__(1024) void cavity_velocity(CavityArgs g, const doub
   }
 }
 
-// Grids of up to kLdsPoints points: both pressure buffers live in LDS for the
-// whole run, each thread keeps its (at most kMaxPts) interior points' indices,
+// Grids of up to kLdsPoints points, kMaxPts interior points a thread: both
+// pressure buffers live in LDS for the whole run, each thread keeps its (at most kMaxPts) interior points' indices,
 // edge flags and b values in registers -- it computes b for the same points
 // it then iterates -- so a pressure iteration touches LDS only.
 __global__ __launch_bounds__(kThreadsC) void cavity_flow_lds(CavityArgs g) {
@@ -678,11 +678,25 @@ int blocked_flow(const CavityArgs& a, hipStream_t stream) {
   return NPBX_OK;
 }
 
-// The one-workgroup form while the grid is at most a point per thread: a
-// phase then costs about 1 us.  50 steps of 5 / 20 iterations on the MI355X:
-// 25 x 25 402 / 1049 us against 499 / 1020 in blocks, 33 x 33 551 / 1354
-// against 527 / 1062, 61 x 61 955 / 2235 against 532 / 1064.
-bool use_lds(int64_t nx, int64_t ny) { return nx * ny <= kLdsPoints; }
+// The one-workgroup form where an iteration costs less than its share of the
+// blocked form's launches: up to some 1500 interior points, and up to two a
+// thread where there are few iterations.  us a step, one workgroup | blocks:
+//   iterations        1            4 or 5        10          20          50
+//   20 x 20       3.2 |  9.7    4.8 | 10.8   6.7 | 12.7  10.7 | 20.9  22.4 | 46.9
+//   33 x 33       6.3 | 10.6    8.6 | 11.2  11.5 | 13.4  17.2 | 21.6  34.4 | 48.5
+//   40 x 40       6.7 | 10.0    9.5 | 11.5  13.2 | 13.1  20.3 | 21.9  41.9 | 48.7
+//   45 x 45       7.2 | 10.3   10.9 | 11.5  15.7 | 13.3  25.1 | 22.0  53.3 | 49.3
+//   400 wide, 3   4.3 |  8.7    5.9 | 10.0   7.9 | 12.2  11.8 | 20.5  23.6 | 47.6
+//   2000 wide, 3 10.2 |  9.1   14.0 | 10.3  18.7 | 12.4  28.2 | 20.8  56.5 | 47.7
+// Without iterations (velocities only) 400 x 3 takes 3.8 | 4.7, 32 x 32 5.5 | 5.3
+// and 1000 x 3 7.0 | 4.6.
+bool use_lds(int64_t nx, int64_t ny, int64_t nit) {
+  const int64_t points = nx * ny, interior = (nx - 2) * (ny - 2);
+  if (points <= 1024) return true;
+  if (points > kLdsPoints || interior > int64_t(kMaxPts) * kThreadsC) return false;
+  if (nit == 0) return interior <= 600;
+  return interior <= 1500 || (nit <= 4 && points <= 4000);
+}
 
 }  // namespace
 }  // namespace npbx
@@ -734,7 +748,7 @@ extern "C" int npbx_cavity_flow(int dtype, int64_t nx, int64_t ny, int64_t nt, i
   g.cpv = dt / (2.0 * rho * dy);
   g.cdx2 = dt / g.dx2;
   g.cdy2 = dt / g.dy2;
-  if (!use_lds(nx, ny)) return blocked_flow(g, as_stream(stream));
+  if (!use_lds(nx, ny, nit)) return blocked_flow(g, as_stream(stream));
   // A time step depends on u, v and p only (b, un, vn are rebuilt each step),
   // so the steps split into launches of about 50 ms of work each: no launch
   // runs for long, whatever nt is.

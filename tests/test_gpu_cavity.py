@@ -96,6 +96,17 @@ def test_cavity_blocked_bitwise(st, ny, nx, nt, nit):
     check(st, nx, ny, nt, nit, u, v, p, 1.3, 0.07, f"blocked {ny}x{nx} nt={nt} nit={nit}")
 
 
+@pytest.mark.parametrize("ny,nx", [(3, 1000), (1000, 3), (3, 2100), (2100, 3), (33, 32), (40, 41),
+                                   (46, 46)])
+@pytest.mark.parametrize("nt,nit", [(3, 0), (2, 1), (1, 4), (2, 5), (1, 25)])
+def test_cavity_forms_bitwise(st, ny, nx, nt, nit):
+    """Both sides of the choice between one workgroup and blocks, by points and
+    by iterations, and grids a row or column of interior points wide on each."""
+    rng = np.random.default_rng(ny * 1000 + nx * 10 + nit)
+    u, v, p = rng.random((ny, nx)), rng.random((ny, nx)) - 0.5, rng.random((ny, nx))
+    check(st, nx, ny, nt, nit, u, v, p, 1.3, 0.07, f"forms {ny}x{nx} nt={nt} nit={nit}")
+
+
 @pytest.mark.parametrize("case", ["rest", "tiny", "huge", "nan"])
 def test_cavity_blocked_division_range(st, case):
     """Exact zeros take the short division; values past its range (a

@@ -62,3 +62,14 @@ def test_heat3d_side_just_past_a_vectors_multiple(st, dtype, n, like):
     a, b = fastest(call(n), 2), fastest(call(like), 2)
     print(f"heat3d {dtype} {n}^3 {a:.1f} us, {like}^3 {b:.1f} us", flush=True)
     assert a < 1.3 * (n / like) ** 3 * b
+
+
+@pytest.mark.parametrize("nx,ny,nit", [(3, 400, 1), (400, 3, 1), (33, 33, 20)])
+def test_cavity_flow_small_grids_cost_as_a_square_one(st, nx, ny, nit):
+    def call(nx, ny):
+        u, v, p = (torch.full((ny, nx), 0.01, dtype=torch.float64, device="cuda")
+                   for _ in range(3))
+        return lambda: st.cavity_flow(nx, ny, 50, nit, u, v, 1e-6, 2 / (nx - 1), 2 / (ny - 1), p,
+                                      1.0, 0.1)
+    compare(f"cavity_flow {nx} x {ny}, {nit} iterations", call(nx, ny),
+            call(32, 32) if nit > 1 else call(20, 20), 1.15 if nit > 1 else 1.8)
