@@ -132,6 +132,16 @@ def test_seidel2d_tile_edges(st, n, tsteps):
           oracle=c_oracle.seidel_2d_kernel)
 
 
+# the one-wave form's sizes beside the first of the tiles, and two launches of it
+@pytest.mark.parametrize("n,tsteps", [(6, 2), (7, 40), (9, 3), (10, 2), (10, 41), (11, 41),
+                                      (4, 65539)])
+def test_seidel2d_small_grids(st, n, tsteps):
+    from oracle import c_oracle
+    A = np.random.default_rng(n).random((n, n))
+    A[n // 2, 1:3] = 1e300  # past the tiles' short division
+    check(st, tsteps, A, f"small n={n} tsteps={tsteps}", oracle=c_oracle.seidel_2d_kernel)
+
+
 @pytest.mark.parametrize("case", ["tiny", "huge", "zeros and signs"])
 def test_seidel2d_division_range(st, case):
     """Values past the short division's range take the operator; zeros of

@@ -73,3 +73,9 @@ def test_cavity_flow_small_grids_cost_as_a_square_one(st, nx, ny, nit):
                                       1.0, 0.1)
     compare(f"cavity_flow {nx} x {ny}, {nit} iterations", call(nx, ny),
             call(32, 32) if nit > 1 else call(20, 20), 1.15 if nit > 1 else 1.8)
+
+
+def test_seidel2d_small_grids_cost_less_than_larger_ones(st):
+    a, b = (torch.full((n, n), 0.5, dtype=torch.float64, device="cuda") for n in (4, 16))
+    compare("seidel_2d 4 x 4, 69 sweeps", lambda: st.seidel2d(a, 70), lambda: st.seidel2d(b, 70),
+            0.7)
