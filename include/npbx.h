@@ -318,9 +318,8 @@ int npbx_channel_flow_launch(int dtype, int64_t nit, void *u, void *v,
 /* ---- 2-D Gauss-Seidel (seidel_2d_numpy.py:4-13) ----------------------------
  * A: (N, N) FP64 (dtype NPBX_F64), updated in place by TSTEPS - 1 sweeps;
  * bitwise the NumPy result.  N <= 16384; N < 3 or TSTEPS <= 1 is a no-op.
- * N <= 10 runs in one wave.  Else
- * tiles of 64 rows and 4 sweeps run as a wavefront over the whole device in
- * launches of at most "seidel.blocks" tiles, so a launch's duration is bounded
+ * N <= 10 runs in one wave; larger grids in tiles of 64 rows and 4 sweeps, as a
+ * wavefront over the whole device, in launches of at most "seidel.blocks" tiles, so a launch's duration is bounded
  * whatever N is.  Under stream capture (and on a device npbx_init was not
  * called for) each wavefront step is a launch of its own.  Calls on different
  * streams do not share state.  Tiles that wait for others give up after

@@ -274,6 +274,9 @@ Shape pick_shape(int dtype, const std::vector<SweepGrid>& grids, int cap, int ma
   Shape best{2, 4, 2};
   double best_us = INFINITY;
   const bool fp64 = dtype == NPBX_F64;
+  // depths past all but a grid's last sweep give the rounds that this one does
+  int64_t most = 0;
+  for (const SweepGrid& g : grids) most = std::max(most, g.nsweeps - 1);
   for (const Shape& sh : kShapes) {
     if (sh.v * sh.rows > max_points) continue;
     const int wj = 64 * sh.v, wi = kWaves * sh.rows;
@@ -305,6 +308,7 @@ Shape pick_shape(int dtype, const std::vector<SweepGrid>& grids, int cap, int ma
         best_us = us;
         best = {sh.v, sh.rows, depth};
       }
+      if (depth >= most) break;
     }
   }
   return best;

@@ -407,7 +407,7 @@ __global__ __launch_bounds__(kThreads) void seidel2d_tiles(SeidelArgs g, int slo
 // Lane 8 (t mod 8) + i - 1 has row i of sweep t; at most seven sweeps have a point
 // in one step, and none of a step's points reads another.  A step is nine LDS reads
 // and some twenty dependent operations; the tiles above spend twelve chunks of
-// mostly masked steps on such a grid.  us, 69 sweeps, tiles | here: 3 x 3 114 | 36,
+// mostly masked steps on such a grid.  us, 69 sweeps, tiles | here: 3 x 3 114 | 29,
 // 10 x 10 154 | 63; one sweep of 3 x 3 9.8 | 8.1.
 constexpr int kSmallN = 10;
 constexpr int64_t kSmallSweeps = 1 << 16;  // per launch: some 40 ms
