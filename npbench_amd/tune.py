@@ -7,7 +7,12 @@ seeded grids (HIP events on the launch stream) and keeps the fastest:
 * T = 1: the plain vector sweep, one launch per sweep and grid, with its
   workgroup shape `shape` (planes per workgroup / planes loaded ahead);
 * T >= 2: the temporal-blocked tile kernel with rows per wave R (heat) and
-  planes per tile `seg`, through a batch plan of all the grids.
+  planes per tile `seg`, through the serving rounds of all the grids.  These
+  settings bind the serving rounds and sweeps with ``tblock`` = T.
+
+A batch plan chooses its own launches, whatever these settings are, so it is
+timed once: the fastest T >= 2 shape is kept where a plan of all the grids is
+faster than their plain sweeps, with the plan's rate.
 
 Every candidate computes bitwise the same result, so the choice only moves
 performance.  Choices are cached in memory and in a JSON file
@@ -15,6 +20,7 @@ performance.  Choices are cached in memory and in a JSON file
 the class and the device name.
 """
 
+import ctypes
 import json
 import os
 import pathlib
@@ -24,6 +30,7 @@ import torch
 from . import _native as nat
 from . import batch
 from . import device as dev
+from . import serve
 from . import stencils as st
 
 DEFAULT_CACHE = pathlib.Path(os.environ.get(
@@ -101,8 +108,40 @@ def _time(fn, reps):
     return t.elapsed_ms() / reps / 1e3
 
 
+def _rounds(kind, grids, cfg, sweeps, queue):
+    """A call that runs every round of ``grids`` as the server's ticks do."""
+    dtype = grids[0][0].dtype
+    cols = [None] * len(grids)
+    if kind == "heat_3d" and dtype == torch.float32:  # packed once a request
+        elems = ctypes.c_int64()
+        nat.call("npbx_cols_elems", grids[0][0].shape[0], ctypes.byref(elems))
+        cols = [torch.empty(elems.value, dtype=dtype, device="cuda") for _ in grids]
+        for (a, b), c in zip(grids, cols):
+            nat.call("npbx_pack_cols", dev.dtype_code(a), dev.ptr(a), dev.ptr(b), a.shape[0],
+                     dev.ptr(c), dev.stream_handle())
+    ticks, level = [], 0
+    for r, depth in enumerate(serve.round_schedule(sweeps, cfg["T"])):
+        specs = (nat.RoundSpec * len(grids))()
+        for s, ab, c in zip(specs, grids, cols):
+            s.kind, s.dtype, s.n = batch.KIND[kind], dev.dtype_code(ab[0]), ab[0].shape[0]
+            s.A, s.B = dev.ptr(ab[0]), dev.ptr(ab[1])
+            s.X, s.Y = dev.ptr(ab[r % 2]), dev.ptr(ab[1 - r % 2])
+            s.level0, s.depth = level, depth
+            s.cols = dev.ptr(c) if c is not None else None
+        ticks.append(specs)
+        level += depth
+
+    def run():
+        for specs in ticks:
+            nat.call("npbx_rounds_launch", specs, len(grids), cfg["T"], cfg["seg"], queue,
+                     dev.stream_handle())
+    run.keep = cols
+    return run
+
+
 def measure(kind, dtype, n, count, cfg, sweeps=16, reps=2, seed=0):
-    """GLUP/s of ``cfg`` on ``count`` seeded grids of side ``n``."""
+    """GLUP/s of ``cfg`` on ``count`` seeded grids of side ``n``; with the key
+    "plan" set, of a batch plan of them."""
     dev.require_device()
     ndim = 2 if kind == "jacobi_2d" else 3
     g = torch.Generator(device="cuda")
@@ -118,6 +157,15 @@ def measure(kind, dtype, n, count, cfg, sweeps=16, reps=2, seed=0):
             for a, b in grids:
                 sweep(a, b, sweeps)
         secs = _time(fn, reps)
+    elif not cfg.get("plan"):
+        apply(cfg)
+        queue = ctypes.c_void_p()
+        nat.call("npbx_queue_create", ctypes.byref(queue))
+        try:
+            secs = _time(_rounds(kind, grids, cfg, sweeps, queue), reps)
+        finally:
+            torch.cuda.synchronize()
+            nat.call("npbx_queue_destroy", queue)
     else:
         apply(cfg)
         plan = batch.Plan([batch.Grid(kind, a, b, sweeps) for a, b in grids], tblock=cfg["T"],
@@ -153,6 +201,13 @@ def best(kind, dtype, n, count=1, cache=DEFAULT_CACHE, retune=False, sweeps=16, 
         results.append((rate, cfg))
         if verbose:
             print(f"tune {key} {cfg}: {rate:.1f} GLUP/s", flush=True)
+    tiles = [r for r in results if r[1]["T"] >= 2]
+    if tiles:
+        shape = max(tiles, key=lambda x: x[0])[1]
+        rate = measure(kind, dtype, n, count, {**shape, "plan": True}, sweeps=sweeps)
+        if verbose:
+            print(f"tune {key} plan: {rate:.1f} GLUP/s", flush=True)
+        results = [r for r in results if r[1]["T"] == 1] + [(rate, shape)]
     rate, cfg = max(results, key=lambda x: x[0])
     out = {**cfg, "glups": round(rate, 2)}
     _memo[key] = out

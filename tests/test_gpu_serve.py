@@ -74,3 +74,21 @@ def test_oversized_request_is_rejected():
     with pytest.raises(ValueError):
         srv.run([req], realtime=False)
     srv.close()
+
+
+def test_tuner_times_tile_shapes_through_the_rounds(monkeypatch):
+    """A shape's time is that of the serving rounds, which it binds; the settings
+    are left as found."""
+    from npbench_amd import _native, batch, tune
+    old = {k: _native.get_tuning(k) for k in ("heat.rows", "heat.seg")}
+    monkeypatch.setattr(batch, "Plan", None)
+    print("tuner: rounds", flush=True)
+    try:
+        for dtype, cfg in ((torch.float32, {"T": 3, "rows": 14, "seg": 32}),
+                           (torch.bfloat16, {"T": 2, "rows": 4, "seg": 32})):
+            assert tune.measure("heat_3d", dtype, 64, 3, cfg, sweeps=7) > 0
+        assert tune.measure("jacobi_2d", torch.float64, 128, 2,
+                            {"T": 2, "rows": 4, "seg": 32}) > 0
+    finally:
+        for k, v in old.items():
+            _native.set_tuning(k, v)

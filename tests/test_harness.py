@@ -254,6 +254,29 @@ def test_tuner_search_space_and_cache(tmp_path, monkeypatch):
     assert len(calls) == n_calls  # served from the file
 
 
+def test_tuner_times_a_plan_once(monkeypatch):
+    """Shapes are compared where they bind, the serving rounds; a plan, which no
+    shape binds, is timed once and decides between plain sweeps and tiles."""
+    torch = pytest.importorskip("torch")
+    from npbench_amd import tune
+    for plan_rate, wins in ((90.0, False), (500.0, True)):
+        calls = []
+
+        def fake_measure(kind, dtype, n, count, cfg, sweeps=16, reps=2, seed=0):
+            calls.append(dict(cfg))
+            if cfg["T"] == 1:
+                return 100.0
+            return plan_rate if cfg.get("plan") else 10.0 * cfg["T"] + 2 * cfg["rows"]
+
+        monkeypatch.setattr(tune, "measure", fake_measure)
+        monkeypatch.setattr(tune, "_memo", {})
+        cfg = tune.best("heat_3d", torch.float32, 256, 8, cache=None)
+        assert [c["T"] >= 2 for c in calls if c.get("plan")] == [True]
+        assert cfg["T"] == (3 if wins else 1)
+        if wins:  # the fastest shape of the rounds, the plan's rate
+            assert (cfg["rows"], cfg["glups"]) == (14, 500.0) and "plan" not in cfg
+
+
 # ------------------------------------------------------------------ report
 def test_speedup_report_from_the_result_store(tmp_path):
     from npbench_amd import report
