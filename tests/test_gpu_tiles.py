@@ -272,6 +272,54 @@ def test_plan_batch_wave_tiles(st, heat_rows, T, rows):
         plan.close()
 
 
+@pytest.mark.parametrize("dtype,T,rows", [("f32", T, rows) for T, rows in WAVE_SHAPES] +
+                         [("f32", 2, 8), ("f32", 3, 6), ("f32", 4, 4), ("f64", 2, 6),
+                          ("bf16", 2, 2), ("bf16", 2, 4)])
+@pytest.mark.parametrize("seg", [3, 32])
+def test_queued_rounds_match_each_grid_alone(st, heat_rows, dtype, T, rows, seg):
+    """The persistent tile queue (npbx_rounds_launch, the server's ticks) with
+    every kind of tile: uneven grids of both kinds whose rounds end at different
+    ticks, A and B of different and equal boundaries, packed columns given and
+    not."""
+    import ctypes
+    from npbench_amd import _native, batch, device, serve
+    heat_rows(rows)
+    cases = _mixed_batch(dtype, 11)
+    queue = ctypes.c_void_p()
+    _native.call("npbx_queue_create", ctypes.byref(queue))
+    live = []
+    for i, (kind, A, B, ns, first) in enumerate(cases):
+        a, b = device.to_device(A, DT[dtype]), device.to_device(B, DT[dtype])
+        cols = None
+        if kind == "heat_3d" and dtype == "f32" and i % 4 != 1:
+            elems = ctypes.c_int64()
+            _native.call("npbx_cols_elems", a.shape[0], ctypes.byref(elems))
+            cols = torch.empty(elems.value, dtype=torch.float32, device="cuda")
+            _native.call("npbx_pack_cols", device.dtype_code(a), device.ptr(a), device.ptr(b),
+                         a.shape[0], device.ptr(cols), device.stream_handle())
+        live.append([kind, a, b, first, serve.round_schedule(ns, T), cols, first])
+    print(f"queued rounds {dtype} T={T} rows={rows} seg={seg}", flush=True)
+    for tick in range(max(len(g[4]) for g in live)):
+        now = [g for g in live if tick < len(g[4])]
+        specs = (_native.RoundSpec * len(now))()
+        for s, g in zip(specs, now):
+            kind, a, b, level, depths, cols, first = g
+            # the array that holds `first`, then in turn
+            x, y = (a, b) if (first + tick) % 2 == 0 else (b, a)
+            s.kind, s.dtype, s.n = batch.KIND[kind], device.dtype_code(a), a.shape[0]
+            s.A, s.B, s.X, s.Y = (device.ptr(t) for t in (a, b, x, y))
+            s.level0, s.depth = level, depths[tick]
+            s.cols = device.ptr(cols) if cols is not None else None
+            g[3] += depths[tick]
+        _native.call("npbx_rounds_launch", specs, len(now), T, seg, queue,
+                     device.stream_handle())
+    torch.cuda.synchronize()
+    _native.call("npbx_queue_destroy", queue)
+    for (kind, a, b, *_), (_, A, B, ns, first) in zip(live, cases):
+        pa, pb = run(st, kind, A, B, dtype, ns, first, 1)
+        assert same(a, pa) and same(b, pb), f"{kind} n={A.shape[0]}"
+
+
 def _device_batch(dtype, specs, same_boundary):
     """(kind, n, nsweeps, first) -> the grids of a plan and copies of them."""
     from npbench_amd import batch
