@@ -1281,7 +1281,7 @@ double plain_us(const std::vector<SweepGrid>& grids) {
   return 3.3 * longest + 1.42e-6 * points;
 }
 
-double march_us(const std::vector<SweepGrid>& grids) {
+double march_us(const std::vector<SweepGrid>& grids, int cus) {
   double longest = 0, planes = 0;
   for (const SweepGrid& g : grids) {
     int tk, tj;
@@ -1290,7 +1290,7 @@ double march_us(const std::vector<SweepGrid>& grids) {
               heat_march_columns(g.n, kHeatMarchDepth, &tk, &tj) * (g.n - 2);
   }
   if (longest == 0) return 0;
-  const double part = std::ceil(planes / longest / compute_units());
+  const double part = std::ceil(planes / longest / cus);
   return longest * 1.25 * (5 + 2.3 * (part + 10)) / kHeatMarchDepth;
 }
 
@@ -1316,10 +1316,11 @@ void split_heat(int dtype, const std::vector<SweepGrid>& grids, std::vector<Swee
       if (g.n >= kHeatMarchRows) sides.push_back(g.n);
     std::sort(sides.begin(), sides.end());
     sides.erase(std::unique(sides.begin(), sides.end()), sides.end());
+    const int cus = compute_units();
     double best_us = plain_us(grids);
     for (const int side : sides) {
       from_side(side);
-      const double us = (march_us(rounds) + plain_us(plain)) * (plain.empty() ? 1 : 1.18);
+      const double us = (march_us(rounds, cus) + plain_us(plain)) * (plain.empty() ? 1 : 1.18);
       if (us < best_us) best_us = us, best = side;
     }
   }
