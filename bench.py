@@ -633,7 +633,7 @@ def kernel_suite(st, dev, torch, clock, reps, copy_only=False, cpu=False):
             "ms_per_call": round(ev / reps * 1e3, 4),
             "us_per_phase": round(ev / reps / phases * 1e6, 3),
             "glups": round(NT * (NIT + 2) * (NXC - 2) * (NYC - 2) * reps / ev / 1e9, 3),
-            "bound": "latency (two launches a time step)"}
+            "bound": "launches and latency (up to 24 iterations a launch, and one for the velocities)"}
         del c0, c1
 
     # channel flow (FP64) at the paper preset from the reference

@@ -505,8 +505,8 @@ __global__ __launch_bounds__(NT) void adi_rows(AdiArgs g) {
 // sides, wave 0 runs the forward recurrence over it in place (q) and then the
 // back substitution (x), and the helpers check q and store x as the chunks are
 // finished.  Wave 0 so issues what the recurrence itself consists of -- five
-// dependent FP64 operations a step forward, two back, about 8.3 ns each --
-// and its LDS accesses; with right-hand sides, checks and staging on the same
+// dependent FP64 operations a step forward, two back, some 3 ns each -- and its
+// LDS accesses; with right-hand sides, checks and staging on the same
 // wave (adi_columns, adi_rows) it was bound by issuing those.  Chunks are
 // handed over by flags in LDS, so no wave waits for another but for data.
 //
@@ -521,8 +521,11 @@ __global__ __launch_bounds__(NT) void adi_rows(AdiArgs g) {
 //
 // Time per half sweep against one-wave workgroups that do it all (path 3):
 // N = 50 7.4 -> 5.4 us, 100 14.6 -> 8.8, 200 23.8 -> 13.6, 300 40.9 -> 18.5,
-// 1000 133 -> 61, 1800 226 -> 103: 58 ns a step, 7 dependent FP64 operations
-// at about 8.3 ns, and 2 us for the launch and the first loads.
+// 1000 133 -> 61, 1800 226 -> 103: 58 ns a step, and 2 us for the launch and the
+// first loads.  The chain is not the bound: a wave's dependent FP64 operation
+// takes 6.5 (fma) or 7.5 cycles (add, multiply) at 2.40 GHz, timed by clock64
+// and by the wall clock, so its seven take 21 ns; the others have not been taken
+// apart (wave 0's LDS reads and flags, the helpers' loads).
 constexpr int kSplitLines = 8;  // L; 16 is 2 % slower, 32 8 %, 64 20 % (N = 200)
 constexpr int kHelpers = 3;     // 7 are level
 constexpr int kAhead = 2;       // chunks a helper loads ahead; 4 are level

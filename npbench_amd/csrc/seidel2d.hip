@@ -33,9 +33,10 @@
 // independent tiles per launch with no counters: for stream capture, where a
 // replay must not share state with other calls.
 //
-// Bound by the chains' latency: 110 to 130 cycles a step (a shift and ten
-// dependent FP64 operations, 20 instructions to issue), about 1.1 us for a
-// chunk with its exchange and barrier, and about 12 chunks from one tile's
+// Bound by the chunks' chain, 1.4 us each (some 420 at N = 400): sixteen steps
+// of a shift and ten dependent FP64 operations, about 90 cycles (14 and 7.5 each,
+// timed on one wave) or 0.6 us at 2.40 GHz, then the chunk's exchange through
+// LDS, the helpers' loads and the barrier; and about 12 chunks from one tile's
 // start to the next one's in either direction (8 of them the bands' skew).
 // N = 400, 99 sweeps on the MI355X: 0.59 ms (slot by slot 2.5 ms; the former
 // kernel, one workgroup running row recurrences back to back, 39.6 ms).

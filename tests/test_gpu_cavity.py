@@ -1,12 +1,11 @@
 """GPU parity of the lid-driven cavity flow (npbx_cavity_flow) against the
 FP64 oracle.
 
-One workgroup runs every phase of every time step with the reference's
-arithmetic, so results must be bitwise the oracle's.  Sizes cover the
-smallest grid (3 x 3), grids whose interior is narrower and wider than the
-1024-thread workgroup, both pressure placements (LDS up to 10240 points,
-device memory above), odd and even iteration counts (the pressure ends in
-either buffer), nit = 0, and the reference's initialisation at its S and M
+One workgroup (small grids) or chip-wide launches of blocks run with the
+reference's arithmetic, so results must be bitwise the oracle's.  Sizes cover the
+smallest grid (3 x 3), both sides of the choice between the forms, several blocks
+per direction with partial last ones, odd and even iteration counts (the pressure
+ends in either buffer), nit = 0, and the reference's initialisation at its S and M
 presets.
 """
 

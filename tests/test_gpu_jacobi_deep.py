@@ -1,10 +1,9 @@
-"""The LDS-blocked 2-D Jacobi kernel (knob "jacobi.deep": up to that many
-sweeps per launch; "jacobi.deep_waves": 4, 8 or 16 waves per workgroup)
-against the one-launch-per-sweep path: bitwise equal for every storage type,
-grid sizes from the smallest to several blocks per side (blocks of 64 rows x
-48 columns), depths 2 .. 8, every wave count and sweep ranges with odd and
-even first sweeps; and the FP64 result against the oracle at the measured
-configuration (1000^2, 200 sweeps)."""
+"""The register-blocked 2-D Jacobi kernel (knob "jacobi.deep": at most that many
+sweeps per launch, 8 as many as the shape chooses; "jacobi.deep_waves" is accepted
+and has no effect) against the one-launch-per-sweep path: bitwise equal for every
+storage type, grid sizes from the smallest to several blocks per side, every
+setting of the knobs and sweep ranges with odd and even first sweeps; and the FP64
+result against the oracle at the measured configuration (1000^2, 200 sweeps)."""
 
 import numpy as np
 import pytest

@@ -1,13 +1,13 @@
 """GPU parity of the 2-D Gauss-Seidel sweeps (npbx_seidel2d) against the FP64
 oracle.
 
-Rows run in wavefront slots with the reference's arithmetic, so results must
-be bitwise the oracle's.  Sizes cover the smallest grid, rows shorter and
-longer than a 256-column block (one, two and three blocks), sweeps spanning
-two slot schedules (at most 64 sweeps each), full 64-row slots (the paper
-preset), launches split at arbitrary slots (the "seidel.blocks" budget), the
-division operator's path (zeros), the reference's initialisation at its S, M,
-L and paper presets, and the largest accepted N.  Large cases are checked
+Tiles of 64 rows and 4 sweeps run with the reference's arithmetic, so results
+must be bitwise the oracle's.  Sizes cover the smallest grids (one wave up to 10
+points a side), row counts around the tiles' bands and sweep counts around their
+groups, launches split by the "seidel.blocks" budget, the division operator's
+path, zeros of either sign, calls on two streams and under capture, a wait that
+gives up, the reference's initialisation at its S, M, L and paper presets, and
+the largest accepted N.  Large cases are checked
 against the oracle's C restatement (pinned bit for bit to the NumPy oracle on
 the CPU).
 """
