@@ -119,7 +119,7 @@ struct InteriorWalk {
 };
 
 constexpr int kChunkV = 2;  // velocity points per chunk (14 loads each)
-constexpr int kMaxPts = 2;  // interior points per thread, in the one-workgroup form
+constexpr int kMaxPts = 4;  // most interior points per thread, in the one-workgroup form
 
 // The point computations take their division as a policy (ShortDiv or
 // FullDiv, run by chunk_eval).
@@ -489,25 +489,26 @@ __global__ __launch_bounds__(1024) void cavity_velocity(CavityArgs g, const doub
   }
 }
 
-// Grids of up to kLdsPoints points, kMaxPts interior points a thread: both
-// pressure buffers live in LDS for the whole run, each thread keeps its (at most kMaxPts) interior points' indices,
+// Grids of up to kLdsPoints points, PTS (2 or kMaxPts) interior points a thread:
+// both pressure buffers live in LDS for the whole run, each thread keeps its (at most PTS) interior points' indices,
 // edge flags and b values in registers -- it computes b for the same points
 // it then iterates -- so a pressure iteration touches LDS only.
+template <int PTS>
 __global__ __launch_bounds__(kThreadsC) void cavity_flow_lds(CavityArgs g) {
   __shared__ double lp[2 * kLdsPoints];
   const int t = threadIdx.x, nx = g.nx, ny = g.ny;
   const int np = nx * ny;
   const CavityDivisors dv = cavity_divisors(g);
   const InteriorWalk walk(t, nx, ny);
-  int pa[kMaxPts];  // past cnt: the safe interior index nx + 1, read and never written
+  int pa[PTS];  // past cnt: the safe interior index nx + 1, read and never written
 #pragma unroll
-  for (int m = 0; m < kMaxPts; ++m) pa[m] = nx + 1;
+  for (int m = 0; m < PTS; ++m) pa[m] = nx + 1;
   int pfl = 0;  // 3 edge-flag bits per point
   int cnt = 0;
-  walk.each<kMaxPts>([&](const int(&a)[kMaxPts], const int(&fl)[kMaxPts],
-                         const bool(&ok)[kMaxPts]) {
+  walk.each<PTS>([&](const int(&a)[PTS], const int(&fl)[PTS],
+                         const bool(&ok)[PTS]) {
 #pragma unroll
-    for (int m = 0; m < kMaxPts; ++m) {
+    for (int m = 0; m < PTS; ++m) {
       pa[m] = a[m];
       pfl |= (ok[m] ? fl[m] : 0) << (3 * m);
       cnt += ok[m] ? 1 : 0;
@@ -522,12 +523,12 @@ __global__ __launch_bounds__(kThreadsC) void cavity_flow_lds(CavityArgs g) {
     // neighbours' addresses each step instead of holding every one of them
     // in registers across the loop
 #pragma unroll
-    for (int m = 0; m < kMaxPts; ++m) asm volatile("" : "+v"(pa[m]));
+    for (int m = 0; m < PTS; ++m) asm volatile("" : "+v"(pa[m]));
     asm volatile("" : "+v"(pfl), "+v"(cnt));
     copy_velocities(g, t, np);
-    double bq[kMaxPts];
+    double bq[PTS];
 #pragma unroll
-    for (int m0 = 0; m0 < kMaxPts; m0 += kChunkV) {
+    for (int m0 = 0; m0 < PTS; m0 += kChunkV) {
       double bc[kChunkV] = {};
       if (m0 < cnt)  // whole waves skip the chunks past their points
         chunk_eval(dv, bc, [&](int c, auto& div) { return source_at(g, dv, pa[m0 + c], div); });
@@ -541,17 +542,17 @@ __global__ __launch_bounds__(kThreadsC) void cavity_flow_lds(CavityArgs g) {
       // compiler would otherwise hoist out of this loop overflow the scalar
       // registers
 #pragma unroll
-      for (int m = 0; m < kMaxPts; ++m) asm volatile("" : "+v"(pa[m]));
+      for (int m = 0; m < PTS; ++m) asm volatile("" : "+v"(pa[m]));
       asm volatile("" : "+v"(pfl), "+v"(cnt));
 #pragma unroll
-      for (int m0 = 0; m0 < kMaxPts; m0 += kMaxPts / 2) {
+      for (int m0 = 0; m0 < PTS; m0 += PTS / 2) {
         if (m0 >= cnt) continue;
-        double val[kMaxPts / 2];
+        double val[PTS / 2];
         chunk_eval(dv, val, [&](int c, auto& div) {
           return pressure_at(g, dv, cur, pa[m0 + c], bq[m0 + c], div);
         });
 #pragma unroll
-        for (int c = 0; c < kMaxPts / 2; ++c)
+        for (int c = 0; c < PTS / 2; ++c)
           if (m0 + c < cnt) store_pressure(nxt, pa[m0 + c], (pfl >> (3 * (m0 + c))) & 7, nx, val[c]);
       }
       for (int k = t; k < nx; k += kThreadsC) nxt[(ny - 1) * nx + k] = 0.0;  // p[-1, :] = 0
@@ -561,7 +562,7 @@ __global__ __launch_bounds__(kThreadsC) void cavity_flow_lds(CavityArgs g) {
       nxt = tmp;
     }
 #pragma unroll
-    for (int m0 = 0; m0 < kMaxPts; m0 += kChunkV) {
+    for (int m0 = 0; m0 < PTS; m0 += kChunkV) {
       if (m0 >= cnt) continue;
       double nu[kChunkV], nv[kChunkV];
       chunk_eval(dv, nu, [&](int c, auto& div) {
@@ -679,13 +680,14 @@ int blocked_flow(const CavityArgs& a, hipStream_t stream) {
 }
 
 // The one-workgroup form where an iteration costs less than its share of the
-// blocked form's launches: up to some 1500 interior points, and up to two a
-// thread where there are few iterations.  us a step, one workgroup | blocks:
-//   iterations        1            4 or 5        10          20          50
+// blocked form's launches: up to some 1500 interior points, and more where there
+// are few iterations.  us a step, one workgroup | blocks:
+//   iterations        1            5             10          20          50
 //   20 x 20       3.2 |  9.7    4.8 | 10.8   6.7 | 12.7  10.7 | 20.9  22.4 | 46.9
 //   33 x 33       6.3 | 10.6    8.6 | 11.2  11.5 | 13.4  17.2 | 21.6  34.4 | 48.5
 //   40 x 40       6.7 | 10.0    9.5 | 11.5  13.2 | 13.1  20.3 | 21.9  41.9 | 48.7
 //   45 x 45       7.2 | 10.3   10.9 | 11.5  15.7 | 13.3  25.1 | 22.0  53.3 | 49.3
+//   50 x 50       8.2 | 10.3   12.3 | 12.3  17.3 | 13.8  27.3 | 22.0
 //   400 wide, 3   4.3 |  8.7    5.9 | 10.0   7.9 | 12.2  11.8 | 20.5  23.6 | 47.6
 //   2000 wide, 3 10.2 |  9.1   14.0 | 10.3  18.7 | 12.4  28.2 | 20.8  56.5 | 47.7
 // Without iterations (velocities only) 400 x 3 takes 3.8 | 4.7, 32 x 32 5.5 | 5.3
@@ -693,9 +695,10 @@ int blocked_flow(const CavityArgs& a, hipStream_t stream) {
 bool use_lds(int64_t nx, int64_t ny, int64_t nit) {
   const int64_t points = nx * ny, interior = (nx - 2) * (ny - 2);
   if (points <= 1024) return true;
-  if (points > kLdsPoints || interior > int64_t(kMaxPts) * kThreadsC) return false;
+  static_assert(2600 <= kMaxPts * kThreadsC);
+  if (points > kLdsPoints || interior > 2600) return false;
   if (nit == 0) return interior <= 600;
-  return interior <= 1500 || (nit <= 4 && points <= 4000);
+  return interior <= 1500 || (nit <= (interior <= 2048 ? 4 : 2) && points <= 4000);
 }
 
 }  // namespace
@@ -755,7 +758,9 @@ extern "C" int npbx_cavity_flow(int dtype, int64_t nx, int64_t ny, int64_t nt, i
   const int64_t per_launch = std::max<int64_t>(1, int64_t(150000000) / (np * (nit + 3)));
   for (int64_t done = 0; done < nt; done += per_launch) {
     g.nt = static_cast<int>(std::min<int64_t>(per_launch, nt - done));
-    hipLaunchKernelGGL(cavity_flow_lds, dim3(1), dim3(kThreadsC), 0, as_stream(stream), g);
+    const auto kernel =
+        (nx - 2) * (ny - 2) <= 2 * kThreadsC ? cavity_flow_lds<2> : cavity_flow_lds<kMaxPts>;
+    hipLaunchKernelGGL(kernel, dim3(1), dim3(kThreadsC), 0, as_stream(stream), g);
     NPBX_LAUNCHED("cavity_flow_lds");
   }
   return NPBX_OK;

@@ -96,7 +96,7 @@ def test_cavity_blocked_bitwise(st, ny, nx, nt, nit):
 
 
 @pytest.mark.parametrize("ny,nx", [(3, 1000), (1000, 3), (3, 2100), (2100, 3), (33, 32), (40, 41),
-                                   (46, 46)])
+                                   (46, 46), (50, 51)])
 @pytest.mark.parametrize("nt,nit", [(3, 0), (2, 1), (1, 4), (2, 5), (1, 25)])
 def test_cavity_forms_bitwise(st, ny, nx, nt, nit):
     """Both sides of the choice between one workgroup and blocks, by points and
