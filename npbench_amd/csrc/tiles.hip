@@ -42,6 +42,7 @@
 #include <vector>
 
 #include "common.h"
+#include "lanes.h"
 #include "points.h"
 #include "tiles.h"
 #include "vecio.h"
@@ -327,15 +328,6 @@ __device__ __forceinline__ void heat_tile(const GridRound g, int tile,
 constexpr int kPrivateRows = 10;  // heat.rows >= this selects the wave-private tile
 constexpr bool wave_private(int rows) { return rows >= kPrivateRows; }
 
-// Full-wave DPP shifts (wave_shr:1, wave_shl:1): lane l receives lane l-1's
-// (from_left) or lane l+1's (from_right) value; lane 0 / lane 63 receive 0,
-// which only ever reaches halo or global-boundary points.
-__device__ __forceinline__ float from_left(float x) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x138, 0xF, 0xF, true));
-}
-__device__ __forceinline__ float from_right(float x) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x130, 0xF, 0xF, true));
-}
 __device__ __forceinline__ float lane_value(float x, int lane) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
 }
@@ -575,8 +567,10 @@ __device__ __forceinline__ void heat_wave_tile(const GridRound g, int tile) {
       // level l's arrival (plane P - l) becomes its newest plane
 #pragma unroll
       for (int r = m; r < JR - m; ++r) {
-        const float left = from_left(in[r][V - 1]);
-        const float right = from_right(in[r][0]);
+        // the 0 that the outer lanes receive only ever reaches halo or
+        // global-boundary points
+        const float left = lane_from_left(in[r][V - 1]);
+        const float right = lane_from_right(in[r][0]);
 #pragma unroll
         for (int v = 0; v < V; ++v) {
           const float km = v > 0 ? in[r][v - 1] : left;
