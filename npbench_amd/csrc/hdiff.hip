@@ -402,10 +402,11 @@ constexpr bool whole_lines(int64_t bytes) { return bytes % 64 == 0 || bytes >= 3
 //        256 x 256 x 160  26.2 | 21.1    26.4 | 20.9    26.0 | 22.1
 // FP64 columns that end inside lines: 2 x 6 x 8 B kept (1000 x 1000 x 3 14.9,
 // streamed 20.0).  FP32 with odd K has 4-byte vectors only (190 x 203 x 137, 4 x 6
-// streamed 14.6, kept 14.0; a point per thread 29.3).  BF16 4 x 6 x 4 B 15.2 at 256 x 256 x 160
-// (2 x 6 x 8 B 15.4), with columns of K = 8 m that end inside lines shape 2
-// (1000 x 1000 x 8 13.1; 4 x 6 x 4 B 25.7 streamed, 13.8 kept), of K = 4 m 2 x 6 x
-// 8 B kept; odd K the tail form (190 x 203 x 137 10.6; a point per thread 21.9).
+// streamed 14.6, kept 14.0; a point per thread 29.3).  BF16 4 x 6 x 4 B 15.2 at
+// 256 x 256 x 160 (2 x 6 x 8 B 15.4), with columns of K = 8 m that end inside
+// lines shape 2 (1000 x 1000 x 8 13.1; 4 x 6 x 4 B 25.9 streamed, 13.8 kept), of
+// K = 4 m 2 x 6 x 8 B kept; odd K the tail form (190 x 203 x 137 10.6; a point per
+// thread 21.9).
 template <class S, class Fits>
 March default_march(int I, int J, int K, Fits&& fits) {
   const int64_t points = int64_t(I) * J * K, bytes = int64_t(K) * sizeof(S);

@@ -323,21 +323,32 @@ int run_points(S* A, S* B, int n, int64_t first, int64_t nsweeps, hipStream_t st
 // points: FP64 385^3 takes four waves of vectors or six of points, 348 | 283 us;
 // FP32 keeps points but where rows are whole multiples of 256, whose planes then
 // fall on few channels (512^3 350 | 4x8/4 314).
-// Measured, us per sweep, V points a lane x planes / ahead:
-//   FP64       2x1/1  2x2/2  2x4/4  2x8/4  2x16/4   1x16    BF16  2x2/2  4x2/2  8x4/2  8x8/4  1x16
-//     64^3       3.7    3.7    3.7    4.9    7.6             64^3   3.5    4.0    7.0
-//     101^3      6.3    6.1    6.3    7.1    8.4            101^3   4.8    5.5    7.5            7.1
-//     160^3     18.3   17.4   16.8   17.5   19.6   19.8     176^3          11.3                 10.9
-//     201^3     29.1   27.6   25.8   25.7   29.8            200^3          13.0                 16.7
-//     385^3                           348           283     258^3          34.7   23.1   26     26.6
-//     400^3                           358           344     400^3                 54.0   57     88
-//     512^3      723    678    626    612    626    669     512^3                  176   176    237
-//   FP32       2x1/1  1x4/4  1x8/4  4x4/4  4x16/4           513^3                  330          199
-//     64^3       3.5    3.2    3.8    3.9    8.5           1024^3                 1393  1289   2122
-//     101^3      5.2    4.7    5.1    5.5    8.5    (4x8/4 512^3 .. 768^3: 513^3 247, 700^3 500,
-//     201^3     20.9   18.4   14.8   15.6   18.2    1x16 562)
-//     256^3     32.0   27.5   22.2   24.7   25.7
-//     384^3             125    123    137    139
+// Measured, us per sweep, V points a lane x planes / ahead (1x16: heat3d_sweep):
+//   FP64       2x1/1  2x2/2  2x4/4  2x8/4  2x16/4   1x16
+//     64^3       3.7    3.7    3.7    4.9    7.6
+//     101^3      6.3    6.1    6.3    7.1    8.4
+//     160^3     18.3   17.4   16.8   17.5   19.6    19.8
+//     201^3     29.1   27.6   25.8   25.7   29.8
+//     385^3             372    349    346    351     283
+//     400^3             385    358    356    361     344
+//     512^3      723    678    626    612    626     665
+//   FP32       2x1/1  1x4/4  1x8/4  4x4/4   4x8/4  4x16/4   1x16
+//     64^3       3.5    3.2    3.8    3.9             8.5
+//     101^3      5.2    4.7    5.1    5.5             8.5
+//     201^3     20.9   18.4   14.8   15.6            18.2
+//     256^3     32.0   27.1   23.0   25.1    25.6    26.3     39
+//     384^3             125    123    167     166     165    144
+//     512^3             322    353    316     315     320    378
+//   BF16       2x2/2  4x2/2  8x4/2  8x8/4   4x8/4   1x16
+//     100^3      5.0    5.9    7.8   11.0     9.2    7.6
+//     176^3     13.8   11.3   13.6   13.7    12.4   10.9
+//     200^3     16.7   13.0   15.5   15.9    14.2   16.7
+//     258^3     36.7   34.8   23.1   25.9    31.6   26.6
+//     400^3      114     79     54     58      69     88
+//     512^3      272    201    176    176     185    237
+//     513^3      332    276    328    323     247    199
+//     700^3      755    549    615    596     500    562
+//     1024^3    2217   1625   1382   1289    1454   2122
 template <class S>
 int run_sweeps(S* A, S* B, int n, int64_t first, int64_t nsweeps, hipStream_t stream) {
   constexpr int N = Vec16<S>::N;
