@@ -490,9 +490,10 @@ __global__ __launch_bounds__(1024) void cavity_velocity(CavityArgs g, const doub
 }
 
 // Grids of up to kLdsPoints points, PTS (2 or kMaxPts) interior points a thread:
-// both pressure buffers live in LDS for the whole run, each thread keeps its (at most PTS) interior points' indices,
-// edge flags and b values in registers -- it computes b for the same points
-// it then iterates -- so a pressure iteration touches LDS only.
+// both pressure buffers live in LDS for the whole run, each thread keeps its (at
+// most PTS) interior points' indices, edge flags and b values in registers -- it
+// computes b for the same points it then iterates -- so a pressure iteration
+// touches LDS only.
 template <int PTS>
 __global__ __launch_bounds__(kThreadsC) void cavity_flow_lds(CavityArgs g) {
   __shared__ double lp[2 * kLdsPoints];

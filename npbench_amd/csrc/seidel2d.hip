@@ -554,7 +554,8 @@ extern "C" int npbx_seidel2d(int dtype, void* A, int64_t N, int64_t tsteps, void
   if (N <= kSmallN) {
     for (int64_t done = 0; done < sweeps; done += kSmallSweeps) {
       hipLaunchKernelGGL(seidel2d_small, dim3(1), dim3(64), 0, s, static_cast<double*>(A),
-                         static_cast<int>(N), static_cast<int>(std::min(kSmallSweeps, sweeps - done)));
+                         static_cast<int>(N),
+                         static_cast<int>(std::min(kSmallSweeps, sweeps - done)));
       NPBX_LAUNCHED("seidel2d_small");
     }
     return NPBX_OK;
